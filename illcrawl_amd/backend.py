@@ -693,8 +693,9 @@ class BatchRenderer:
                     num_particles=gi.num_particles)
 
     def set_tile(self, w, h, workgroup=256):
-        """Gather tile of w x h points, one tile per workgroup of `workgroup`
-        threads (256, or 64 for one-wave 16x16 tiles)."""
+        """Gather tile of w x h points.  The gather works in tiles of 16x16 or
+        8x8 points, chosen by the number of points; workgroup=64 with (16, 16)
+        or (8, 8) asks for that tile whatever the number."""
         N.call("ilc_batch_set_tile_wg", self._h, int(w), int(h), int(workgroup))
 
     def tile(self):

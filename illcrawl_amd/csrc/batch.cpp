@@ -112,6 +112,7 @@ struct ilc_batch {
   int mode = ILC_MODE_REFERENCE;
   int kernel = ILC_KERNEL_QUARTIC_REF;
   tile_shape ts{32, 4};
+  sum_shape ss{16};  // the planned render's tiles
 
   particle_soa ps{};
   bool have_particles = false;
@@ -519,10 +520,13 @@ void plan(ilc_batch* b, hipStream_t s) {
     if (psa != psc) return psa > psc;
     return uint64_t(ca.nx) * ca.ny > uint64_t(cc.nx) * cc.ny;
   });
-  uint64_t nitems = 0;
+  uint64_t nitems = 0, npoints = 0;
+  for (size_t v = 0; v < nv; ++v)
+    npoints += uint64_t(b->views[v]->v.cam.nx) * b->views[v]->v.cam.ny;
+  b->ss = sum_shape_of(b->ts, npoints);
   for (size_t v = 0; v < nv; ++v) {
     view_state& vs = *b->views[v];
-    tile_grid(b->ts, vs.v.cam.nx, vs.v.cam.ny, &vs.tiles_x, &vs.ntiles);
+    tile_grid(b->ss, vs.v.cam.nx, vs.v.cam.ny, &vs.tiles_x, &vs.ntiles);
     nitems += vs.ntiles;
   }
   ILC_REQUIRE(nitems < (uint64_t(1) << 32), "too many work items");
@@ -555,7 +559,7 @@ void plan(ilc_batch* b, hipStream_t s) {
   b->planned = true;
   b->grid_blocks = gather_batch_grid(
       b->clip ? OP_CLIP : (b->mode == ILC_MODE_REFERENCE ? OP_REFERENCE : OP_EXACT), b->kernel,
-      b->ts);
+      b->ss);
 }
 
 // An event for timing the gather launch(es) of an eager render.
@@ -781,7 +785,8 @@ void device_work(ilc_batch* b, bool persistent, hipStream_t s, bool timed = fals
       build_view(b, vs, main, true);
       const view_desc d = make_desc(b, v);
       if (timed) ILC_HIP(hipEventRecord(timing_event(b), s));
-      launch_gather(d.g, d.p, op, b->kernel, b->ts, vs.acc.p, nullptr, b->cubic.p, s);
+      // as the single-view backend tiles the view
+      launch_gather(d.g, d.p, op, b->kernel, sum_shape_of(b->ts, d.p.n), vs.acc.p, nullptr, b->cubic.p, s);
       if (timed) ILC_HIP(hipEventRecord(timing_event(b), s));
       launch_retrieve(vs.acc.p, d.p.n, vs.v.scale, vs.img.p, s);
     }
@@ -812,11 +817,11 @@ void device_work(ilc_batch* b, bool persistent, hipStream_t s, bool timed = fals
                            hipMemcpyHostToDevice, s));
     ILC_HIP(hipMemcpyAsync(b->items_dev.p, b->items_host.p, sizeof(uint2) * b->nitems,
                            hipMemcpyHostToDevice, s));
-    launch_order_items(b->desc_dev.p, b->items_dev.p, b->segs, b->nitems, b->ts, b->item_keys.p,
+    launch_order_items(b->desc_dev.p, b->items_dev.p, b->segs, b->nitems, b->ss, b->item_keys.p,
                        b->item_idx.p, b->item_temp.p, b->items_ord.p, s);
     if (timed) ILC_HIP(hipEventRecord(timing_event(b), s));
     launch_gather_batch(b->desc_dev.p, b->items_ord.p, b->segs, b->qcounters.p, op, b->kernel,
-                        b->ts, b->cubic.p, b->grid_blocks, s);
+                        b->ss, b->cubic.p, b->grid_blocks, s);
     if (timed) ILC_HIP(hipEventRecord(timing_event(b), s));
     // the gather wrote every view's accumulator and image
   }
@@ -1055,7 +1060,7 @@ ilc_status ilc_batch_count_evals(ilc_batch* b, uint64_t* per_view_host, void* st
       cnt.ensure(P);
       launch_fill_u32(reinterpret_cast<uint32_t*>(cnt.p), 0u, 2 * P, s);
       point_view p{vs.pts.p, static_cast<uint32_t>(P), vs.v.cam.nx, vs.v.cam.ny};
-      launch_gather(grid_of(b, vs), p, OP_COUNT, b->kernel, b->ts, nullptr, cnt.p, nullptr, s);
+      launch_gather(grid_of(b, vs), p, OP_COUNT, b->kernel, b->ss, nullptr, cnt.p, nullptr, s);
       per_view_host[v] = launch_sum_u64(cnt.p, P, tmp.p, s);
     }
   });
@@ -1174,9 +1179,9 @@ ilc_status ilc_batch_autotune(ilc_batch* b, int32_t* tile_w, int32_t* tile_h, do
     require_ready(b);
     device_guard dg(b->device);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // one tile per workgroup of 256 threads, and 16x16 tiles of one wave
-    static const tile_shape cand[] = {{16, 1, 256}, {32, 2, 256}, {32, 4, 256}, {64, 4, 256},
-                                      {16, 4, 64},  {8, 1, 64}};
+    // the two tile sides; the 256-thread shapes pick one of them by the
+    // number of points
+    static const tile_shape cand[] = {{16, 4, 64}, {8, 1, 64}};
     ensure_cubic(b);  // the cubic gather reads its table from the first launch
     struct events {
       hipEvent_t e[2] = {nullptr, nullptr};

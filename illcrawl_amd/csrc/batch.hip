@@ -940,7 +940,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_u32(const uint32_t* __restric
 // stride over taller boxes) and 8 layers: it is an estimate.
 __global__ __launch_bounds__(kBlock) void k_item_cost(const view_desc* __restrict__ views,
                                                       const uint2* __restrict__ items,
-                                                      queue_segs segs, uint32_t n, int tw, int th,
+                                                      queue_segs segs, uint32_t n, int side,
                                                       uint32_t* __restrict__ keys,
                                                       uint32_t* __restrict__ idx) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
@@ -952,10 +952,10 @@ __global__ __launch_bounds__(kBlock) void k_item_cost(const view_desc* __restric
   const grid_view& g = vd.g;
   uint64_t cost = 0;
   const uint32_t tx = it.y % vd.tiles_x, ty = it.y / vd.tiles_x;
-  const uint32_t px0 = tx * uint32_t(tw), py0 = ty * uint32_t(th);
+  const uint32_t px0 = tx * uint32_t(side), py0 = ty * uint32_t(side);
   if (px0 < vd.p.lnx && py0 < vd.p.lny && g.nc[0] > 0 && g.nc[1] > 0 && g.nc[2] > 0) {
-    const uint32_t px1 = min(px0 + uint32_t(tw), vd.p.lnx) - 1u;
-    const uint32_t py1 = min(py0 + uint32_t(th), vd.p.lny) - 1u;
+    const uint32_t px1 = min(px0 + uint32_t(side), vd.p.lnx) - 1u;
+    const uint32_t py1 = min(py0 + uint32_t(side), vd.p.lny) - 1u;
     const uint64_t ia = uint64_t(py0) * vd.p.lnx + px0, ib = uint64_t(py1) * vd.p.lnx + px1;
     if (ib < vd.p.n) {
       const float4 a = vd.p.pts[ia], b = vd.p.pts[ib];
@@ -1170,12 +1170,11 @@ void launch_local_keys(const uint32_t* gkey, const uint32_t* cbase, int nv, uint
 }
 
 void launch_order_items(const view_desc* views, const uint2* items, const queue_segs& segs,
-                        uint32_t n, const tile_shape& ts, uint32_t* keys, uint32_t* idx,
+                        uint32_t n, const sum_shape& ts, uint32_t* keys, uint32_t* idx,
                         uint32_t* radix_temp, uint2* out, hipStream_t s) {
   if (!n) return;
-  const int th = (kBlock / ts.tw) * ts.ppt;
   hipLaunchKernelGGL(k_item_cost, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, views,
-                     items, segs, n, ts.tw, th, keys, idx);
+                     items, segs, n, ts.side, keys, idx);
   ILC_HIP(hipGetLastError());
   launch_radix_sort(keys, idx, n, 8, radix_temp, s);
   hipLaunchKernelGGL(k_permute_items, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, items,

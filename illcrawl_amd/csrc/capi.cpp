@@ -240,7 +240,7 @@ ilc_status ilc_psg_run(ilc_psg* h, void* stream) {
     ensure_cubic(h);
     point_view p{h->pts, static_cast<uint32_t>(h->npts), h->lnx, h->lny};
     launch_gather(h->grid.view(), p, h->mode == ILC_MODE_REFERENCE ? OP_REFERENCE : OP_EXACT,
-                  h->kernel, h->ts, h->acc.p, nullptr, h->cubic.p, as_stream(stream));
+                  h->kernel, sum_shape_of(h->ts, h->npts), h->acc.p, nullptr, h->cubic.p, as_stream(stream));
   });
 }
 
@@ -346,7 +346,7 @@ ilc_status ilc_psg_count_evals(ilc_psg* h, uint64_t* counts_dev, uint64_t* total
     h->cnt_scratch.ensure(1);
     launch_fill_u32(reinterpret_cast<uint32_t*>(h->cnt.p), 0u, 2 * h->npts, s);
     point_view p{h->pts, static_cast<uint32_t>(h->npts), h->lnx, h->lny};
-    launch_gather(h->grid.view(), p, OP_COUNT, h->kernel, h->ts, nullptr, h->cnt.p, nullptr, s);
+    launch_gather(h->grid.view(), p, OP_COUNT, h->kernel, sum_shape_of(h->ts, h->npts), nullptr, h->cnt.p, nullptr, s);
     if (counts_dev)
       ILC_HIP(hipMemcpyAsync(counts_dev, h->cnt.p, sizeof(unsigned long long) * h->npts,
                              hipMemcpyDeviceToDevice, s));

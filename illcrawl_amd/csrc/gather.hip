@@ -3,9 +3,8 @@
 // Replaces projective_smoothing_grid -> spg_run_reconstruction
 // (projective_smoothing_backend_grid.cl:30-56, smoothing_particle_grid.cl:31-127).
 //
-// One 256-thread workgroup (4 waves of 64) owns a tile of TW x TH points of
-// the point array seen as an image; each thread owns PPT points of one column.
-// The workgroup
+// One 256-thread workgroup (4 waves of 64) owns a tile of T x T points (16 or
+// 8) of the point array seen as an image.  The workgroup
 //   1. loads its points and, in reference mode, each point's search box
 //      exactly as the reference computes it (cell of the point, radius =
 //      min(max_h[cell] + cell_radius, max_h), index box of p -/+ radius, from
@@ -13,23 +12,28 @@
 //   2. reduces the tile's bounding box and the union / intersection of the
 //      points' index boxes;
 //   3. visits the candidate cells 256 at a time, skips every cell whose max h
-//      cannot reach the tile, and streams the particles of the others with a
-//      block-wide offset table (coalesced 16-byte loads).  A cell holds its
-//      particles by descending h, so a binary search on h finds the prefix
-//      that can reach the tile and the rest is never read;
+//      cannot reach the tile, and builds an offset table of the others'
+//      particles.  A cell holds its particles by descending h, so a binary
+//      search on h finds the prefix that can reach the tile and the rest is
+//      never read.
+// The waves then stream the chunk's particles, 64 at a time in turn
+// (coalesced 16-byte loads).  Each wave
 //   4. culls each particle against the tile (support disk vs tile box) and
-//      compacts the survivors into LDS lists with wave ballots:
+//      compacts the survivors into its own LDS lists with ballots:
+//        far    - (16x16 tiles) the tile lies well inside its support: summed
+//                 at 64 nodes and interpolated, see is_far;
 //        big    - every point may use it and its support is at least twice
-//                 the tile's half-diagonal: stored as the coefficients of
-//                 its kernel argument expanded about the tile centre;
+//                 the tile's half-diagonal: stored, like far, as the
+//                 coefficients of its kernel argument expanded about the
+//                 tile centre;
 //        small  - every point may use it, stored by position;
-//        masked - reference mode, its cell is inside some points' index box
-//                 and outside others': stored by position and cell;
-//   5. when a list is full, every thread evaluates the listed particles for
-//      its points from LDS (broadcast reads), FP32 over 32 particles, then
-//      into a per-point FP64 accumulator.
-// The small and masked lists share one LDS array from its two ends (as the
-// big list's two kinds do), which keeps the workgroup at 17 KB of LDS.
+//        masked - reference mode, its cell may be inside some points' index
+//                 box and outside others': stored by position and cell;
+//   5. when a list is full, evaluates it from LDS (broadcast reads) for every
+//      point of the tile (far: every node), FP32 over 32 particles, then into
+//      FP64 accumulators.
+// At the end of the tile the waves' sums are added, in wave order, and the
+// far field is interpolated.
 //
 // Kernel arithmetic.  With c = coef^0.4, the quartic term coef*s^2.5,
 // s = 1 - r^2/h^2, equals (c*s)^2.5, and c*s is affine in the point's
@@ -109,7 +113,7 @@ __device__ inline uint32_t prefix_count(uint64_t mask) {
 }
 
 __device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
+__device__ inline float uniformf(float v) { return __int_as_float(uniform(__float_as_int(v))); }
 
 // Exclusive scan over the NB threads of the workgroup; *total = sum.
 // Contains two workgroup barriers.
@@ -987,24 +991,823 @@ __device__ __attribute__((always_inline)) inline void gather_tile(
   }
 }
 
-#ifndef ILC_WG64_WAVES
-#define ILC_WG64_WAVES 5
-#endif
-// waves per SIMD asked of the compiler: one point per lane keeps the
-// candidate pipeline's latency hidden behind many waves
-constexpr int gather_waves(int ppt, int nb) {
-  return ppt <= 1 ? 8 : (nb == 64 ? ILC_WG64_WAVES : (ppt <= 2 ? 5 : 4));
+// ---- the far field of a tile
+//
+// Over a tile well inside a particle's support the quartic's s^2.5 is smooth,
+// and the sum of all such particles is evaluated at 8 x 8 Chebyshev nodes of
+// the tile box instead of at its points, then interpolated once per point (in
+// FP64): a particle costs one wave 64 evaluations instead of the tile's 256.
+constexpr int kNodes = 8;
+// nodes cos((2 i + 1) pi / 16), and the Lagrange weights 1 / prod_{j != i}
+// (x_i - x_j) = (-1)^i 16 sin((2 i + 1) pi / 16)
+__device__ constexpr double kNodeX[kNodes] = {
+    0.98078528040323044913,  0.83146961230254523708,  0.55557023301960222474,
+    0.19509032201612826785,  -0.19509032201612826785, -0.55557023301960222474,
+    -0.83146961230254523708, -0.98078528040323044913};
+__device__ constexpr double kNodeW[kNodes] = {
+    16 * 0.19509032201612826785,  -16 * 0.55557023301960222474, 16 * 0.83146961230254523708,
+    -16 * 0.98078528040323044913, 16 * 0.98078528040323044913,  -16 * 0.83146961230254523708,
+    16 * 0.55557023301960222474,  -16 * 0.19509032201612826785};
+
+// the Lagrange basis of the nodes at u
+__device__ inline void node_basis(double u, double* b) {
+  double pre = 1.0;
+#pragma unroll
+  for (int i = 0; i < kNodes; ++i) {
+    b[i] = pre * kNodeW[i];
+    pre *= u - kNodeX[i];
+  }
+  double suf = 1.0;
+#pragma unroll
+  for (int i = kNodes - 1; i >= 0; --i) {
+    b[i] *= suf;
+    suf *= u - kNodeX[i];
+  }
 }
 
-template <int TW, int PPT, int OP, int KERNEL, int NB>
-__global__ __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(gather_waves(PPT, NB), 8))) void k_gather(grid_view g, point_view p, uint32_t tiles_x,
-                                                   uint32_t ntiles, double* __restrict__ acc_out,
-                                                   unsigned long long* __restrict__ counts,
-                                                   const float* __restrict__ cubic_table,
-                                                   float support) {
-  __shared__ gather_smem<OP == OP_REFERENCE, KERNEL, false, OP == OP_CLIP, NB> sm;
+// A particle at r from the tile centre is far when the tile's half-diagonal a
+// is at most (0.4 + 0.22 r / h) (h - r): the interpolation then errs by at
+// most 4e-8 of the particle's value at the tile centre (the largest over all
+// directions and r / h in [0, 0.99]; s^2.5 is singular at the support's edge
+// only, h - r and h + r away), below the FP32 rounding of the direct form.
+// ih2 = 1 / h^2, r2 = r^2, a2 = a^2.
+__device__ inline bool is_far(float r2, float ih2, float a2) {
+  const float x = __builtin_amdgcn_sqrtf(r2 * ih2);  // r / h
+  const float lim = fmaf(x, 0.22f, 0.4f) * (1.0f - x);
+  return x < 1.0f && a2 * ih2 <= lim * lim;
+}
+
+// ---- tiles of the sums (every op but the adjoint)
+//
+// A workgroup of 4 waves owns a tile of T x T points, and every wave works on
+// all of them (T * T / 64 per lane) with its own share of the candidates and
+// its own LDS lists: between the workgroup's cell chunks a wave never waits
+// for the others, and a list entry read from LDS serves T * T / 64 points per
+// lane.  The waves' sums are added once, at the end of the tile.  (With the
+// points dealt to the waves and shared lists, every 256 candidates cost two
+// workgroup barriers, and a tile of 64 points had one wave: one wave per tile
+// takes 1.25 ms for a 512^2 view of 1M particles, four 0.80, eight 0.79, at
+// 8x8 points; 6 frames of 160x120 1.12, 0.71, 0.73.)
+constexpr int kSumW = 4;
+
+// a wave evaluates a list when it reaches kWaveFlush entries; a batch of 64
+// candidates lands on a list of at most kWaveFlush - 1
+constexpr int kWaveFlush = 32;
+// one list, and two lists sharing an array from its two ends, with room to
+// pad either to a multiple of 4 entries
+constexpr int kWaveCap = kWaveFlush - 1 + 64 + 1;
+constexpr int kWavePool = 2 * (kWaveFlush - 1) + 64 + 6;
+static_assert(kWaveCap % 4 == 0 && kWavePool % 4 == 0, "whole groups of 4 entries");
+
+template <bool REF, int KERNEL, bool CLIP, bool COUNT>
+struct wave_lists {
+  static constexpr bool QUARTIC = KERNEL == 0 && !COUNT;
+  alignas(16) float4 X[QUARTIC ? kWavePool : 1];  // expansion form: far from the front, big from the back
+  float4 S[REF ? kWavePool : kWaveCap];  // position form: small from the front, masked from the back
+  alignas(16) int M[REF ? kWaveCap : 1];  // masked: packed cell (cx | cy << 16)
+  // line-of-sight clip: per entry, the depth range relative to the particle
+  // in units of h, times c^(1/2) (see clip_pow)
+  float2 Xz[CLIP ? kWavePool : 1];
+  float2 Sz[CLIP ? kWaveCap : 1];
+};
+
+template <int T, bool REF, int KERNEL, bool CLIP, bool COUNT>
+struct tile_smem {
+  static constexpr int W = kSumW, NB = 64 * W;
+  union {
+    wave_lists<REF, KERNEL, CLIP, COUNT> L[W];
+    struct {                      // at the end of the tile: the waves' sums
+      double sum[W][T * T];
+      double node[KERNEL == 0 && !CLIP && !COUNT && T * T > 64 ? W : 1][64];
+    };
+  };
+  int far_used;
+  float2 pt[T * T];          // the tile's points
+  uint2 box[REF ? T * T : 1];  // their search boxes: (x0 | xw << 16, y0 | yw << 16)
+  float tab[KERNEL == 2 ? kCubicTable : 1];
+  uint32_t cell_b[NB];
+  uint32_t cell_off[NB];
+  int cell_info[NB];  // cells: packed cell cx | cy << 16 (unsigned); rows: base key
+  int cell_y[NB];     // cells: 1 when in every point's search box; rows: the row's cy
+  uint32_t scan_ws[W];
+  float redf[W][5];
+  int redi[W][11];
+};
+
+// orders this wave's LDS accesses: its lists are written by some lanes and
+// read by others
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One tile (tx, ty) of the point image: everything between the point loads
+// and the accumulator update.  All threads of the workgroup call it with the
+// same arguments.
+template <int T, int OP, int KERNEL>
+__device__ __attribute__((always_inline)) inline void sum_tile(
+    const grid_view& g, const point_view& p, uint32_t tx, uint32_t ty, double* __restrict__ acc_out,
+    unsigned long long* __restrict__ counts, float support,
+    tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT>& sm,
+    float* __restrict__ img_out = nullptr, float img_scale = 1.0f, int fused = 0) {
+  constexpr int W = kSumW, NB = 64 * W, NP = T * T, PPT = NP / 64;
+  constexpr bool REF = OP == OP_REFERENCE;
+  constexpr bool COUNT = OP == OP_COUNT;
+  constexpr bool CLIP = OP == OP_CLIP;
+  constexpr bool QUARTIC = KERNEL == 0 && !COUNT;
+  // with one point per lane the nodes would save nothing
+  constexpr bool FAR = QUARTIC && !CLIP && PPT > 1;
+  static_assert(!CLIP || KERNEL == 0, "the line-of-sight clip is the quartic's");
+  static_assert(NP % 64 == 0, "whole points per lane");
+
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6;
+
+  // ---- the tile's points (thread t: points t, t + NB, ...), their search
+  // boxes, and the tile reductions
+  float bminx = INFINITY, bminy = INFINITY, bmaxx = -INFINITY, bmaxy = -INFINITY;
+  int ulx = INT32_MAX, uly = INT32_MAX, uhx = INT32_MIN, uhy = INT32_MIN;
+  int ilx = INT32_MIN, ily = INT32_MIN, ihx = INT32_MAX, ihy = INT32_MAX;
+  int anyz = 0, allz = 1, anyv = 0;
+  float minr = INFINITY;  // reference mode: the smallest search radius of the points
+#pragma unroll 1
+  for (int pt = t; pt < NP; pt += NB) {
+    const uint32_t px = tx * T + uint32_t(pt % T), py = ty * T + uint32_t(pt / T);
+    const uint32_t pid = py * p.lnx + px;
+    const bool pv = px < p.lnx && py < p.lny && pid < p.n;
+    float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (pv) q = p.gen ? pixel_point(p.pg, px, py) : p.pts[pid];
+    sm.pt[pt] = make_float2(q.x, q.y);
+    if constexpr (REF) sm.box[pt] = make_uint2(0xffffu, 0xffffu);  // no such cell in a grid of < 2^32
+    if (pv) {
+      anyv = 1;
+      bminx = fminf(bminx, q.x);
+      bmaxx = fmaxf(bmaxx, q.x);
+      bminy = fminf(bminy, q.y);
+      bmaxy = fmaxf(bmaxy, q.y);
+      if constexpr (REF) {
+        // search radius of spg_run_reconstruction (smoothing_particle_grid.cl:54-75)
+        const int32_t c0 = cell_of(q.x, 0.0f, g.minc[0], g.cs[0]);
+        const int32_t c1 = cell_of(q.y, 0.0f, g.minc[1], g.cs[1]);
+        const int32_t c2 = cell_of(q.z, 0.0f, g.minc[2], g.cs[2]);
+        const uint64_t nx = uint64_t(int64_t(g.nc[0])), ny = uint64_t(int64_t(g.nc[1]));
+        const uint64_t key = uint64_t(int64_t(c0)) + uint64_t(int64_t(c1)) * nx +
+                             uint64_t(int64_t(c2)) * nx * ny;
+        float R = g.max_h;
+        if (key < uint64_t(g.ncells)) {
+#pragma clang fp contract(off)
+          R = fminf(__uint_as_float(g.maxh_bits[key]) + g.cell_radius, g.max_h);
+        }
+        minr = fminf(minr, R);
+        const int lox = cell_of(q.x, -R, g.minc[0], g.cs[0]);
+        const int hix = cell_of(q.x, R, g.minc[0], g.cs[0]);
+        const int loy = cell_of(q.y, -R, g.minc[1], g.cs[1]);
+        const int hiy = cell_of(q.y, R, g.minc[1], g.cs[1]);
+        const int32_t loz = cell_of(q.z, -R, g.minc[2], g.cs[2]);
+        const int32_t hiz = cell_of(q.z, R, g.minc[2], g.cs[2]);
+        const bool zin = loz <= g.kz0 && g.kz0 <= hiz;
+        ilx = max(ilx, lox);
+        ihx = min(ihx, hix);
+        ily = max(ily, loy);
+        ihy = min(ihy, hiy);
+        allz &= int(zin);
+        if (zin) {
+          anyz = 1;
+          ulx = min(ulx, lox);
+          uhx = max(uhx, hix);
+          uly = min(uly, loy);
+          uhy = max(uhy, hiy);
+          // the box clamped to the cells a list entry can have (0..65535 per
+          // axis), as first cell and width
+          const int x0 = max(lox, 0), x1 = min(hix, 65535);
+          const int y0 = max(loy, 0), y1 = min(hiy, 65535);
+          if (x0 <= x1 && y0 <= y1)
+            sm.box[pt] = make_uint2(uint32_t(x0) | uint32_t(x1 - x0) << 16,
+                                    uint32_t(y0) | uint32_t(y1 - y0) << 16);
+        }
+      }
+    }
+  }
+  {
+    const float v0 = wmin(bminx), v1 = wmin(bminy), v2 = wmax(bmaxx), v3 = wmax(bmaxy);
+    int iv[11] = {0};
+    float v4 = INFINITY;
+    if constexpr (REF) {
+      v4 = wmin(minr);
+      iv[0] = wmini(ulx);
+      iv[1] = wmini(uly);
+      iv[2] = wmaxi(uhx);
+      iv[3] = wmaxi(uhy);
+      iv[4] = wmaxi(ilx);
+      iv[5] = wmaxi(ily);
+      iv[6] = wmini(ihx);
+      iv[7] = wmini(ihy);
+      iv[8] = wmaxi(anyz);
+      iv[9] = wmini(allz);
+    }
+    iv[10] = wmaxi(anyv);
+    if (lane == 0) {
+      sm.redf[wave][0] = v0;
+      sm.redf[wave][1] = v1;
+      sm.redf[wave][2] = v2;
+      sm.redf[wave][3] = v3;
+      sm.redf[wave][4] = v4;
+      for (int j = 0; j < 11; ++j) sm.redi[wave][j] = iv[j];
+    }
+  }
+  __syncthreads();
+  float tbx0 = INFINITY, tby0 = INFINITY, tbx1 = -INFINITY, tby1 = -INFINITY, r_minr = INFINITY;
+  int r_ulx = INT32_MAX, r_uly = INT32_MAX, r_uhx = INT32_MIN, r_uhy = INT32_MIN;
+  int r_ilx = INT32_MIN, r_ily = INT32_MIN, r_ihx = INT32_MAX, r_ihy = INT32_MAX;
+  int r_anyz = 0, r_allz = 1, any_valid = 0;
+  for (int w = 0; w < W; ++w) {
+    tbx0 = fminf(tbx0, sm.redf[w][0]);
+    tby0 = fminf(tby0, sm.redf[w][1]);
+    tbx1 = fmaxf(tbx1, sm.redf[w][2]);
+    tby1 = fmaxf(tby1, sm.redf[w][3]);
+    r_minr = fminf(r_minr, sm.redf[w][4]);
+    r_ulx = min(r_ulx, sm.redi[w][0]);
+    r_uly = min(r_uly, sm.redi[w][1]);
+    r_uhx = max(r_uhx, sm.redi[w][2]);
+    r_uhy = max(r_uhy, sm.redi[w][3]);
+    r_ilx = max(r_ilx, sm.redi[w][4]);
+    r_ily = max(r_ily, sm.redi[w][5]);
+    r_ihx = min(r_ihx, sm.redi[w][6]);
+    r_ihy = min(r_ihy, sm.redi[w][7]);
+    r_anyz |= sm.redi[w][8];
+    r_allz &= sm.redi[w][9];
+    any_valid |= sm.redi[w][10];
+  }
+  tbx0 = uniformf(tbx0);
+  tby0 = uniformf(tby0);
+  tbx1 = uniformf(tbx1);
+  tby1 = uniformf(tby1);
+  r_ilx = uniform(r_ilx);
+  r_ily = uniform(r_ily);
+  r_ihx = uniform(r_ihx);
+  r_ihy = uniform(r_ihy);
+  if (!uniform(any_valid)) {
+    __syncthreads();  // the reductions are read; the caller may start the next tile
+    return;
+  }
+
+  // tile centre: the origin of the expansion form
+  const float tcx = 0.5f * (tbx0 + tbx1), tcy = 0.5f * (tby0 + tby1);
+  // a particle is "big" when h >= 2 * tile half-diagonal
+  const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
+  const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
+  const float big_r2 = 4.0f * hd2 * 1.0001f + 1e-30f;
+
+  // ---- candidate cell box
+  int cx0, cx1, cy0, cy1, cz0, cz1;
+  if constexpr (REF) {
+    if (!uniform(r_anyz) || g.kz0 < 0 || g.kz0 >= g.nc[2]) {
+      cx0 = 1;
+      cx1 = 0;
+    } else {
+      cx0 = max(r_ulx, 0);
+      cx1 = min(r_uhx, g.nc[0] - 1);
+    }
+    cy0 = max(r_uly, 0);
+    cy1 = min(r_uhy, g.nc[1] - 1);
+    cz0 = cz1 = g.kz0;
+  } else {
+    // one extra cell on each side absorbs rounding in p -/+ reach
+    const float reach = support * g.max_h;
+    cx0 = max(max(cell_of(tbx0, -reach, g.minc[0], g.cs[0]), INT32_MIN + 1) - 1, 0);
+    cx1 = min(min(cell_of(tbx1, reach, g.minc[0], g.cs[0]), INT32_MAX - 1) + 1, g.nc[0] - 1);
+    cy0 = max(max(cell_of(tby0, -reach, g.minc[1], g.cs[1]), INT32_MIN + 1) - 1, 0);
+    cy1 = min(min(cell_of(tby1, reach, g.minc[1], g.cs[1]), INT32_MAX - 1) + 1, g.nc[1] - 1);
+    cz0 = 0;
+    cz1 = g.nc[2] - 1;
+  }
+  cx0 = uniform(cx0);
+  cx1 = uniform(cx1);
+  cy0 = uniform(cy0);
+  cy1 = uniform(cy1);
+  cz0 = uniform(cz0);
+  cz1 = uniform(cz1);
+  const bool allz_u = uniform(r_allz) != 0;
+  // A particle whose h is below every point's search radius R is in the box of
+  // every point its support covers: with |x - x_p| < h the particle's cell is
+  // at or above the box's first cell, floor((fl(x_p - R) - min) / w), since
+  // the cell arithmetic is monotone and fl(x_p - R) <= x once R - h exceeds
+  // half an ulp of x_p - R (the same on the other side and in y); at the other
+  // points it adds 0 either way.  The margin (1e-6 of the coordinates, 1e-5
+  // of R) also covers the rounding of the support test.  A dense cell's small
+  // particles thus need no box test: a slab's lists were 94% masked, since R
+  // takes the largest h of the cell over all depths (16 slabs of 2048^2, 32M
+  // cells: 21.9 -> 14.5 ms a render; a 256^2 crawler block of 600k rows: 6.0 ->
+  // 3.7 ms).
+  float unmask_ih2 = INFINITY;
+  if constexpr (REF) {
+    r_minr = uniformf(r_minr);
+    const float pmax = fmaxf(fmaxf(fabsf(tbx0), fabsf(tbx1)), fmaxf(fabsf(tby0), fabsf(tby1)));
+    const float rs = 0.99999f * r_minr - 1e-6f * (pmax + r_minr);
+    if (allz_u && rs > 0.0f && rs < INFINITY) unmask_ih2 = 1.0f / (rs * rs);
+  }
+  const float cull2 = COUNT ? support * support * 1.0001f : support * support;
+
+  double a64[PPT];
+  uint32_t cnt_acc[COUNT ? PPT : 1];
+#pragma unroll
+  for (int k = 0; k < PPT; ++k) a64[k] = 0.0;
+  if constexpr (COUNT)
+    for (int k = 0; k < PPT; ++k) cnt_acc[k] = 0;
+
+  auto& L = sm.L[wave];
+  // list sizes (wave-uniform)
+  int nf = 0, nb = 0, ns = 0, nm = 0;
+  // the far field: the sum at this lane's node, and whether the wave used it
+  double node64 = 0.0;
+  int far_used = 0;
+  if constexpr (FAR)
+    if (t == 0) sm.far_used = 0;
+
+  // ---- evaluation of the wave's lists for every point of the tile (lane l:
+  // points l, l + 64, ...).  Each pads its list to a multiple of 4 with
+  // entries that add nothing.
+  auto eval_big = [&]() {
+    if constexpr (QUARTIC) {
+      const int n = uniform(nb), n4 = (n + 3) & ~3;
+      if (lane < n4 - n) L.X[kWavePool - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (CLIP)
+        if (lane < n4 - n) L.Xz[kWavePool - 1 - (n + lane)] = make_float2(0.f, 0.f);
+      wave_sync();
+      float lx[PPT], ly[PPT], l2[PPT];
+#pragma unroll
+      for (int k = 0; k < PPT; ++k) {
+        const float2 e = sm.pt[lane + 64 * k];
+        lx[k] = e.x - tcx;
+        ly[k] = e.y - tcy;
+        l2[k] = fmaf(ly[k], ly[k], lx[k] * lx[k]);
+      }
+      for (int j0 = 0; j0 < n4; j0 += 32) {
+        const int jn = min(32, n4 - j0);
+        float a[PPT];
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
+        for (int j = 0; j < jn; j += 4) {
+          float4 q[4];
+          float2 z[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            q[u] = L.X[kWavePool - 1 - (j0 + j + u)];
+            if constexpr (CLIP) z[u] = L.Xz[kWavePool - 1 - (j0 + j + u)];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int k = 0; k < PPT; ++k) {
+              const float v = fmaf(q[u].y, lx[k], fmaf(q[u].z, ly[k], fmaf(q[u].w, l2[k], q[u].x)));
+              if constexpr (CLIP)
+                a[k] += clip_pow(v, z[u]);
+              else
+                a[k] += pow25(v);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
+      }
+      wave_sync();
+    }
+    nb = 0;
+  };
+  // far entries at the nodes (lane l: node l % 8, l / 8)
+  auto eval_far = [&]() {
+    if constexpr (FAR) {
+      const int n = uniform(nf), n4 = (n + 3) & ~3;
+      if (lane < n4 - n) L.X[n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      wave_sync();
+      float fx = 0.f, fy = 0.f;
+#pragma unroll
+      for (int i = 0; i < kNodes; ++i) {
+        if ((lane & 7) == i) fx = float(kNodeX[i]);
+        if ((lane >> 3) == i) fy = float(kNodeX[i]);
+      }
+      const float lx = hd_x * fx, ly = hd_y * fy;
+      const float l2 = fmaf(ly, ly, lx * lx);
+      for (int j0 = 0; j0 < n4; j0 += 32) {
+        const int jn = min(32, n4 - j0);
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < jn; j += 4) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float4 q = L.X[j0 + j + u];
+            a[u] += pow25(fmaf(q.y, lx, fmaf(q.z, ly, fmaf(q.w, l2, q.x))));
+          }
+        }
+        node64 += double((a[0] + a[1]) + (a[2] + a[3]));
+      }
+      wave_sync();
+      far_used = 1;
+    }
+    nf = 0;
+  };
+  auto eval_small = [&]() {
+    const int n = uniform(ns), n4 = (n + 3) & ~3;
+    if (lane < n4 - n) L.S[n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (CLIP)
+      if (lane < n4 - n) L.Sz[n + lane] = make_float2(0.f, 0.f);
+    wave_sync();
+    float ex[PPT], ey[PPT];
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) {
+      const float2 e = sm.pt[lane + 64 * k];
+      ex[k] = e.x;
+      ey[k] = e.y;
+    }
+    if constexpr (COUNT) {
+#pragma clang fp contract(off)
+      for (int j = 0; j < n; ++j) {
+        const float4 q = L.S[j];
+        const double hs = double(support) * double(q.z);
+        const double hs2 = hs * hs;
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) {
+          const double dx = double(q.x) - double(ex[k]);
+          const double dy = double(q.y) - double(ey[k]);
+          const double r2 = dx * dx + dy * dy;
+          cnt_acc[k] += (r2 < hs2) ? 1u : 0u;
+        }
+      }
+    } else {
+      for (int j0 = 0; j0 < n4; j0 += 32) {
+        const int jn = min(32, n4 - j0);
+        float a[PPT];
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
+        for (int j = 0; j < jn; j += 4) {
+          float4 q[4];
+          float2 z[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            q[u] = L.S[j0 + j + u];
+            if constexpr (CLIP) z[u] = L.Sz[j0 + j + u];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int k = 0; k < PPT; ++k) {
+              const float dx = q[u].x - ex[k], dy = q[u].y - ey[k];
+              const float r2 = fmaf(dy, dy, dx * dx);
+              if constexpr (KERNEL == 2)
+                a[k] = fmaf(q[u].z, cubic_shape(r2 * q[u].w, sm.tab), a[k]);
+              else if constexpr (CLIP)
+                a[k] += clip_pow(fmaf(-r2, q[u].z, q[u].w), z[u]);
+              else
+                a[k] += pow25(fmaf(-r2, q[u].z, q[u].w));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
+      }
+    }
+    wave_sync();
+    ns = 0;
+  };
+  // masked entries: each point tests the entry's cell against its own search
+  // box, as unsigned(cx - x0) <= width (and the same for y)
+  auto eval_masked = [&]() {
+    if constexpr (REF) {
+      const int n = uniform(nm), n4 = (n + 3) & ~3;
+      if (lane < n4 - n) {
+        L.S[kWavePool - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+        L.M[n + lane] = 0;
+      }
+      wave_sync();
+      float ex[PPT], ey[PPT];
+      uint2 bx[PPT];
+#pragma unroll
+      for (int k = 0; k < PPT; ++k) {
+        const float2 e = sm.pt[lane + 64 * k];
+        ex[k] = e.x;
+        ey[k] = e.y;
+        bx[k] = sm.box[lane + 64 * k];
+      }
+      for (int j0 = 0; j0 < n4; j0 += 32) {
+        const int jn = min(32, n4 - j0);
+        float a[PPT];
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
+        for (int j = 0; j < jn; j += 4) {
+          const int4 c4 = *reinterpret_cast<const int4*>(&L.M[j0 + j]);
+          const int cc[4] = {uniform(c4.x), uniform(c4.y), uniform(c4.z), uniform(c4.w)};
+          float4 q[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) q[u] = L.S[kWavePool - 1 - (j0 + j + u)];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint32_t cx = uint32_t(cc[u]) & 0xffffu, cy = uint32_t(cc[u]) >> 16;
+#pragma unroll
+            for (int k = 0; k < PPT; ++k) {
+              const bool in = cx - (bx[k].x & 0xffffu) <= bx[k].x >> 16 &&
+                              cy - (bx[k].y & 0xffffu) <= bx[k].y >> 16;
+              const float dx = q[u].x - ex[k], dy = q[u].y - ey[k];
+              const float r2 = fmaf(dy, dy, dx * dx);
+              a[k] = fmaf(in ? 1.0f : 0.0f, pow25(fmaf(-r2, q[u].z, q[u].w)), a[k]);
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
+      }
+      wave_sync();
+    }
+    nm = 0;
+  };
+
+  // ---- candidates.  The particles of the cells cx0..cx1 of one row (y, z)
+  // are contiguous in the sorted order, so the box's particles form nrows *
+  // nlays ranges.  Dense grids visit the box's cells NB at a time (x
+  // fastest) and skip the cells whose max h cannot reach the tile; sparse
+  // grids (well under one particle per cell, e.g. the depth-cut lists of a
+  // slab) stream the row ranges and cull per particle.  Both give the same
+  // candidates in the same order (rows, cells by x, particles in sorted
+  // order).  A sparse grid can still be dense where the tile is (a halo
+  // inside a slab): when the first chunk of rows holds more than
+  // kDenseRows particles per cell of the box, the tile switches to the cell
+  // enumeration, whose max-h skip and prefix search read far fewer.
+  const int ncols = cx1 >= cx0 ? cx1 - cx0 + 1 : 0;
+  const int nrows = cy1 >= cy0 ? cy1 - cy0 + 1 : 0;
+  const int nlays = cz1 >= cz0 ? cz1 - cz0 + 1 : 0;
+  // the box lies inside the grid, whose cells have 32-bit keys: 32-bit
+  // counts and indices (one layer, as in reference mode, skips a division)
+  const uint32_t ncand = uint32_t(ncols) * uint32_t(nrows) * uint32_t(nlays);
+  const uint32_t nrowz = ncols > 0 ? uint32_t(nrows) * uint32_t(nlays) : 0u;
+  const uint32_t nxny = uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
+  const float sup_h2 = support * support * 1.00002f;
+  bool rows_mode = g.sparse != 0 && ncand > uint32_t(NB);
+  const bool one_layer = nlays == 1;
+  uint64_t nitems = rows_mode ? nrowz : ncand;
+  for (uint64_t c0 = 0; c0 < nitems; c0 += NB) {
+    const bool in_box = c0 + uint64_t(t) < nitems;
+    const uint32_t ci = uint32_t(c0) + uint32_t(t);
+    uint32_t cb = 0, cn = 0;
+    int ccx = 0, ccy = 0, cfull = 0;
+    if (rows_mode) {
+      if (in_box) {
+        const uint32_t lay = one_layer ? 0u : ci / uint32_t(nrows);
+        ccy = cy0 + int(ci - lay * uint32_t(nrows));
+        const uint32_t kb = uint32_t(ccy) * uint32_t(g.nc[0]) + uint32_t(cz0 + int(lay)) * nxny;
+        cb = g.start[kb + uint32_t(cx0)];
+        cn = g.start[kb + uint32_t(cx1) + 1] - cb;
+        ccx = int(kb);  // stored as the row's base key
+      }
+    } else if (in_box) {
+      const uint32_t rest = ci / uint32_t(ncols);
+      const int col_c = int(ci - rest * uint32_t(ncols));
+      const uint32_t lay = one_layer ? 0u : rest / uint32_t(nrows);
+      ccx = cx0 + col_c;
+      ccy = cy0 + int(rest - lay * uint32_t(nrows));
+      const int ccz = cz0 + int(lay);
+      const uint32_t key = uint32_t(ccx) + uint32_t(ccy) * uint32_t(g.nc[0]) + uint32_t(ccz) * nxny;
+      cb = g.start[key];
+      const uint32_t ce = g.start[key + 1];
+      if (ce > cb) {
+        const float mh = __uint_as_float(g.maxh_bits[key]);
+        const float lo_x = g.minc[0] + float(ccx) * g.cs[0];
+        const float lo_y = g.minc[1] + float(ccy) * g.cs[1];
+        // a particle's cell comes from fl((x - min) / w): its coordinate can
+        // sit a few ulps of |x| + |min| outside the cell's float edges
+        const float mgx = 1e-4f * g.cs[0] + 4e-7f * (fabsf(g.minc[0]) + fabsf(lo_x) + g.cs[0]);
+        const float mgy = 1e-4f * g.cs[1] + 4e-7f * (fabsf(g.minc[1]) + fabsf(lo_y) + g.cs[1]);
+        const float dx = fmaxf(fmaxf((lo_x - mgx) - tbx1, tbx0 - (lo_x + g.cs[0] + mgx)), 0.0f);
+        const float dy = fmaxf(fmaxf((lo_y - mgy) - tby1, tby0 - (lo_y + g.cs[1] + mgy)), 0.0f);
+        const float d2c = dx * dx + dy * dy;
+        if (d2c < mh * mh * sup_h2) {
+          // the cell's particles come by descending h (to the top 16 bits of
+          // its pattern): only a prefix can reach the tile.  With h rounded
+          // up to its 16-bit bucket the test is monotone along the cell.
+          uint32_t lo = 0, hi = ce - cb;
+          while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            const float hu = __uint_as_float(__float_as_uint(g.hs[cb + mid]) | 0xffffu);
+            if (d2c < hu * hu * sup_h2)
+              lo = mid + 1;
+            else
+              hi = mid;
+          }
+          cn = lo;
+        }
+        if constexpr (REF)
+          cfull = (allz_u && ccy >= r_ily && ccy <= r_ihy && ccx >= r_ilx && ccx <= r_ihx) ? 1 : 0;
+      }
+    }
+    uint32_t tot;
+    const uint32_t coff = block_scan_excl<NB>(cn, &tot, sm.scan_ws);
+    tot = uint32_t(uniform(int(tot)));
+    if (rows_mode && c0 == 0 && uint64_t(tot) > uint64_t(kDenseRows) * ncand) {
+      // nothing of this chunk is in LDS yet: start over with the cells
+      rows_mode = false;
+      nitems = ncand;
+      c0 = uint64_t(0) - uint64_t(NB);
+      continue;
+    }
+    sm.cell_b[t] = cb;
+    sm.cell_off[t] = coff;
+    if (rows_mode) {
+      sm.cell_info[t] = ccx;
+      sm.cell_y[t] = ccy;
+    } else {
+      sm.cell_info[t] = int(uint32_t(ccx) | (uint32_t(ccy) << 16));
+      sm.cell_y[t] = cfull;
+    }
+    __syncthreads();
+    // the chunk's particles, 64 at a time, dealt to the waves in turn; after
+    // the last of them the wave's lists are evaluated whatever their size
+    // (here and not behind the loop: one copy of the evaluation code)
+    const bool last_chunk = c0 + NB >= nitems;
+    for (uint32_t v0 = uint32_t(wave) * 64u;; v0 += NB) {
+      const bool done = v0 >= tot;
+      if (done && !last_chunk) break;
+      const uint32_t v = v0 + uint32_t(lane);
+      float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+      bool keep = false, full = false, big = false, far = false;
+      int cinf = 0, cf = 0;
+      float2 tcl = make_float2(0.0f, 0.0f);
+      if (v < tot) {
+        // last cell whose offset is <= v (it has a nonzero count)
+        int lo = 0;
+#pragma unroll
+        for (int step = NB / 2; step > 0; step >>= 1)
+          if (sm.cell_off[lo + step] <= v) lo += step;
+        const uint32_t sidx = sm.cell_b[lo] + (v - sm.cell_off[lo]);
+        if constexpr (REF) {
+          cinf = sm.cell_info[lo];
+          cf = sm.cell_y[lo];
+          if (rows_mode) {
+            // the particle's cell from its key and the row's base key
+            const int px_c = int(g.key[sidx] - uint32_t(cinf));
+            const int py_c = cf;
+            cinf = int(uint32_t(px_c) | (uint32_t(py_c) << 16));
+            cf = (allz_u && py_c >= r_ily && py_c <= r_ihy && px_c >= r_ilx && px_c <= r_ihx) ? 1 : 0;
+          }
+        }
+        // (x, y, coef, 1/h^2); the quartic's z is c = coef^0.4
+        const float4 q = g.part[sidx];
+        if (q.z != 0.0f) {
+          const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
+          const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
+          const float d2 = fmaf(dy, dy, dx * dx);
+          keep = d2 * q.w < cull2;
+        }
+        if constexpr (CLIP) {
+          // the depth range relative to the particle, in units of h: its
+          // support must overlap it
+          const float2 zc = g.clip[sidx];
+          keep = keep && zc.x < 1.0f && zc.y > -1.0f;
+          const float rc = __builtin_amdgcn_sqrtf(q.z);
+          tcl = make_float2(zc.x * rc, zc.y * rc);
+        }
+        full = keep && (!REF || cf || q.w >= unmask_ih2);
+        if (keep) {
+          if constexpr (COUNT) {
+            e = make_float4(q.x, q.y, g.hs[sidx], 0.0f);
+          } else if constexpr (KERNEL == 2) {
+            e = q;
+          } else {
+            const float c = q.z;        // coef^0.4
+            const float ci2 = c * q.w;  // c / h^2
+            big = full && big_r2 * q.w <= 1.0f;
+            if (big) {
+              const float xr = q.x - tcx, yr = q.y - tcy;
+              const float d2r = fmaf(yr, yr, xr * xr);
+              e = make_float4(c * fmaf(-q.w, d2r, 1.0f), 2.0f * ci2 * xr, 2.0f * ci2 * yr, -ci2);
+              if constexpr (FAR) far = is_far(d2r, q.w, hd2);
+            } else {
+              e = make_float4(q.x, q.y, ci2, c);
+            }
+          }
+        }
+      }
+      const uint64_t bf = FAR ? __ballot(far) : 0ull;
+      const uint64_t bb = __ballot(big && !far);
+      const uint64_t bs = __ballot(full && !big);
+      const uint64_t bm = __ballot(keep && !full);
+      if constexpr (FAR)
+        if (far) L.X[nf + int(prefix_count(bf))] = e;
+      if constexpr (QUARTIC) {
+        if (big && !far) {
+          const int pos = kWavePool - 1 - (nb + int(prefix_count(bb)));
+          L.X[pos] = e;
+          if constexpr (CLIP) L.Xz[pos] = tcl;
+        }
+      }
+      if (full && !big) {
+        const int pos = ns + int(prefix_count(bs));
+        L.S[pos] = e;
+        if constexpr (CLIP) L.Sz[pos] = tcl;
+      }
+      if constexpr (REF) {
+        if (keep && !full) {
+          const int pos = nm + int(prefix_count(bm));
+          L.S[kWavePool - 1 - pos] = e;
+          L.M[pos] = cinf;
+        }
+      }
+      if constexpr (FAR) nf += __popcll(bf);
+      nb += __popcll(bb);
+      ns += __popcll(bs);
+      nm += __popcll(bm);
+      const int lim = done ? 1 : kWaveFlush;
+      if constexpr (FAR) {
+        if (done && !far_used && nf > 0) {
+          // too few far entries to pay for the tile's interpolation
+          const int n = uniform(nf);
+          const float4 x = lane < n ? L.X[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+          wave_sync();
+          if (lane < n) L.X[kWavePool - 1 - (nb + lane)] = x;
+          nb += n;
+          nf = 0;
+        }
+        if (nf >= lim) eval_far();
+      }
+      if (nb >= lim) eval_big();
+      if (ns >= lim) eval_small();
+      if (nm >= lim) eval_masked();
+      if (done) break;
+    }
+    __syncthreads();  // the cell table is rewritten by the next chunk
+  }
+  if constexpr (FAR)
+    if (far_used && lane == 0) sm.far_used = 1;
+
+  // ---- the waves' sums, in wave order
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PPT; ++k) {
+    double v = a64[k];
+    if constexpr (COUNT) v = double(cnt_acc[k]);
+    sm.sum[wave][lane + 64 * k] = v;
+  }
+  bool interp = false;
+  if constexpr (FAR) {
+    interp = sm.far_used != 0;
+    sm.node[wave][lane] = node64;
+  }
+  __syncthreads();
+  if constexpr (FAR && W > 1) {
+    if (interp) {
+      if (t < 64) {
+        double n = sm.node[0][t];
+        for (int w = 1; w < W; ++w) n += sm.node[w][t];
+        sm.node[0][t] = n;
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll 1
+  for (int pt = t; pt < NP; pt += NB) {
+    const uint32_t px = tx * T + uint32_t(pt % T), py = ty * T + uint32_t(pt / T);
+    const uint32_t pid = py * p.lnx + px;
+    if (!(px < p.lnx && py < p.lny && pid < p.n)) continue;
+    double v = sm.sum[0][pt];
+    for (int w = 1; w < W; ++w) v += sm.sum[w][pt];
+    if constexpr (FAR) {
+      if (interp) {
+        // the far field at the point
+        const float2 e = sm.pt[pt];
+        double bx[kNodes], by[kNodes];
+        node_basis(hd_x > 0.0f ? double(e.x - tcx) / double(hd_x) : 0.0, bx);
+        node_basis(hd_y > 0.0f ? double(e.y - tcy) / double(hd_y) : 0.0, by);
+        double f = 0.0;
+#pragma unroll
+        for (int iy = 0; iy < kNodes; ++iy) {
+          double r = 0.0;
+#pragma unroll
+          for (int ix = 0; ix < kNodes; ++ix) r = fma(bx[ix], sm.node[0][8 * iy + ix], r);
+          f = fma(by[iy], r, f);
+        }
+        v += f;
+      }
+    }
+    if constexpr (COUNT) {
+      if (counts) counts[pid] += static_cast<unsigned long long>(v);
+    } else if (fused) {
+      // the only visit of this point in the launch: no read of the
+      // accumulator, and the image as the retrieval computes it
+      acc_out[pid] = v;
+      img_out[pid] = static_cast<float>(v * static_cast<double>(img_scale));
+    } else {
+      acc_out[pid] += v;
+    }
+  }
+}
+
+// Waves per SIMD asked of the compiler: at 5 (96 VGPRs, 12 spilled in the
+// reference-mode batch) 32 views of a 16M snapshot take 50.0 ms, at 4 (no
+// spills) 53.5, at 3 60.2.  The LDS allows 5 workgroups per CU.
+constexpr int kSumWaves = 5;
+
+template <int T, int OP, int KERNEL>
+__global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSumWaves, 8))) void k_gather(
+    grid_view g, point_view p, uint32_t tiles_x, uint32_t ntiles, double* __restrict__ acc_out,
+    unsigned long long* __restrict__ counts, const float* __restrict__ cubic_table, float support) {
+  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT> sm;
   if constexpr (KERNEL == 2) {
-    for (int i = threadIdx.x; i < kCubicTable; i += NB) sm.tab[i] = cubic_table[i];
+    for (int i = threadIdx.x; i < kCubicTable; i += 64 * kSumW) sm.tab[i] = cubic_table[i];
   }
   // XCD-contiguous tile order: workgroups are dealt round-robin to the 8
   // XCDs, so give XCD x the x-th eighth of the tiles (shared L2 reuse of the
@@ -1013,7 +1816,7 @@ __global__ __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(gather_waves
   const uint32_t per = ntiles / 8u;
   const uint32_t tile = bid < per * 8u ? (bid % 8u) * per + bid / 8u : bid;
   const uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
-  gather_tile<TW, PPT, OP, KERNEL, NB>(g, p, tx, ty, acc_out, counts, support, sm);
+  sum_tile<T, OP, KERNEL>(g, p, tx, ty, acc_out, counts, support, sm);
 }
 
 // Persistent gather over (view, tile) items.  Workgroups are dealt to the 8
@@ -1022,17 +1825,14 @@ __global__ __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(gather_waves
 // on at a time are neighbours that read the same particle spans.  A
 // workgroup drains its XCD's queue, then helps with the others; every queue
 // counter only grows, so every workgroup leaves once all queues are empty.
-template <int TW, int PPT, int OP, int KERNEL, int NB>
-__global__ __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(gather_waves(PPT, NB), 8))) void k_gather_batch(const view_desc* __restrict__ views,
-                                                         const uint2* __restrict__ items,
-                                                         queue_segs segs,
-                                                         uint32_t* __restrict__ counters,
-                                                         const float* __restrict__ cubic_table,
-                                                         float support) {
-  __shared__ gather_smem<OP == OP_REFERENCE, KERNEL, false, OP == OP_CLIP, NB> sm;
+template <int T, int OP, int KERNEL>
+__global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSumWaves, 8))) void k_gather_batch(
+    const view_desc* __restrict__ views, const uint2* __restrict__ items, queue_segs segs,
+    uint32_t* __restrict__ counters, const float* __restrict__ cubic_table, float support) {
+  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT> sm;
   __shared__ uint32_t next;
   if constexpr (KERNEL == 2) {
-    for (int i = threadIdx.x; i < kCubicTable; i += NB) sm.tab[i] = cubic_table[i];
+    for (int i = threadIdx.x; i < kCubicTable; i += 64 * kSumW) sm.tab[i] = cubic_table[i];
   }
   const uint32_t home = blockIdx.x % uint32_t(kQueues);
   for (uint32_t k = 0; k < uint32_t(kQueues); ++k) {
@@ -1048,9 +1848,8 @@ __global__ __launch_bounds__(NB) __attribute__((amdgpu_waves_per_eu(gather_waves
       const uint32_t vi = uint32_t(uniform(int(it.x))), ti = uint32_t(uniform(int(it.y)));
       const view_desc& vd = views[vi];
       const uint32_t tiles_x = vd.tiles_x;
-      gather_tile<TW, PPT, OP, KERNEL, NB>(vd.g, vd.p, ti % tiles_x, ti / tiles_x, vd.acc,
-                                           nullptr, support, sm, nullptr, vd.img, vd.scale,
-                                           vd.fused);
+      sum_tile<T, OP, KERNEL>(vd.g, vd.p, ti % tiles_x, ti / tiles_x, vd.acc, nullptr, support,
+                                 sm, vd.img, vd.scale, vd.fused);
     }
   }
 }
@@ -1090,78 +1889,61 @@ __global__ __launch_bounds__(kBlock) void k_unpermute4(const uint32_t* __restric
   od[i] = d[s];
 }
 
-template <int TW, int PPT, int OP, int KERNEL, int NB>
+template <int T, int OP, int KERNEL>
 struct plain_launcher {
   static int run(const grid_view& g, const point_view& p, double* acc,
                  unsigned long long* counts, const float* tab, float support, hipStream_t s) {
-    constexpr int TH = (NB / TW) * PPT;
-    const uint32_t tiles_x = (p.lnx + TW - 1) / TW;
-    const uint32_t tiles_y = (p.lny + TH - 1) / TH;
+    const uint32_t tiles_x = (p.lnx + T - 1) / T;
+    const uint32_t tiles_y = (p.lny + T - 1) / T;
     const uint32_t ntiles = tiles_x * tiles_y;
     if (!ntiles) return 0;
-    hipLaunchKernelGGL((k_gather<TW, PPT, OP, KERNEL, NB>), dim3(ntiles), dim3(NB), 0, s, g, p,
+    hipLaunchKernelGGL((k_gather<T, OP, KERNEL>), dim3(ntiles), dim3(64 * kSumW), 0, s, g, p,
                        tiles_x, ntiles, acc, counts, tab, support);
     ILC_HIP(hipGetLastError());
     return 0;
   }
 };
 
-template <int TW, int PPT, int OP, int KERNEL, int NB>
+template <int T, int OP, int KERNEL>
 struct batch_launcher {
   static int run(const view_desc* v, const uint2* it, const queue_segs& segs, uint32_t* c,
                  const float* tab, float sup, int grid, hipStream_t s) {
-    hipLaunchKernelGGL((k_gather_batch<TW, PPT, OP, KERNEL, NB>), dim3(grid), dim3(NB), 0, s, v,
+    hipLaunchKernelGGL((k_gather_batch<T, OP, KERNEL>), dim3(grid), dim3(64 * kSumW), 0, s, v,
                        it, segs, c, tab, sup);
     ILC_HIP(hipGetLastError());
     return 0;
   }
 };
 
-template <int TW, int PPT, int OP, int KERNEL, int NB>
+template <int T, int OP, int KERNEL>
 struct batch_occ {
   static int run() {
     int per_cu = 0;
     ILC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, k_gather_batch<TW, PPT, OP, KERNEL, NB>, NB, 0));
+        &per_cu, k_gather_batch<T, OP, KERNEL>, 64 * kSumW, 0));
     return per_cu;
   }
 };
 
-// dispatch over (tile shape, op, kernel) to F<TW, PPT, OP, KERNEL, NB>::run
-template <template <int, int, int, int, int> class F, class... A>
-int dispatch(const tile_shape& ts, int op, int kernel, A&&... a) {
-  auto by_op = [&](auto tw, auto ppt, auto nb) -> int {
-    constexpr int TW = decltype(tw)::value, PPT = decltype(ppt)::value;
-    constexpr int NB = decltype(nb)::value;
+// dispatch over (tile side, op, kernel) to F<T, OP, KERNEL>::run
+template <template <int, int, int> class F, class... A>
+int dispatch(const sum_shape& ts, int op, int kernel, A&&... a) {
+  auto by_op = [&](auto tt) -> int {
+    constexpr int T = decltype(tt)::value;
     if (op == OP_CLIP) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "the line-of-sight clip needs a quartic kernel");
-      return F<TW, PPT, OP_CLIP, 0, NB>::run(a...);
+      return F<T, OP_CLIP, 0>::run(a...);
     }
     if (op == OP_REFERENCE) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "reference mode uses the quartic kernel");
-      return F<TW, PPT, OP_REFERENCE, 0, NB>::run(a...);
+      return F<T, OP_REFERENCE, 0>::run(a...);
     }
-    if (kernel == ILC_KERNEL_CUBIC) return F<TW, PPT, OP_EXACT, 2, NB>::run(a...);
-    return F<TW, PPT, OP_EXACT, 0, NB>::run(a...);
+    if (kernel == ILC_KERNEL_CUBIC) return F<T, OP_EXACT, 2>::run(a...);
+    return F<T, OP_EXACT, 0>::run(a...);
   };
-  using I16 = std::integral_constant<int, 16>;
-  using I32 = std::integral_constant<int, 32>;
-  using I64 = std::integral_constant<int, 64>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I4 = std::integral_constant<int, 4>;
-  using W64 = std::integral_constant<int, 64>;
-  using W256 = std::integral_constant<int, 256>;
-  if (ts.nb == 256) {
-    if (ts.tw == 16 && ts.ppt == 1) return by_op(I16{}, I1{}, W256{});
-    if (ts.tw == 32 && ts.ppt == 2) return by_op(I32{}, I2{}, W256{});
-    if (ts.tw == 32 && ts.ppt == 4) return by_op(I32{}, I4{}, W256{});
-    if (ts.tw == 64 && ts.ppt == 4) return by_op(I64{}, I4{}, W256{});
-  } else if (ts.nb == 64) {
-    if (ts.tw == 16 && ts.ppt == 4) return by_op(I16{}, I4{}, W64{});
-    if (ts.tw == 8 && ts.ppt == 1) return by_op(std::integral_constant<int, 8>{}, I1{}, W64{});
-  }
-  fail(ILC_EINVAL, "gather: unsupported tile shape tw=%d ppt=%d nb=%d", ts.tw, ts.ppt, ts.nb);
+  if (ts.side == 16) return by_op(std::integral_constant<int, 16>{});
+  if (ts.side == 8) return by_op(std::integral_constant<int, 8>{});
+  fail(ILC_EINVAL, "gather: no tile of side %d", ts.side);
 }
 
 }  // namespace
@@ -1194,14 +1976,35 @@ void launch_unpermute4(const uint32_t* perm, uint32_t n, const float* a, const f
   ILC_HIP(hipGetLastError());
 }
 
-void tile_grid(const tile_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
-               uint32_t* ntiles) {
-  const uint32_t th = uint32_t(ts.nb / ts.tw) * uint32_t(ts.ppt);
-  *tiles_x = (lnx + ts.tw - 1) / ts.tw;
-  *ntiles = *tiles_x * ((lny + th - 1) / th);
+// 16x16 tiles list a candidate once per 256 points and sum the far particles
+// at 64 nodes; 8x8 tiles give four times the workgroups and waste fewer pairs
+// at the supports' edges.  Below kPointsFor16 points the launch cannot fill
+// the GPU with 16x16 tiles and the heaviest one sets its time.  One view of
+// 1M / 16M / 100k particles, 8x8 against 16x16 tiles: 300^2 points 0.64, 3.1,
+// 0.33 against 1.30, 4.8, 0.48 ms; 700^2 1.03, 3.9, 0.51 against 1.26, 4.3,
+// 0.52; 1024^2 1.59, 5.0, 0.75 against 1.51, 4.7, 0.62; 2048^2 4.8, 11.1, 2.2
+// against 3.0, 7.4, 1.2.
+constexpr uint64_t kPointsFor16 = 3u << 18;
+
+sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints) {
+  if (ts.nb == 256) {
+    if ((ts.tw == 16 && ts.ppt == 1) || (ts.tw == 32 && (ts.ppt == 2 || ts.ppt == 4)) ||
+        (ts.tw == 64 && ts.ppt == 4))
+      return sum_shape{npoints < kPointsFor16 ? 8 : 16};
+  } else if (ts.nb == 64) {
+    if (ts.tw == 16 && ts.ppt == 4) return sum_shape{16};
+    if (ts.tw == 8 && ts.ppt == 1) return sum_shape{8};
+  }
+  fail(ILC_EINVAL, "gather: unsupported tile shape tw=%d ppt=%d nb=%d", ts.tw, ts.ppt, ts.nb);
 }
 
-int gather_batch_grid(int op, int kernel, const tile_shape& ts) {
+void tile_grid(const sum_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
+               uint32_t* ntiles) {
+  *tiles_x = (lnx + ts.side - 1) / ts.side;
+  *ntiles = *tiles_x * ((lny + ts.side - 1) / ts.side);
+}
+
+int gather_batch_grid(int op, int kernel, const sum_shape& ts) {
   int dev = 0, cus = 0;
   ILC_HIP(hipGetDevice(&dev));
   ILC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1210,7 +2013,7 @@ int gather_batch_grid(int op, int kernel, const tile_shape& ts) {
 }
 
 void launch_gather_batch(const view_desc* views, const uint2* items, const queue_segs& segs,
-                         uint32_t* counters, int op, int kernel, const tile_shape& ts,
+                         uint32_t* counters, int op, int kernel, const sum_shape& ts,
                          const float* cubic_table, int grid_blocks, hipStream_t s) {
   if (kernel == ILC_KERNEL_CUBIC && !cubic_table)
     fail(ILC_EINVAL, "cubic gather without its table");
@@ -1222,12 +2025,12 @@ void launch_gather_batch(const view_desc* views, const uint2* items, const queue
 }
 
 void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
-                   const tile_shape& ts, double* acc, unsigned long long* counts,
+                   const sum_shape& ts, double* acc, unsigned long long* counts,
                    const float* cubic_table, hipStream_t s) {
   const float support = kernel == ILC_KERNEL_CUBIC ? 2.0f : 1.0f;
   if (op == OP_COUNT) {
     // the count has its own tile shape: its cost is independent of the render's
-    plain_launcher<32, 4, OP_COUNT, 0, 256>::run(g, p, nullptr, counts, nullptr, support, s);
+    plain_launcher<16, OP_COUNT, 0>::run(g, p, nullptr, counts, nullptr, support, s);
     return;
   }
   if (kernel == ILC_KERNEL_CUBIC && !cubic_table)

@@ -239,14 +239,23 @@ struct point_view {
 // OP_CLIP: exact mode with the line-of-sight kernel clip (grid_view::clip)
 enum gather_op { OP_REFERENCE = 0, OP_EXACT = 1, OP_COUNT = 2, OP_ADJOINT = 3, OP_CLIP = 4 };
 
+// The caller's tile, as the ABI states it (see sum_shape).
 struct tile_shape {
   int tw;         // tile width (points)
   int ppt;        // points per thread (tile height = nb/tw * ppt)
-  int nb = 256;   // threads per workgroup (one tile per workgroup)
+  int nb = 256;   // threads: 256 or 64
 };
 
+// The tiles that a launch over npoints points works in: side x side points
+// (16 or 8), one per workgroup.  64-thread shapes ask for their own side, the
+// others leave it to the number of points.
+struct sum_shape {
+  int side;
+};
+sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints);
+
 void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
-                   const tile_shape& ts, double* acc, unsigned long long* counts,
+                   const sum_shape& ts, double* acc, unsigned long long* counts,
                    const float* cubic_table, hipStream_t s);
 
 // Adjoint of the exact-mode gather: adds into per-sorted-particle gradient
@@ -280,10 +289,10 @@ struct view_desc {
 };
 
 // tiles of a point image for a tile shape
-void tile_grid(const tile_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
+void tile_grid(const sum_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
                uint32_t* ntiles);
 // workgroups of the persistent batch gather that fit on the device at once
-int gather_batch_grid(int op, int kernel, const tile_shape& ts);
+int gather_batch_grid(int op, int kernel, const sum_shape& ts);
 // Work items split into kQueues queues (queue q: items[seg[q] .. seg[q+1])):
 // a workgroup drains the queue of its XCD (blockIdx % kQueues) first, then
 // the others.  counters: kQueues counters kQueueStride words apart, zeroed.
@@ -296,10 +305,10 @@ struct queue_segs {
 // most particles under them first (stable inside a cost class).  keys, idx:
 // n words each; radix_temp: radix_temp_words(n); out: n items.
 void launch_order_items(const view_desc* views, const uint2* items, const queue_segs& segs,
-                        uint32_t n, const tile_shape& ts, uint32_t* keys, uint32_t* idx,
+                        uint32_t n, const sum_shape& ts, uint32_t* keys, uint32_t* idx,
                         uint32_t* radix_temp, uint2* out, hipStream_t s);
 void launch_gather_batch(const view_desc* views, const uint2* items, const queue_segs& segs,
-                         uint32_t* counters, int op, int kernel, const tile_shape& ts,
+                         uint32_t* counters, int op, int kernel, const sum_shape& ts,
                          const float* cubic_table, int grid_blocks, hipStream_t s);
 
 // ---- project.hip

@@ -69,7 +69,7 @@ typedef struct {
                                         (dm_reconstruction_backend_grid.hpp:39) */
   int mode;                          /* ilc_mode */
   int kernel;                        /* ilc_kernel */
-  int tile_w, tile_h;                /* gather tile in points; 0 -> autotuned default */
+  int tile_w, tile_h;                /* gather tile in points; 0 -> default */
 } ilc_psg_config;
 
 typedef struct {
@@ -454,13 +454,13 @@ ilc_status ilc_batch_backward(ilc_batch* b, const float* const* dl_dimage_dev, f
  * of the last non-graph render: the one persistent launch, or the sum of the
  * per-view launches of a plain render.  Measurement only. */
 ilc_status ilc_batch_last_gather_ms(const ilc_batch* b, float* ms);
-/* Gather tile (points); tile_w * tile_h must be a multiple of 256.  One
- * tile per workgroup of 256 threads. */
+/* Gather tile (points); tile_w * tile_h must be a multiple of 256.  The
+ * gather works in tiles of 16x16 or 8x8 points, whichever is faster for the
+ * launch's number of points. */
 ilc_status ilc_batch_set_tile(ilc_batch* b, int32_t tile_w, int32_t tile_h);
-/* The same with the workgroup size: 256 threads (the shapes of
- * ilc_batch_set_tile), or 64 (one wave per 16x16 tile, four points per
- * lane: four times the tiles in flight per CU, for latency-bound sparse
- * views).  No reference counterpart: tuning of this build's gather. */
+/* The same with a workgroup size: 256 (the shapes of ilc_batch_set_tile), or
+ * 64, which asks for tiles of exactly 16x16 or 8x8 points whatever the
+ * launch's size.  No reference counterpart: tuning of this build's gather. */
 ilc_status ilc_batch_set_tile_wg(ilc_batch* b, int32_t tile_w, int32_t tile_h,
                                  int32_t workgroup);
 /* The current tile shape and workgroup size (after ilc_batch_autotune). */
@@ -475,8 +475,8 @@ ilc_status ilc_batch_get_tile(const ilc_batch* b, int32_t* tile_w, int32_t* tile
  * exact mode and a quartic kernel; renders must be persistent (not plain),
  * and backward is not provided for it. */
 ilc_status ilc_batch_set_depth_clip(ilc_batch* b, int32_t clip);
-/* Times the batched render for each supported tile shape, keeps the
- * fastest and returns it (no reference counterpart: measurement-driven
+/* Times the batched render in 16x16 and in 8x8 tiles, keeps the
+ * faster and returns it (no reference counterpart: measurement-driven
  * tuning). */
 ilc_status ilc_batch_autotune(ilc_batch* b, int32_t* tile_w, int32_t* tile_h, double* best_ms,
                               void* stream);

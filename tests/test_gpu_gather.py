@@ -65,3 +65,77 @@ def test_search_box_is_skipped_only_where_it_drops_nothing(B, orc, spread, targe
         linf, s = rel_errors(got, ref)
         print(f"  tile={tile} linf={linf:.2e} sum={s:.2e}", flush=True)
         assert linf < LINF_TOL and s < SUM_TOL
+
+
+def batch_image(B, p4, h, view, tile, mode):
+    r = B.BatchRenderer(mode=mode, kernel="quartic_ref", tile=tile)
+    r.set_particles(p4[:, :3].copy(), p4[:, 3].copy(), h)
+    r.set_views([view])
+    r.render()
+    return r.image_f64(0).cpu().numpy().reshape(-1)
+
+
+@pytest.mark.parametrize("mode", ["reference", "exact"])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (1, 40), (33, 1), (8, 8), (17, 15), (50, 31)])
+def test_tiles_with_far_and_near_particles(B, orc, mode, nx, ny):
+    """Partial, one-row and one-column tiles of both sides, with supports from
+    a fraction of a pixel to many tiles wide: particles whose support covers a
+    tile (summed at the nodes), crosses it, or lies inside it."""
+    rng = np.random.default_rng(nx * 100 + ny)
+    n = 5000
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :2] = rng.uniform(-150, 150, (n, 2))
+    p4[:, 2] = rng.uniform(-10, 10, n)
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    h = np.exp(rng.uniform(np.log(0.3), np.log(120.0), n)).astype(np.float32)
+    view = dict(position=np.array([0.0, 0.0, -20.0]), look_at=np.array([0.0, 0.0, 1.0]),
+                roll=0.3, width=float(nx), nx=nx, ny=ny, depth=40.0)
+    cam = orc.Camera(view["position"], view["look_at"], view["roll"], view["width"], nx, ny)
+    pp = cam.project_particles(p4, view["depth"])
+    pts = cam.pixel_points()
+    ref = orc.Grid(pp, h).gather_ref(pts, acc_mode=1) if mode == "reference" else \
+        orc.gather_exact(pp, h, pts, kind=0)
+    for tile in ((16, 16, 64), (8, 8, 64), None):
+        got = batch_image(B, p4, h, view, tile, mode)
+        linf, s = rel_errors(got, ref)
+        print(f"tiles {nx}x{ny} {mode} tile={tile}: linf={linf:.2e} sum={s:.2e}", flush=True)
+        assert linf < LINF_TOL and s < SUM_TOL
+
+
+def test_tile_side_follows_the_number_of_points(B, orc):
+    """Both sides of the rule (16x16 tiles from 3 << 18 points): the images of
+    a lattice one row shorter and one row longer agree with the oracle on
+    sampled points."""
+    rng = np.random.default_rng(3)
+    n = 20000
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :2] = rng.uniform(-300, 300, (n, 2))
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    h = rng.uniform(2.0, 90.0, n).astype(np.float32)
+    nx = 1024
+    for ny in (767, 768):
+        pts = lattice(nx, ny, -200.0, -150.0, 0.39)
+        got = render(B, p4, h, pts, nx)
+        idx = rng.choice(nx * ny, 1200, replace=False)
+        ref = orc.Grid(p4, h).gather_ref(pts[idx], acc_mode=1)
+        linf, s = rel_errors(got[idx], ref)
+        print(f"rule {nx}x{ny}: linf={linf:.2e} sum={s:.2e}", flush=True)
+        assert linf < LINF_TOL and s < SUM_TOL
+
+
+@pytest.mark.parametrize("kernel", ["quartic", "cubic"])
+def test_coincident_points(B, orc, kernel):
+    """A tile of no extent: every point the same."""
+    rng = np.random.default_rng(5)
+    n = 4000
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :2] = rng.uniform(-40, 40, (n, 2))
+    p4[:, 3] = 1.0
+    h = rng.uniform(1.0, 60.0, n).astype(np.float32)
+    pts = np.zeros((300, 4), np.float32)
+    pts[:, 0], pts[:, 1] = 1.25, -2.5
+    got = render(B, p4, h, pts, 20, mode="exact", kernel=kernel)
+    ref = orc.gather_exact(p4, h, pts[:1], kind={"quartic": 1, "cubic": 2}[kernel])
+    assert np.all(got == got[0])
+    # the cubic kernel is tabulated: the parity tests' 2e-5
+    assert abs(got[0] - ref[0]) / ref[0] < (2e-5 if kernel == "cubic" else LINF_TOL)

@@ -60,18 +60,9 @@ namespace ilc {
 
 namespace {
 
-// a workgroup of nb threads evaluates a list when it reaches flush_of(nb)
-// entries (one-wave workgroups: fewer, to keep their LDS small)
-constexpr int flush_of(int nb) { return nb >= 256 ? 64 : 32; }
-// list capacity (entries): a batch of nb candidates lands on a list holding
-// at most flush_of(nb) - 1
-constexpr int cap_of(int nb) { return nb >= 256 ? 320 : 96; }
-constexpr int kCap = cap_of(256);
 // a tile of a sparse grid leaves the row streaming for the cell enumeration
 // above this many particles per candidate cell
 constexpr uint32_t kDenseRows = 2;
-static_assert(flush_of(256) - 1 + 256 <= cap_of(256) && flush_of(64) - 1 + 64 <= cap_of(64),
-              "list capacity");
 constexpr int kCubicTable = 4096;
 
 __device__ inline int32_t floor_to_int(float f) {
@@ -174,7 +165,7 @@ __device__ inline float cubic_shape(float u, const float* tab) {
   return fmaf(f, b - a, a);
 }
 
-// Adjoint inputs and outputs (OP_ADJOINT only).
+// Adjoint inputs and outputs.
 struct adjoint_io {
   const float* grad;  // dL/d(point value), one per point
   float scale;        // points' value = scale * accumulator
@@ -187,544 +178,109 @@ struct adjoint_io {
   float* gy;
 };
 
-// the small and masked lists share one array from its two ends: before a
-// batch of nb candidates each holds at most flush_of(nb) - 1 entries
-constexpr int pool_of(int nb) { return cap_of(nb) + flush_of(nb); }
-static_assert(2 * (flush_of(256) - 1) + 256 <= pool_of(256) &&
-                  2 * (flush_of(64) - 1) + 64 <= pool_of(64),
-              "pool capacity");
+// ---- the far field of a tile
+//
+// Over a tile well inside a particle's support the quartic's s^2.5 is smooth,
+// and the sum of all such particles is evaluated at 8 x 8 Chebyshev nodes of
+// the tile box instead of at its points, then interpolated once per point (in
+// FP64): a particle costs one wave 64 evaluations instead of the tile's 256.
+constexpr int kNodes = 8;
+// nodes cos((2 i + 1) pi / 16), and the Lagrange weights 1 / prod_{j != i}
+// (x_i - x_j) = (-1)^i 16 sin((2 i + 1) pi / 16)
+__device__ constexpr double kNodeX[kNodes] = {
+    0.98078528040323044913,  0.83146961230254523708,  0.55557023301960222474,
+    0.19509032201612826785,  -0.19509032201612826785, -0.55557023301960222474,
+    -0.83146961230254523708, -0.98078528040323044913};
+__device__ constexpr double kNodeW[kNodes] = {
+    16 * 0.19509032201612826785,  -16 * 0.55557023301960222474, 16 * 0.83146961230254523708,
+    -16 * 0.98078528040323044913, 16 * 0.98078528040323044913,  -16 * 0.83146961230254523708,
+    16 * 0.55557023301960222474,  -16 * 0.19509032201612826785};
 
-template <bool REF, int KERNEL, bool ADJ = false, bool CLIP = false, int NB = 256>
-struct gather_smem {
-  static constexpr int CAP = cap_of(NB), POOL = pool_of(NB);
-  float4 Lb[KERNEL == 0 && !ADJ ? CAP : 1];  // big: expansion coefficients
-  // small (position form) from the front; reference mode: masked (position
-  // form) from the back, the m-th at Ls[POOL - 1 - m]
-  float4 Ls[REF ? POOL : CAP];
-  alignas(16) int Lmc[REF ? CAP : 1];  // masked: packed cell (cx | cy << 16)
-  // line-of-sight clip: per big / small entry, the depth range relative to
-  // the particle in units of h, times c^(1/2) (see clip_pow)
-  float2 Lbz[CLIP ? CAP : 1];
-  float2 Lsz[CLIP ? CAP : 1];
-  uint32_t wcnt[2][16];
-  float redf[4][REF ? 5 : 4];
-  int redi[4][10];
-  float tab[KERNEL == 2 ? kCubicTable : 1];
-  float dtab[KERNEL == 2 && ADJ ? kCubicTable : 1];
-  uint32_t cell_b[NB];
-  uint32_t cell_off[NB];
-  int cell_info[NB];  // cells: packed cell cx | cy << 16 (unsigned); rows: base key
-  int cell_y[NB];     // cells: 1 when in every point's search box; rows: the row's cy
-  uint32_t scan_ws[4];
-  uint32_t Lidx[ADJ ? CAP : 1];    // adjoint: sorted particle index
-  float4 Pt[ADJ ? NB * 4 : 1];  // adjoint: tile points (x, y, dL/dvalue, -), row-major
-  float4 Sb[ADJ ? 16 : 1];          // adjoint: 8x8 point blocks' boxes (x0, y0, x1, y1)
+// the Lagrange basis of the nodes at u
+__device__ inline void node_basis(double u, double* b) {
+  double pre = 1.0;
+#pragma unroll
+  for (int i = 0; i < kNodes; ++i) {
+    b[i] = pre * kNodeW[i];
+    pre *= u - kNodeX[i];
+  }
+  double suf = 1.0;
+#pragma unroll
+  for (int i = kNodes - 1; i >= 0; --i) {
+    b[i] *= suf;
+    suf *= u - kNodeX[i];
+  }
+}
+
+// A particle at r from the tile centre is far when the tile's half-diagonal a
+// is at most (0.4 + 0.22 r / h) (h - r): the interpolation then errs by at
+// most 4e-8 of the particle's value at the tile centre (the largest over all
+// directions and r / h in [0, 0.99]; s^2.5 is singular at the support's edge
+// only, h - r and h + r away), below the FP32 rounding of the direct form.
+// The adjoint's s^1.5 meets the same bound with a slope of 0.16.
+// ih2 = 1 / h^2, r2 = r^2, a2 = a^2.
+__device__ inline bool is_far(float r2, float ih2, float a2, float slope = 0.22f) {
+  const float x = __builtin_amdgcn_sqrtf(r2 * ih2);  // r / h
+  const float lim = fmaf(x, slope, 0.4f) * (1.0f - x);
+  return x < 1.0f && a2 * ih2 <= lim * lim;
+}
+
+// ---- tiles of the sums (every op but the adjoint)
+//
+// A workgroup of 4 waves owns a tile of T x T points, and every wave works on
+// all of them (T * T / 64 per lane) with its own share of the candidates and
+// its own LDS lists: between the workgroup's cell chunks a wave never waits
+// for the others, and a list entry read from LDS serves T * T / 64 points per
+// lane.  The waves' sums are added once, at the end of the tile.  (With the
+// points dealt to the waves and shared lists, every 256 candidates cost two
+// workgroup barriers, and a tile of 64 points had one wave: one wave per tile
+// takes 1.25 ms for a 512^2 view of 1M particles, four 0.80, eight 0.79, at
+// 8x8 points; 6 frames of 160x120 1.12, 0.71, 0.73.)
+constexpr int kSumW = 4;
+
+// a wave evaluates a list when it reaches kWaveFlush entries; a batch of 64
+// candidates lands on a list of at most kWaveFlush - 1
+constexpr int kWaveFlush = 32;
+// one list, and two lists sharing an array from its two ends, with room to
+// pad either to a multiple of 4 entries
+constexpr int kWaveCap = kWaveFlush - 1 + 64 + 1;
+constexpr int kWavePool = 2 * (kWaveFlush - 1) + 64 + 6;
+static_assert(kWaveCap % 4 == 0 && kWavePool % 4 == 0, "whole groups of 4 entries");
+
+template <bool REF, int KERNEL, bool CLIP, bool COUNT>
+struct wave_lists {
+  static constexpr bool QUARTIC = KERNEL == 0 && !COUNT;
+  alignas(16) float4 X[QUARTIC ? kWavePool : 1];  // expansion form: far from the front, big from the back
+  float4 S[REF ? kWavePool : kWaveCap];  // position form: small from the front, masked from the back
+  alignas(16) int M[REF ? kWaveCap : 1];  // masked: packed cell (cx | cy << 16)
+  // line-of-sight clip: per entry, the depth range relative to the particle
+  // in units of h, times c^(1/2) (see clip_pow)
+  float2 Xz[CLIP ? kWavePool : 1];
+  float2 Sz[CLIP ? kWaveCap : 1];
 };
 
-// One tile (tx, ty) of the point image: everything between the point loads
-// and the accumulator update.  All NB threads of the workgroup (NB / 64
-// waves) call it with the same arguments.
-template <int TW, int PPT, int OP, int KERNEL, int NB = 256>
-__device__ __attribute__((always_inline)) inline void gather_tile(
-    const grid_view& g, const point_view& p, uint32_t tx, uint32_t ty, double* __restrict__ acc_out,
-    unsigned long long* __restrict__ counts, float support,
-    gather_smem<OP == OP_REFERENCE, KERNEL, OP == OP_ADJOINT, OP == OP_CLIP, NB>& sm,
-    const adjoint_io* adj = nullptr, float* __restrict__ img_out = nullptr, float img_scale = 1.0f,
-    int fused = 0) {
-  constexpr int NW = NB / 64;
-  constexpr int kCap = cap_of(NB), kPool = pool_of(NB), kFlush = flush_of(NB);
-  constexpr int ROWS = NB / TW;
-  constexpr int TH = ROWS * PPT;
-  constexpr bool REF = OP == OP_REFERENCE;
-  constexpr bool COUNT = OP == OP_COUNT;
-  constexpr bool ADJ = OP == OP_ADJOINT;
-  constexpr bool CLIP = OP == OP_CLIP;
-  constexpr bool QUARTIC = KERNEL == 0 && !COUNT && !ADJ;
-  static_assert(!CLIP || KERNEL == 0, "the line-of-sight clip is the quartic's");
-  static_assert(!ADJ || (NB == 256 && PPT <= 4), "adjoint tile table");
+// The workgroup's chunk of candidate cells (or of rows of them).
+struct cell_table {
+  uint32_t b[64 * kSumW];    // first particle
+  uint32_t off[64 * kSumW];  // exclusive sum of the particles
+  int info[64 * kSumW];      // cells: packed cell cx | cy << 16 (unsigned); rows: base key
+  int y[64 * kSumW];         // cells: 1 when in every point's search box; rows: the row's cy
+  uint32_t scan_ws[kSumW];
+};
 
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  // Point ownership: the wave's 64 * PPT points, in row-major order within
-  // its (64 * PPT / TW) rows of the tile; lane l owns point
-  // 16 (l / 16 + 4 k) + l % 16 of them, k < PPT.
-  static_assert((64 * PPT) % TW == 0, "a wave covers whole rows");
-  constexpr int WROWS = (64 * PPT) / TW;
-  int prow[PPT], pcol[PPT];
-#pragma unroll
-  for (int k = 0; k < PPT; ++k) {
-    const int pw = 16 * ((lane >> 4) + 4 * k) + (lane & 15);
-    prow[k] = wave * WROWS + pw / TW;
-    pcol[k] = pw % TW;
-  }
-
-  float ex[PPT], ey[PPT];
-  uint32_t pid[PPT];
-  bool pv[PPT];
-  int lox[PPT], hix[PPT], loy[PPT], hiy[PPT];
-  bool zin[PPT];
-  double a64[PPT];
-  uint32_t cnt_acc[PPT];
-
-  float bminx = INFINITY, bminy = INFINITY, bmaxx = -INFINITY, bmaxy = -INFINITY;
-  int ulx = INT32_MAX, uly = INT32_MAX, uhx = INT32_MIN, uhy = INT32_MIN;
-  int ilx = INT32_MIN, ily = INT32_MIN, ihx = INT32_MAX, ihy = INT32_MAX;
-  int anyz = 0, allz = 1, anyv = 0;
-  float minr = INFINITY;  // reference mode: the smallest search radius of the points
-
-#pragma unroll
-  for (int k = 0; k < PPT; ++k) {
-    const uint32_t px = tx * TW + uint32_t(pcol[k]);
-    const uint32_t py = ty * TH + uint32_t(prow[k]);
-    pid[k] = py * p.lnx + px;
-    pv[k] = px < p.lnx && py < p.lny && pid[k] < p.n;
-    float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (pv[k]) q = p.gen ? pixel_point(p.pg, px, py) : p.pts[pid[k]];
-    ex[k] = q.x;
-    ey[k] = q.y;
-    a64[k] = 0.0;
-    cnt_acc[k] = 0;
-    lox[k] = hix[k] = loy[k] = hiy[k] = 0;
-    zin[k] = false;
-    if (pv[k]) {
-      anyv = 1;
-      bminx = fminf(bminx, q.x);
-      bmaxx = fmaxf(bmaxx, q.x);
-      bminy = fminf(bminy, q.y);
-      bmaxy = fmaxf(bmaxy, q.y);
-      if constexpr (REF) {
-        // search radius of spg_run_reconstruction (smoothing_particle_grid.cl:54-75)
-        const int32_t c0 = cell_of(q.x, 0.0f, g.minc[0], g.cs[0]);
-        const int32_t c1 = cell_of(q.y, 0.0f, g.minc[1], g.cs[1]);
-        const int32_t c2 = cell_of(q.z, 0.0f, g.minc[2], g.cs[2]);
-        const uint64_t nx = uint64_t(int64_t(g.nc[0])), ny = uint64_t(int64_t(g.nc[1]));
-        const uint64_t key = uint64_t(int64_t(c0)) + uint64_t(int64_t(c1)) * nx +
-                             uint64_t(int64_t(c2)) * nx * ny;
-        float R = g.max_h;
-        if (key < uint64_t(g.ncells)) {
-#pragma clang fp contract(off)
-          R = fminf(__uint_as_float(g.maxh_bits[key]) + g.cell_radius, g.max_h);
-        }
-        minr = fminf(minr, R);
-        lox[k] = cell_of(q.x, -R, g.minc[0], g.cs[0]);
-        hix[k] = cell_of(q.x, R, g.minc[0], g.cs[0]);
-        loy[k] = cell_of(q.y, -R, g.minc[1], g.cs[1]);
-        hiy[k] = cell_of(q.y, R, g.minc[1], g.cs[1]);
-        const int32_t loz = cell_of(q.z, -R, g.minc[2], g.cs[2]);
-        const int32_t hiz = cell_of(q.z, R, g.minc[2], g.cs[2]);
-        zin[k] = loz <= g.kz0 && g.kz0 <= hiz;
-        ilx = max(ilx, lox[k]);
-        ihx = min(ihx, hix[k]);
-        ily = max(ily, loy[k]);
-        ihy = min(ihy, hiy[k]);
-        allz &= int(zin[k]);
-        if (zin[k]) {
-          anyz = 1;
-          ulx = min(ulx, lox[k]);
-          uhx = max(uhx, hix[k]);
-          uly = min(uly, loy[k]);
-          uhy = max(uhy, hiy[k]);
-        }
-      }
-    }
-  }
-
-  // ---- tile reductions
-  {
-    const float v0 = wmin(bminx), v1 = wmin(bminy), v2 = wmax(bmaxx), v3 = wmax(bmaxy);
-    int iv[10] = {wmini(ulx), wmini(uly), wmaxi(uhx), wmaxi(uhy), wmaxi(ilx),
-                  wmaxi(ily), wmini(ihx), wmini(ihy), wmaxi(anyz), wmini(allz)};
-    const int av = wmaxi(anyv);
-    const float v4 = wmin(minr);
-    if (lane == 0) {
-      sm.redf[wave][0] = v0;
-      sm.redf[wave][1] = v1;
-      sm.redf[wave][2] = v2;
-      sm.redf[wave][3] = v3;
-      if constexpr (REF) sm.redf[wave][4] = v4;
-      for (int j = 0; j < 10; ++j) sm.redi[wave][j] = iv[j];
-      // waves without a valid point must not narrow the intersection
-      if (!av) {
-        sm.redi[wave][4] = INT32_MIN;
-        sm.redi[wave][5] = INT32_MIN;
-        sm.redi[wave][6] = INT32_MAX;
-        sm.redi[wave][7] = INT32_MAX;
-        sm.redi[wave][9] = 1;
-      }
-      sm.wcnt[0][wave] = av;
-    }
-  }
-  __syncthreads();
-  float tbx0 = sm.redf[0][0], tby0 = sm.redf[0][1], tbx1 = sm.redf[0][2], tby1 = sm.redf[0][3];
-  float r_minr = INFINITY;
-  if constexpr (REF) r_minr = sm.redf[0][4];
-  int r_ulx = sm.redi[0][0], r_uly = sm.redi[0][1], r_uhx = sm.redi[0][2], r_uhy = sm.redi[0][3];
-  int r_ilx = sm.redi[0][4], r_ily = sm.redi[0][5], r_ihx = sm.redi[0][6], r_ihy = sm.redi[0][7];
-  int r_anyz = sm.redi[0][8], r_allz = sm.redi[0][9];
-  int any_valid = sm.wcnt[0][0];
-  for (int w = 1; w < NW; ++w) {
-    tbx0 = fminf(tbx0, sm.redf[w][0]);
-    tby0 = fminf(tby0, sm.redf[w][1]);
-    tbx1 = fmaxf(tbx1, sm.redf[w][2]);
-    tby1 = fmaxf(tby1, sm.redf[w][3]);
-    if constexpr (REF) r_minr = fminf(r_minr, sm.redf[w][4]);
-    r_ulx = min(r_ulx, sm.redi[w][0]);
-    r_uly = min(r_uly, sm.redi[w][1]);
-    r_uhx = max(r_uhx, sm.redi[w][2]);
-    r_uhy = max(r_uhy, sm.redi[w][3]);
-    r_ilx = max(r_ilx, sm.redi[w][4]);
-    r_ily = max(r_ily, sm.redi[w][5]);
-    r_ihx = min(r_ihx, sm.redi[w][6]);
-    r_ihy = min(r_ihy, sm.redi[w][7]);
-    r_anyz = max(r_anyz, sm.redi[w][8]);
-    r_allz = min(r_allz, sm.redi[w][9]);
-    any_valid |= sm.wcnt[0][w];
-  }
-  __syncthreads();
-  if (!uniform(any_valid)) return;
-
-  if constexpr (ADJ) {
-    // the tile's points with their incoming gradients (0 outside the image),
-    // then the bounding box of the points with a nonzero gradient in each
-    // 8x8 block of the tile (one wave per block)
-    static_assert(TW == 32 && TH == 32, "adjoint tile is 32 x 32");
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-      const float gk = pv[k] ? adj->grad[pid[k]] * adj->scale : 0.0f;
-      sm.Pt[prow[k] * TW + pcol[k]] = make_float4(ex[k], ey[k], gk, 0.0f);
-    }
-    __syncthreads();
-    for (int sb = wave; sb < 16; sb += 4) {
-      const float4 q = sm.Pt[((sb >> 2) * 8 + (lane >> 3)) * TW + (sb & 3) * 8 + (lane & 7)];
-      const bool on = q.z != 0.0f;
-      const float x0 = wmin(on ? q.x : INFINITY), y0 = wmin(on ? q.y : INFINITY);
-      const float x1 = wmax(on ? q.x : -INFINITY), y1 = wmax(on ? q.y : -INFINITY);
-      if (lane == 0) sm.Sb[sb] = make_float4(x0, y0, x1, y1);
-    }
-    __syncthreads();
-    int live = 0;
-    for (int sb = 0; sb < 16; ++sb) live |= sm.Sb[sb].x <= sm.Sb[sb].z ? 1 : 0;
-    if (!uniform(live)) return;
-  }
-
-  // tile centre and the points relative to it (big-particle expansion)
-  const float tcx = 0.5f * (tbx0 + tbx1), tcy = 0.5f * (tby0 + tby1);
-  float lx[PPT], ly[PPT], l2[PPT];
-#pragma unroll
-  for (int k = 0; k < PPT; ++k) {
-    lx[k] = ex[k] - tcx;
-    ly[k] = ey[k] - tcy;
-    l2[k] = fmaf(ly[k], ly[k], lx[k] * lx[k]);
-  }
-  // a particle is "big" when h >= 2 * tile half-diagonal
-  const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
-  const float big_r2 = 4.0f * fmaf(hd_y, hd_y, hd_x * hd_x) * 1.0001f + 1e-30f;
-
-  // ---- candidate cell box
-  int cx0, cx1, cy0, cy1, cz0, cz1;
-  if constexpr (REF) {
-    if (!uniform(r_anyz) || g.kz0 < 0 || g.kz0 >= g.nc[2]) {
-      cx0 = 1;
-      cx1 = 0;
-    } else {
-      cx0 = max(r_ulx, 0);
-      cx1 = min(r_uhx, g.nc[0] - 1);
-    }
-    cy0 = max(r_uly, 0);
-    cy1 = min(r_uhy, g.nc[1] - 1);
-    cz0 = cz1 = g.kz0;
-  } else {
-    // one extra cell on each side absorbs rounding in p -/+ reach
-    const float reach = support * g.max_h;
-    cx0 = max(max(cell_of(tbx0, -reach, g.minc[0], g.cs[0]), INT32_MIN + 1) - 1, 0);
-    cx1 = min(min(cell_of(tbx1, reach, g.minc[0], g.cs[0]), INT32_MAX - 1) + 1, g.nc[0] - 1);
-    cy0 = max(max(cell_of(tby0, -reach, g.minc[1], g.cs[1]), INT32_MIN + 1) - 1, 0);
-    cy1 = min(min(cell_of(tby1, reach, g.minc[1], g.cs[1]), INT32_MAX - 1) + 1, g.nc[1] - 1);
-    cz0 = 0;
-    cz1 = g.nc[2] - 1;
-  }
-  cx0 = uniform(cx0);
-  cx1 = uniform(cx1);
-  cy0 = uniform(cy0);
-  cy1 = uniform(cy1);
-  cz0 = uniform(cz0);
-  cz1 = uniform(cz1);
-  const bool allz_u = uniform(r_allz) != 0;
-  // A particle whose h is below every point's search radius R is in the box of
-  // every point its support covers: with |x - x_p| < h the particle's cell is
-  // at or above the box's first cell, floor((fl(x_p - R) - min) / w), since
-  // the cell arithmetic is monotone and fl(x_p - R) <= x once R - h exceeds
-  // half an ulp of x_p - R (the same on the other side and in y); at the other
-  // points it adds 0 either way.  The margin (1e-6 of the coordinates, 1e-5
-  // of R) also covers the rounding of the support test.  A dense cell's small
-  // particles thus need no box test: a slab's lists were 94% masked, since R
-  // takes the largest h of the cell over all depths (16 slabs of 2048^2, 32M
-  // cells: 21.9 -> 14.5 ms a render; a 256^2 crawler block of 600k rows: 6.0 ->
-  // 3.7 ms).
-  float unmask_ih2 = INFINITY;
-  if constexpr (REF) {
-    const float pmax = fmaxf(fmaxf(fabsf(tbx0), fabsf(tbx1)), fmaxf(fabsf(tby0), fabsf(tby1)));
-    const float rs = 0.99999f * r_minr - 1e-6f * (pmax + r_minr);
-    if (allz_u && rs > 0.0f && rs < INFINITY) unmask_ih2 = 1.0f / (rs * rs);
-  }
-  const float cull2 = COUNT ? support * support * 1.0001f : support * support;
-  constexpr int kPoolN = REF ? kPool : kCap;
-
-  // list sizes (identical in every thread).  The big list holds the
-  // particles whose support covers the whole tile (argument positive at every
-  // point, no clamp) from the front of Lb, the others from the back.
-  int nb = 0, nbp = 0, ns = 0, nm = 0;
-  int slot = 0;
-
-  // ---- evaluation of the lists (loop bounds are wave-uniform)
-  auto eval_big = [&](int cnt, int cntp) {
-    if constexpr (QUARTIC) {
-      auto run = [&](int base, int n, auto clamp) {
-        n = uniform(n);
-        for (int j0 = 0; j0 < n; j0 += 32) {
-          const int jn = min(32, n - j0);
-          float a[PPT];
-#pragma unroll
-          for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
-          int j = 0;
-          for (; j + 4 <= jn; j += 4) {
-            float4 q[4];
-            float2 z[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              q[u] = sm.Lb[base + j0 + j + u];
-              if constexpr (CLIP) z[u] = sm.Lbz[base + j0 + j + u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-              for (int k = 0; k < PPT; ++k) {
-                const float v = fmaf(q[u].y, lx[k], fmaf(q[u].z, ly[k], fmaf(q[u].w, l2[k], q[u].x)));
-                if constexpr (CLIP)
-                  a[k] += clip_pow(v, z[u]);
-                else
-                  a[k] += decltype(clamp)::value ? pow25(v) : pow25_pos(v);
-              }
-          }
-          for (; j < jn; ++j) {
-            const float4 q = sm.Lb[base + j0 + j];
-#pragma unroll
-            for (int k = 0; k < PPT; ++k) {
-              const float v = fmaf(q.y, lx[k], fmaf(q.z, ly[k], fmaf(q.w, l2[k], q.x)));
-              if constexpr (CLIP)
-                a[k] += clip_pow(v, sm.Lbz[base + j0 + j]);
-              else
-                a[k] += decltype(clamp)::value ? pow25(v) : pow25_pos(v);
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
-        }
-      };
-      run(0, cnt, std::false_type{});
-      run(kCap - cntp, cntp, std::true_type{});
-    }
-  };
-  auto eval_small = [&](int cnt) {
-    cnt = uniform(cnt);
-    for (int j0 = 0; j0 < cnt; j0 += 32) {
-      const int jn = min(32, cnt - j0);
-      float a[PPT];
-#pragma unroll
-      for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
-      int j = 0;
-      if constexpr (!COUNT) {
-        for (; j + 4 <= jn; j += 4) {
-          float4 q[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) q[u] = sm.Ls[j0 + j + u];
-          float2 z[4];
-          if constexpr (CLIP) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) z[u] = sm.Lsz[j0 + j + u];
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-#pragma unroll
-            for (int k = 0; k < PPT; ++k) {
-              const float dx = q[u].x - ex[k], dy = q[u].y - ey[k];
-              const float r2 = fmaf(dy, dy, dx * dx);
-              if constexpr (KERNEL == 2)
-                a[k] = fmaf(q[u].z, cubic_shape(r2 * q[u].w, sm.tab), a[k]);
-              else if constexpr (CLIP)
-                a[k] += clip_pow(fmaf(-r2, q[u].z, q[u].w), z[u]);
-              else
-                a[k] += pow25(fmaf(-r2, q[u].z, q[u].w));
-            }
-          }
-        }
-      }
-      for (; j < jn; ++j) {
-        const float4 q = sm.Ls[j0 + j];
-        if constexpr (COUNT) {
-#pragma clang fp contract(off)
-          const double hs = double(support) * double(q.z);
-          const double hs2 = hs * hs;
-#pragma unroll
-          for (int k = 0; k < PPT; ++k) {
-            const double dx = double(q.x) - double(ex[k]);
-            const double dy = double(q.y) - double(ey[k]);
-            const double r2 = dx * dx + dy * dy;
-            cnt_acc[k] += (r2 < hs2) ? 1u : 0u;
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < PPT; ++k) {
-            const float dx = q.x - ex[k], dy = q.y - ey[k];
-            const float r2 = fmaf(dy, dy, dx * dx);
-            if constexpr (KERNEL == 2)
-              a[k] = fmaf(q.z, cubic_shape(r2 * q.w, sm.tab), a[k]);
-            else if constexpr (CLIP)
-              a[k] += clip_pow(fmaf(-r2, q.z, q.w), sm.Lsz[j0 + j]);
-            else
-              a[k] += pow25(fmaf(-r2, q.z, q.w));
-          }
-        }
-      }
-      if constexpr (!COUNT) {
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
-      }
-    }
-  };
-  // masked entries: each point tests the entry's cell against its own search
-  // box, as unsigned(cx - x0) <= width (and the same for y) on the box
-  // clamped to the cells a list entry can have (0..65535 per axis; an empty
-  // box or a point outside the grid layer fails every cell).  Four entries and
-  // their cells are read at once.
-  auto eval_masked = [&](int cnt) {
-    if constexpr (REF) {
-      cnt = uniform(cnt);
-      int bx0[PPT], by0[PPT];
-      uint32_t bxw[PPT], byw[PPT];
-#pragma unroll
-      for (int k = 0; k < PPT; ++k) {
-        const int x0 = max(lox[k], 0), x1 = min(hix[k], 65535);
-        const int y0 = max(loy[k], 0), y1 = min(hiy[k], 65535);
-        const bool ok = zin[k] && x0 <= x1 && y0 <= y1;
-        bx0[k] = ok ? x0 : INT32_MAX;
-        by0[k] = y0;
-        bxw[k] = ok ? uint32_t(x1 - x0) : 0u;
-        byw[k] = ok ? uint32_t(y1 - y0) : 0u;
-      }
-      auto add = [&](float* a, const float4& q, int c) {
-        const int cx = c & 0xffff, cy = int(uint32_t(c) >> 16);
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) {
-          const bool in = uint32_t(cx - bx0[k]) <= bxw[k] && uint32_t(cy - by0[k]) <= byw[k];
-          const float dx = q.x - ex[k], dy = q.y - ey[k];
-          const float r2 = fmaf(dy, dy, dx * dx);
-          a[k] = fmaf(in ? 1.0f : 0.0f, pow25(fmaf(-r2, q.z, q.w)), a[k]);
-        }
-      };
-      for (int j0 = 0; j0 < cnt; j0 += 32) {
-        const int jn = min(32, cnt - j0);
-        float a[PPT];
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) a[k] = 0.0f;
-        int j = 0;
-        for (; j + 4 <= jn; j += 4) {
-          const int4 cc = *reinterpret_cast<const int4*>(&sm.Lmc[j0 + j]);
-          float4 q[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) q[u] = sm.Ls[kPoolN - 1 - (j0 + j + u)];
-          add(a, q[0], uniform(cc.x));
-          add(a, q[1], uniform(cc.y));
-          add(a, q[2], uniform(cc.z));
-          add(a, q[3], uniform(cc.w));
-        }
-        for (; j < jn; ++j) add(a, sm.Ls[kPoolN - 1 - (j0 + j)], uniform(sm.Lmc[j0 + j]));
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) a64[k] += double(a[k]);
-      }
-    }
-  };
-
-  // adjoint: one listed particle per thread.  The thread visits the 8x8
-  // point blocks its support reaches and sums, over their points, five
-  // moments of g = dL/dvalue * s^1.5 (s = 1 - r^2/h^2); the weights are
-  // recomputed, not stored.  One atomic add per gradient component per
-  // particle and tile:
-  //   dL/dw = K/h^2        sum g s
-  //   dL/dh = w K/h^3      sum g (7 r^2/h^2 - 2)
-  //   dL/dx = -5 w K/h^4   sum g (x - x_point)     (same for y)
-  auto eval_adjoint = [&](int cnt) {
-    if constexpr (ADJ) {
-      cnt = uniform(cnt);
-      for (int j0 = 0; j0 < cnt; j0 += NB) {
-        const int j = j0 + t;
-        const bool act = j < cnt;
-        const float4 q = act ? sm.Ls[j] : make_float4(0.f, 0.f, 0.f, 0.f);  // (x, y, 1/h^2, coef)
-        float A0 = 0.f, A1 = 0.f, A2 = 0.f, A3 = 0.f, A4 = 0.f;
-        for (int sb = 0; sb < 16; ++sb) {
-          const float4 bx = sm.Sb[sb];
-          const float bdx = fmaxf(fmaxf(bx.x - q.x, q.x - bx.z), 0.0f);
-          const float bdy = fmaxf(fmaxf(bx.y - q.y, q.y - bx.w), 0.0f);
-          if (!(act && fmaf(bdy, bdy, bdx * bdx) * q.z < cull2)) continue;
-          const int base = (sb >> 2) * 8 * TW + (sb & 3) * 8;
-          for (int rr = 0; rr < 8; ++rr) {
-#pragma unroll
-            for (int cc = 0; cc < 8; ++cc) {
-              const float4 pt = sm.Pt[base + rr * TW + cc];
-              const float dx = q.x - pt.x, dy = q.y - pt.y;
-              const float r2 = fmaf(dy, dy, dx * dx);
-              if constexpr (KERNEL == 2) {
-                // F and dF/du at u = r^2/h^2, linear in the tables (0 beyond u = 4)
-                const float uu = r2 * q.z;
-                const float xx =
-                    fminf(uu * (float(kCubicTable - 1) / 4.0f), float(kCubicTable - 1));
-                const int ti = min(int(xx), kCubicTable - 2);
-                const float tf = xx - float(ti);
-                const float F = fmaf(tf, sm.tab[ti + 1] - sm.tab[ti], sm.tab[ti]);
-                const float D = fmaf(tf, sm.dtab[ti + 1] - sm.dtab[ti], sm.dtab[ti]);
-                const float gd = pt.z * D;
-                A0 = fmaf(pt.z, F, A0);
-                A1 = fmaf(gd, uu, A1);
-                A3 = fmaf(gd, dx, A3);
-                A4 = fmaf(gd, dy, A4);
-              } else {
-                const float sv = fmaxf(fmaf(-r2, q.z, 1.0f), 0.0f);
-                const float gq = pt.z * (sv * __builtin_amdgcn_sqrtf(sv));
-                A0 = fmaf(gq, sv, A0);
-                A1 += gq;
-                A2 = fmaf(gq, r2, A2);
-                A3 = fmaf(gq, dx, A3);
-                A4 = fmaf(gq, dy, A4);
-              }
-            }
-          }
-        }
-        if (act) {
-          const uint32_t si = sm.Lidx[j];
-          if constexpr (KERNEL == 2) {
-            // value = w K F(u) / h^2: d/dh = -2 w K / h^3 (F + u F'),
-            // d/dx = 2 w K / h^4 F' (x - x_point)
-            const float c2 = 2.0f * q.w * q.z;
-            atomicAdd(adj->gw + si, adj->norm * q.z * A0);
-            atomicAdd(adj->gh + si, -2.0f * q.w * __builtin_amdgcn_sqrtf(q.z) * (A0 + A1));
-            atomicAdd(adj->gx + si, c2 * A3);
-            atomicAdd(adj->gy + si, c2 * A4);
-          } else {
-            const float c5 = -5.0f * q.w * q.z;  // -5 w K / h^4
-            atomicAdd(adj->gw + si, adj->norm * q.z * A0);
-            atomicAdd(adj->gh + si,
-                      q.w * __builtin_amdgcn_sqrtf(q.z) * fmaf(7.0f * q.z, A2, -2.0f * A1));
-            atomicAdd(adj->gx + si, c5 * A3);
-            atomicAdd(adj->gy + si, c5 * A4);
-          }
-        }
-      }
-    }
-  };
-
+// Streams the candidate particles of the cell box [cx0, cx1] x [cy0, cy1] x
+// [cz0, cz1] for the tile box (tbx0, tby0, tbx1, tby1): calls batch(have,
+// sorted index, packed cell, in_all(cell), done) on the waves, 64 candidates
+// at a time dealt to the waves in turn, and once per wave at the end with
+// done set and no candidate.  Every thread of the workgroup takes part.
+template <bool REF, class InAll, class Batch>
+__device__ __attribute__((always_inline)) inline void stream_candidates(
+    const grid_view& g, int cx0, int cx1, int cy0, int cy1, int cz0, int cz1, float tbx0,
+    float tby0, float tbx1, float tby1, float support, InAll&& in_all, cell_table& ct,
+    Batch&& batch) {
   // ---- candidates.  The particles of the cells cx0..cx1 of one row (y, z)
   // are contiguous in the sorted order, so the box's particles form nrows *
-  // nlays ranges.  Dense grids visit the box's cells 256 at a time (x
+  // nlays ranges.  Dense grids visit the box's cells NB at a time (x
   // fastest) and skip the cells whose max h cannot reach the tile; sparse
   // grids (well under one particle per cell, e.g. the depth-cut lists of a
   // slab) stream the row ranges and cull per particle.  Both give the same
@@ -733,6 +289,9 @@ __device__ __attribute__((always_inline)) inline void gather_tile(
   // inside a slab): when the first chunk of rows holds more than
   // kDenseRows particles per cell of the box, the tile switches to the cell
   // enumeration, whose max-h skip and prefix search read far fewer.
+  constexpr int NB = 64 * kSumW;
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6;
   const int ncols = cx1 >= cx0 ? cx1 - cx0 + 1 : 0;
   const int nrows = cy1 >= cy0 ? cy1 - cy0 + 1 : 0;
   const int nlays = cz1 >= cz0 ? cz1 - cz0 + 1 : 0;
@@ -796,11 +355,11 @@ __device__ __attribute__((always_inline)) inline void gather_tile(
           cn = lo;
         }
         if constexpr (REF)
-          cfull = (allz_u && ccy >= r_ily && ccy <= r_ihy && ccx >= r_ilx && ccx <= r_ihx) ? 1 : 0;
+          cfull = in_all(ccx, ccy) ? 1 : 0;
       }
     }
     uint32_t tot;
-    const uint32_t coff = block_scan_excl<NB>(cn, &tot, sm.scan_ws);
+    const uint32_t coff = block_scan_excl<NB>(cn, &tot, ct.scan_ws);
     tot = uint32_t(uniform(int(tot)));
     if (rows_mode && c0 == 0 && uint64_t(tot) > uint64_t(kDenseRows) * ncand) {
       // nothing of this chunk is in LDS yet: start over with the cells
@@ -809,267 +368,53 @@ __device__ __attribute__((always_inline)) inline void gather_tile(
       c0 = uint64_t(0) - uint64_t(NB);
       continue;
     }
-    sm.cell_b[t] = cb;
-    sm.cell_off[t] = coff;
+    ct.b[t] = cb;
+    ct.off[t] = coff;
     if (rows_mode) {
-      sm.cell_info[t] = ccx;
-      sm.cell_y[t] = ccy;
+      ct.info[t] = ccx;
+      ct.y[t] = ccy;
     } else {
-      sm.cell_info[t] = int(uint32_t(ccx) | (uint32_t(ccy) << 16));
-      sm.cell_y[t] = cfull;
+      ct.info[t] = int(uint32_t(ccx) | (uint32_t(ccy) << 16));
+      ct.y[t] = cfull;
     }
     __syncthreads();
-    for (uint32_t v0 = 0; v0 < tot; v0 += NB) {
-      const uint32_t v = v0 + uint32_t(t);
-      float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
-      bool keep = false, full = false, big = false, cover = false;
+    // the chunk's particles, 64 at a time, dealt to the waves in turn; after
+    // the last of them the wave's lists are evaluated whatever their size
+    // (here and not behind the loop: one copy of the evaluation code)
+    const bool last_chunk = c0 + NB >= nitems;
+    for (uint32_t v0 = uint32_t(wave) * 64u;; v0 += NB) {
+      const bool done = v0 >= tot;
+      if (done && !last_chunk) break;
+      const uint32_t v = v0 + uint32_t(lane);
+      bool have = false;
+      uint32_t sidx = 0;
       int cinf = 0, cf = 0;
-      uint32_t adj_idx = 0;
-      float2 tcl = make_float2(0.0f, 0.0f);
       if (v < tot) {
         // last cell whose offset is <= v (it has a nonzero count)
         int lo = 0;
 #pragma unroll
         for (int step = NB / 2; step > 0; step >>= 1)
-          if (sm.cell_off[lo + step] <= v) lo += step;
-        const uint32_t sidx = sm.cell_b[lo] + (v - sm.cell_off[lo]);
-        cinf = sm.cell_info[lo];
+          if (ct.off[lo + step] <= v) lo += step;
+        sidx = ct.b[lo] + (v - ct.off[lo]);
         if constexpr (REF) {
-          if (!rows_mode) cf = sm.cell_y[lo];
+          cinf = ct.info[lo];
+          cf = ct.y[lo];
           if (rows_mode) {
             // the particle's cell from its key and the row's base key
             const int px_c = int(g.key[sidx] - uint32_t(cinf));
-            const int py_c = sm.cell_y[lo];
-            const int pf = (allz_u && py_c >= r_ily && py_c <= r_ihy && px_c >= r_ilx &&
-                            px_c <= r_ihx) ? 1 : 0;
+            const int py_c = cf;
             cinf = int(uint32_t(px_c) | (uint32_t(py_c) << 16));
-            cf = pf;
+            cf = in_all(px_c, py_c) ? 1 : 0;
           }
         }
-        // (x, y, coef, 1/h^2); the quartic's z is c = coef^0.4
-        const float4 q = g.part[sidx];
-        if (ADJ || q.z != 0.0f) {
-          const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
-          const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
-          const float d2 = fmaf(dy, dy, dx * dx);
-          keep = d2 * q.w < cull2;
-        }
-        if constexpr (CLIP) {
-          // the depth range relative to the particle, in units of h: its
-          // support must overlap it
-          const float2 zc = g.clip[sidx];
-          keep = keep && zc.x < 1.0f && zc.y > -1.0f;
-          const float rc = __builtin_amdgcn_sqrtf(q.z);
-          tcl = make_float2(zc.x * rc, zc.y * rc);
-        }
-        full = keep && (!REF || cf || q.w >= unmask_ih2);
-        if (keep) {
-          if constexpr (COUNT) {
-            e = make_float4(q.x, q.y, g.hs[sidx], 0.0f);
-          } else if constexpr (ADJ) {
-            // (x, y, 1/h^2, coef)
-            e = make_float4(q.x, q.y, q.w, KERNEL == 2 ? q.z : pow25_pos(q.z));
-            adj_idx = sidx;
-          } else if constexpr (KERNEL == 2) {
-            e = q;
-          } else {
-            const float c = q.z;        // coef^0.4
-            const float ci2 = c * q.w;  // c / h^2
-            big = full && big_r2 * q.w <= 1.0f;
-            if (big) {
-              const float xr = q.x - tcx, yr = q.y - tcy;
-              const float d2r = fmaf(yr, yr, xr * xr);
-              e = make_float4(c * fmaf(-q.w, d2r, 1.0f), 2.0f * ci2 * xr, 2.0f * ci2 * yr, -ci2);
-              // s >= 0.01 at every point of the tile box: far beyond the
-              // rounding of the expanded argument (~1e-6 of c)
-              const float fx = fmaxf(q.x - tbx0, tbx1 - q.x), fy = fmaxf(q.y - tby0, tby1 - q.y);
-              cover = fmaf(fy, fy, fx * fx) * q.w < 0.99f;
-            } else {
-              e = make_float4(q.x, q.y, ci2, c);
-            }
-          }
-        }
+        have = true;
       }
-      const uint64_t bb = __ballot(big && cover);
-      const uint64_t bp = __ballot(big && !cover);
-      const uint64_t bs = __ballot(full && !big);
-      const uint64_t bm = __ballot(keep && !full);
-      if (lane == 0) {
-        sm.wcnt[slot][wave] = __popcll(bb);
-        sm.wcnt[slot][4 + wave] = __popcll(bs);
-        sm.wcnt[slot][8 + wave] = __popcll(bm);
-        sm.wcnt[slot][12 + wave] = __popcll(bp);
-      }
-      __syncthreads();
-      int baseb = nb, basebp = nbp, bases = ns, basem = nm, totb = 0, totbp = 0, tots = 0,
-          totm = 0;
-      for (int w = 0; w < NW; ++w) {
-        const int cb_ = sm.wcnt[slot][w], cs_ = sm.wcnt[slot][4 + w],
-                  cm_ = sm.wcnt[slot][8 + w], cp_ = sm.wcnt[slot][12 + w];
-        if (w < wave) {
-          baseb += cb_;
-          basebp += cp_;
-          bases += cs_;
-          basem += cm_;
-        }
-        totb += cb_;
-        totbp += cp_;
-        tots += cs_;
-        totm += cm_;
-      }
-      if constexpr (QUARTIC) {
-        // nb + nbp <= kFlush - 1 + NB <= kCap: the two ends never meet
-        if (big && cover) {
-          const int pb = baseb + int(prefix_count(bb));
-          sm.Lb[pb] = e;
-          if constexpr (CLIP) sm.Lbz[pb] = tcl;
-        }
-        if (big && !cover) {
-          const int pc = kCap - 1 - (basebp + int(prefix_count(bp)));
-          sm.Lb[pc] = e;
-          if constexpr (CLIP) sm.Lbz[pc] = tcl;
-        }
-      }
-      if (full && !big) {
-        const int pos = bases + prefix_count(bs);
-        sm.Ls[pos] = e;
-        if constexpr (ADJ) sm.Lidx[pos] = adj_idx;
-        if constexpr (CLIP) sm.Lsz[pos] = tcl;
-      }
-      if constexpr (REF) {
-        if (keep && !full) {
-          const int pos = basem + prefix_count(bm);
-          sm.Ls[kPool - 1 - pos] = e;
-          sm.Lmc[pos] = cinf;
-        }
-      }
-      nb += totb;
-      nbp += totbp;
-      ns += tots;
-      nm += totm;
-      slot ^= 1;
-      if (nb + nbp >= kFlush || ns >= kFlush || nm >= kFlush) {
-        __syncthreads();
-        if constexpr (ADJ) {
-          eval_adjoint(ns);
-        } else {
-          eval_big(nb, nbp);
-          eval_small(ns);
-          eval_masked(nm);
-        }
-        __syncthreads();
-        nb = nbp = ns = nm = 0;
-      }
+      batch(have, sidx, cinf, cf != 0, done);
+      if (done) break;
     }
     __syncthreads();  // the cell table is rewritten by the next chunk
   }
-  if (nb > 0 || nbp > 0 || ns > 0 || nm > 0) {
-    __syncthreads();
-    if constexpr (ADJ) {
-      eval_adjoint(ns);
-    } else {
-      eval_big(nb, nbp);
-      eval_small(ns);
-      eval_masked(nm);
-    }
-  }
-  if constexpr (ADJ) return;
-
-#pragma unroll
-  for (int k = 0; k < PPT; ++k) {
-    if (!pv[k]) continue;
-    if constexpr (COUNT) {
-      if (counts) counts[pid[k]] += cnt_acc[k];
-    } else if (fused) {
-      // the only visit of this point in the launch: no read of the
-      // accumulator, and the image as the retrieval computes it
-      acc_out[pid[k]] = a64[k];
-      img_out[pid[k]] = static_cast<float>(a64[k] * static_cast<double>(img_scale));
-    } else {
-      acc_out[pid[k]] += a64[k];
-    }
-  }
 }
-
-// ---- the far field of a tile
-//
-// Over a tile well inside a particle's support the quartic's s^2.5 is smooth,
-// and the sum of all such particles is evaluated at 8 x 8 Chebyshev nodes of
-// the tile box instead of at its points, then interpolated once per point (in
-// FP64): a particle costs one wave 64 evaluations instead of the tile's 256.
-constexpr int kNodes = 8;
-// nodes cos((2 i + 1) pi / 16), and the Lagrange weights 1 / prod_{j != i}
-// (x_i - x_j) = (-1)^i 16 sin((2 i + 1) pi / 16)
-__device__ constexpr double kNodeX[kNodes] = {
-    0.98078528040323044913,  0.83146961230254523708,  0.55557023301960222474,
-    0.19509032201612826785,  -0.19509032201612826785, -0.55557023301960222474,
-    -0.83146961230254523708, -0.98078528040323044913};
-__device__ constexpr double kNodeW[kNodes] = {
-    16 * 0.19509032201612826785,  -16 * 0.55557023301960222474, 16 * 0.83146961230254523708,
-    -16 * 0.98078528040323044913, 16 * 0.98078528040323044913,  -16 * 0.83146961230254523708,
-    16 * 0.55557023301960222474,  -16 * 0.19509032201612826785};
-
-// the Lagrange basis of the nodes at u
-__device__ inline void node_basis(double u, double* b) {
-  double pre = 1.0;
-#pragma unroll
-  for (int i = 0; i < kNodes; ++i) {
-    b[i] = pre * kNodeW[i];
-    pre *= u - kNodeX[i];
-  }
-  double suf = 1.0;
-#pragma unroll
-  for (int i = kNodes - 1; i >= 0; --i) {
-    b[i] *= suf;
-    suf *= u - kNodeX[i];
-  }
-}
-
-// A particle at r from the tile centre is far when the tile's half-diagonal a
-// is at most (0.4 + 0.22 r / h) (h - r): the interpolation then errs by at
-// most 4e-8 of the particle's value at the tile centre (the largest over all
-// directions and r / h in [0, 0.99]; s^2.5 is singular at the support's edge
-// only, h - r and h + r away), below the FP32 rounding of the direct form.
-// ih2 = 1 / h^2, r2 = r^2, a2 = a^2.
-__device__ inline bool is_far(float r2, float ih2, float a2) {
-  const float x = __builtin_amdgcn_sqrtf(r2 * ih2);  // r / h
-  const float lim = fmaf(x, 0.22f, 0.4f) * (1.0f - x);
-  return x < 1.0f && a2 * ih2 <= lim * lim;
-}
-
-// ---- tiles of the sums (every op but the adjoint)
-//
-// A workgroup of 4 waves owns a tile of T x T points, and every wave works on
-// all of them (T * T / 64 per lane) with its own share of the candidates and
-// its own LDS lists: between the workgroup's cell chunks a wave never waits
-// for the others, and a list entry read from LDS serves T * T / 64 points per
-// lane.  The waves' sums are added once, at the end of the tile.  (With the
-// points dealt to the waves and shared lists, every 256 candidates cost two
-// workgroup barriers, and a tile of 64 points had one wave: one wave per tile
-// takes 1.25 ms for a 512^2 view of 1M particles, four 0.80, eight 0.79, at
-// 8x8 points; 6 frames of 160x120 1.12, 0.71, 0.73.)
-constexpr int kSumW = 4;
-
-// a wave evaluates a list when it reaches kWaveFlush entries; a batch of 64
-// candidates lands on a list of at most kWaveFlush - 1
-constexpr int kWaveFlush = 32;
-// one list, and two lists sharing an array from its two ends, with room to
-// pad either to a multiple of 4 entries
-constexpr int kWaveCap = kWaveFlush - 1 + 64 + 1;
-constexpr int kWavePool = 2 * (kWaveFlush - 1) + 64 + 6;
-static_assert(kWaveCap % 4 == 0 && kWavePool % 4 == 0, "whole groups of 4 entries");
-
-template <bool REF, int KERNEL, bool CLIP, bool COUNT>
-struct wave_lists {
-  static constexpr bool QUARTIC = KERNEL == 0 && !COUNT;
-  alignas(16) float4 X[QUARTIC ? kWavePool : 1];  // expansion form: far from the front, big from the back
-  float4 S[REF ? kWavePool : kWaveCap];  // position form: small from the front, masked from the back
-  alignas(16) int M[REF ? kWaveCap : 1];  // masked: packed cell (cx | cy << 16)
-  // line-of-sight clip: per entry, the depth range relative to the particle
-  // in units of h, times c^(1/2) (see clip_pow)
-  float2 Xz[CLIP ? kWavePool : 1];
-  float2 Sz[CLIP ? kWaveCap : 1];
-};
 
 template <int T, bool REF, int KERNEL, bool CLIP, bool COUNT>
 struct tile_smem {
@@ -1085,11 +430,7 @@ struct tile_smem {
   float2 pt[T * T];          // the tile's points
   uint2 box[REF ? T * T : 1];  // their search boxes: (x0 | xw << 16, y0 | yw << 16)
   float tab[KERNEL == 2 ? kCubicTable : 1];
-  uint32_t cell_b[NB];
-  uint32_t cell_off[NB];
-  int cell_info[NB];  // cells: packed cell cx | cy << 16 (unsigned); rows: base key
-  int cell_y[NB];     // cells: 1 when in every point's search box; rows: the row's cy
-  uint32_t scan_ws[W];
+  cell_table cells;
   float redf[W][5];
   int redi[W][11];
 };
@@ -1518,219 +859,99 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     nm = 0;
   };
 
-  // ---- candidates.  The particles of the cells cx0..cx1 of one row (y, z)
-  // are contiguous in the sorted order, so the box's particles form nrows *
-  // nlays ranges.  Dense grids visit the box's cells NB at a time (x
-  // fastest) and skip the cells whose max h cannot reach the tile; sparse
-  // grids (well under one particle per cell, e.g. the depth-cut lists of a
-  // slab) stream the row ranges and cull per particle.  Both give the same
-  // candidates in the same order (rows, cells by x, particles in sorted
-  // order).  A sparse grid can still be dense where the tile is (a halo
-  // inside a slab): when the first chunk of rows holds more than
-  // kDenseRows particles per cell of the box, the tile switches to the cell
-  // enumeration, whose max-h skip and prefix search read far fewer.
-  const int ncols = cx1 >= cx0 ? cx1 - cx0 + 1 : 0;
-  const int nrows = cy1 >= cy0 ? cy1 - cy0 + 1 : 0;
-  const int nlays = cz1 >= cz0 ? cz1 - cz0 + 1 : 0;
-  // the box lies inside the grid, whose cells have 32-bit keys: 32-bit
-  // counts and indices (one layer, as in reference mode, skips a division)
-  const uint32_t ncand = uint32_t(ncols) * uint32_t(nrows) * uint32_t(nlays);
-  const uint32_t nrowz = ncols > 0 ? uint32_t(nrows) * uint32_t(nlays) : 0u;
-  const uint32_t nxny = uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
-  const float sup_h2 = support * support * 1.00002f;
-  bool rows_mode = g.sparse != 0 && ncand > uint32_t(NB);
-  const bool one_layer = nlays == 1;
-  uint64_t nitems = rows_mode ? nrowz : ncand;
-  for (uint64_t c0 = 0; c0 < nitems; c0 += NB) {
-    const bool in_box = c0 + uint64_t(t) < nitems;
-    const uint32_t ci = uint32_t(c0) + uint32_t(t);
-    uint32_t cb = 0, cn = 0;
-    int ccx = 0, ccy = 0, cfull = 0;
-    if (rows_mode) {
-      if (in_box) {
-        const uint32_t lay = one_layer ? 0u : ci / uint32_t(nrows);
-        ccy = cy0 + int(ci - lay * uint32_t(nrows));
-        const uint32_t kb = uint32_t(ccy) * uint32_t(g.nc[0]) + uint32_t(cz0 + int(lay)) * nxny;
-        cb = g.start[kb + uint32_t(cx0)];
-        cn = g.start[kb + uint32_t(cx1) + 1] - cb;
-        ccx = int(kb);  // stored as the row's base key
-      }
-    } else if (in_box) {
-      const uint32_t rest = ci / uint32_t(ncols);
-      const int col_c = int(ci - rest * uint32_t(ncols));
-      const uint32_t lay = one_layer ? 0u : rest / uint32_t(nrows);
-      ccx = cx0 + col_c;
-      ccy = cy0 + int(rest - lay * uint32_t(nrows));
-      const int ccz = cz0 + int(lay);
-      const uint32_t key = uint32_t(ccx) + uint32_t(ccy) * uint32_t(g.nc[0]) + uint32_t(ccz) * nxny;
-      cb = g.start[key];
-      const uint32_t ce = g.start[key + 1];
-      if (ce > cb) {
-        const float mh = __uint_as_float(g.maxh_bits[key]);
-        const float lo_x = g.minc[0] + float(ccx) * g.cs[0];
-        const float lo_y = g.minc[1] + float(ccy) * g.cs[1];
-        // a particle's cell comes from fl((x - min) / w): its coordinate can
-        // sit a few ulps of |x| + |min| outside the cell's float edges
-        const float mgx = 1e-4f * g.cs[0] + 4e-7f * (fabsf(g.minc[0]) + fabsf(lo_x) + g.cs[0]);
-        const float mgy = 1e-4f * g.cs[1] + 4e-7f * (fabsf(g.minc[1]) + fabsf(lo_y) + g.cs[1]);
-        const float dx = fmaxf(fmaxf((lo_x - mgx) - tbx1, tbx0 - (lo_x + g.cs[0] + mgx)), 0.0f);
-        const float dy = fmaxf(fmaxf((lo_y - mgy) - tby1, tby0 - (lo_y + g.cs[1] + mgy)), 0.0f);
-        const float d2c = dx * dx + dy * dy;
-        if (d2c < mh * mh * sup_h2) {
-          // the cell's particles come by descending h (to the top 16 bits of
-          // its pattern): only a prefix can reach the tile.  With h rounded
-          // up to its 16-bit bucket the test is monotone along the cell.
-          uint32_t lo = 0, hi = ce - cb;
-          while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            const float hu = __uint_as_float(__float_as_uint(g.hs[cb + mid]) | 0xffffu);
-            if (d2c < hu * hu * sup_h2)
-              lo = mid + 1;
-            else
-              hi = mid;
+  stream_candidates<REF>(
+      g, cx0, cx1, cy0, cy1, cz0, cz1, tbx0, tby0, tbx1, tby1, support,
+      [&](int cx, int cy) {
+        return allz_u && cy >= r_ily && cy <= r_ihy && cx >= r_ilx && cx <= r_ihx;
+      },
+      sm.cells, [&](bool have, uint32_t sidx, int cinf, bool cf, bool done) {
+        float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+        bool keep = false, full = false, big = false, far = false;
+        float2 tcl = make_float2(0.0f, 0.0f);
+        if (have) {
+          // (x, y, coef, 1/h^2); the quartic's z is c = coef^0.4
+          const float4 q = g.part[sidx];
+          if (q.z != 0.0f) {
+            const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
+            const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
+            const float d2 = fmaf(dy, dy, dx * dx);
+            keep = d2 * q.w < cull2;
           }
-          cn = lo;
-        }
-        if constexpr (REF)
-          cfull = (allz_u && ccy >= r_ily && ccy <= r_ihy && ccx >= r_ilx && ccx <= r_ihx) ? 1 : 0;
-      }
-    }
-    uint32_t tot;
-    const uint32_t coff = block_scan_excl<NB>(cn, &tot, sm.scan_ws);
-    tot = uint32_t(uniform(int(tot)));
-    if (rows_mode && c0 == 0 && uint64_t(tot) > uint64_t(kDenseRows) * ncand) {
-      // nothing of this chunk is in LDS yet: start over with the cells
-      rows_mode = false;
-      nitems = ncand;
-      c0 = uint64_t(0) - uint64_t(NB);
-      continue;
-    }
-    sm.cell_b[t] = cb;
-    sm.cell_off[t] = coff;
-    if (rows_mode) {
-      sm.cell_info[t] = ccx;
-      sm.cell_y[t] = ccy;
-    } else {
-      sm.cell_info[t] = int(uint32_t(ccx) | (uint32_t(ccy) << 16));
-      sm.cell_y[t] = cfull;
-    }
-    __syncthreads();
-    // the chunk's particles, 64 at a time, dealt to the waves in turn; after
-    // the last of them the wave's lists are evaluated whatever their size
-    // (here and not behind the loop: one copy of the evaluation code)
-    const bool last_chunk = c0 + NB >= nitems;
-    for (uint32_t v0 = uint32_t(wave) * 64u;; v0 += NB) {
-      const bool done = v0 >= tot;
-      if (done && !last_chunk) break;
-      const uint32_t v = v0 + uint32_t(lane);
-      float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
-      bool keep = false, full = false, big = false, far = false;
-      int cinf = 0, cf = 0;
-      float2 tcl = make_float2(0.0f, 0.0f);
-      if (v < tot) {
-        // last cell whose offset is <= v (it has a nonzero count)
-        int lo = 0;
-#pragma unroll
-        for (int step = NB / 2; step > 0; step >>= 1)
-          if (sm.cell_off[lo + step] <= v) lo += step;
-        const uint32_t sidx = sm.cell_b[lo] + (v - sm.cell_off[lo]);
-        if constexpr (REF) {
-          cinf = sm.cell_info[lo];
-          cf = sm.cell_y[lo];
-          if (rows_mode) {
-            // the particle's cell from its key and the row's base key
-            const int px_c = int(g.key[sidx] - uint32_t(cinf));
-            const int py_c = cf;
-            cinf = int(uint32_t(px_c) | (uint32_t(py_c) << 16));
-            cf = (allz_u && py_c >= r_ily && py_c <= r_ihy && px_c >= r_ilx && px_c <= r_ihx) ? 1 : 0;
+          if constexpr (CLIP) {
+            // the depth range relative to the particle, in units of h: its
+            // support must overlap it
+            const float2 zc = g.clip[sidx];
+            keep = keep && zc.x < 1.0f && zc.y > -1.0f;
+            const float rc = __builtin_amdgcn_sqrtf(q.z);
+            tcl = make_float2(zc.x * rc, zc.y * rc);
           }
-        }
-        // (x, y, coef, 1/h^2); the quartic's z is c = coef^0.4
-        const float4 q = g.part[sidx];
-        if (q.z != 0.0f) {
-          const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
-          const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
-          const float d2 = fmaf(dy, dy, dx * dx);
-          keep = d2 * q.w < cull2;
-        }
-        if constexpr (CLIP) {
-          // the depth range relative to the particle, in units of h: its
-          // support must overlap it
-          const float2 zc = g.clip[sidx];
-          keep = keep && zc.x < 1.0f && zc.y > -1.0f;
-          const float rc = __builtin_amdgcn_sqrtf(q.z);
-          tcl = make_float2(zc.x * rc, zc.y * rc);
-        }
-        full = keep && (!REF || cf || q.w >= unmask_ih2);
-        if (keep) {
-          if constexpr (COUNT) {
-            e = make_float4(q.x, q.y, g.hs[sidx], 0.0f);
-          } else if constexpr (KERNEL == 2) {
-            e = q;
-          } else {
-            const float c = q.z;        // coef^0.4
-            const float ci2 = c * q.w;  // c / h^2
-            big = full && big_r2 * q.w <= 1.0f;
-            if (big) {
-              const float xr = q.x - tcx, yr = q.y - tcy;
-              const float d2r = fmaf(yr, yr, xr * xr);
-              e = make_float4(c * fmaf(-q.w, d2r, 1.0f), 2.0f * ci2 * xr, 2.0f * ci2 * yr, -ci2);
-              if constexpr (FAR) far = is_far(d2r, q.w, hd2);
+          full = keep && (!REF || cf || q.w >= unmask_ih2);
+          if (keep) {
+            if constexpr (COUNT) {
+              e = make_float4(q.x, q.y, g.hs[sidx], 0.0f);
+            } else if constexpr (KERNEL == 2) {
+              e = q;
             } else {
-              e = make_float4(q.x, q.y, ci2, c);
+              const float c = q.z;        // coef^0.4
+              const float ci2 = c * q.w;  // c / h^2
+              big = full && big_r2 * q.w <= 1.0f;
+              if (big) {
+                const float xr = q.x - tcx, yr = q.y - tcy;
+                const float d2r = fmaf(yr, yr, xr * xr);
+                e = make_float4(c * fmaf(-q.w, d2r, 1.0f), 2.0f * ci2 * xr, 2.0f * ci2 * yr, -ci2);
+                if constexpr (FAR) far = is_far(d2r, q.w, hd2);
+              } else {
+                e = make_float4(q.x, q.y, ci2, c);
+              }
             }
           }
         }
-      }
-      const uint64_t bf = FAR ? __ballot(far) : 0ull;
-      const uint64_t bb = __ballot(big && !far);
-      const uint64_t bs = __ballot(full && !big);
-      const uint64_t bm = __ballot(keep && !full);
-      if constexpr (FAR)
-        if (far) L.X[nf + int(prefix_count(bf))] = e;
-      if constexpr (QUARTIC) {
-        if (big && !far) {
-          const int pos = kWavePool - 1 - (nb + int(prefix_count(bb)));
-          L.X[pos] = e;
-          if constexpr (CLIP) L.Xz[pos] = tcl;
+        const uint64_t bf = FAR ? __ballot(far) : 0ull;
+        const uint64_t bb = __ballot(big && !far);
+        const uint64_t bs = __ballot(full && !big);
+        const uint64_t bm = __ballot(keep && !full);
+        if constexpr (FAR)
+          if (far) L.X[nf + int(prefix_count(bf))] = e;
+        if constexpr (QUARTIC) {
+          if (big && !far) {
+            const int pos = kWavePool - 1 - (nb + int(prefix_count(bb)));
+            L.X[pos] = e;
+            if constexpr (CLIP) L.Xz[pos] = tcl;
+          }
         }
-      }
-      if (full && !big) {
-        const int pos = ns + int(prefix_count(bs));
-        L.S[pos] = e;
-        if constexpr (CLIP) L.Sz[pos] = tcl;
-      }
-      if constexpr (REF) {
-        if (keep && !full) {
-          const int pos = nm + int(prefix_count(bm));
-          L.S[kWavePool - 1 - pos] = e;
-          L.M[pos] = cinf;
+        if (full && !big) {
+          const int pos = ns + int(prefix_count(bs));
+          L.S[pos] = e;
+          if constexpr (CLIP) L.Sz[pos] = tcl;
         }
-      }
-      if constexpr (FAR) nf += __popcll(bf);
-      nb += __popcll(bb);
-      ns += __popcll(bs);
-      nm += __popcll(bm);
-      const int lim = done ? 1 : kWaveFlush;
-      if constexpr (FAR) {
-        if (done && !far_used && nf > 0) {
-          // too few far entries to pay for the tile's interpolation
-          const int n = uniform(nf);
-          const float4 x = lane < n ? L.X[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-          wave_sync();
-          if (lane < n) L.X[kWavePool - 1 - (nb + lane)] = x;
-          nb += n;
-          nf = 0;
+        if constexpr (REF) {
+          if (keep && !full) {
+            const int pos = nm + int(prefix_count(bm));
+            L.S[kWavePool - 1 - pos] = e;
+            L.M[pos] = cinf;
+          }
         }
-        if (nf >= lim) eval_far();
-      }
-      if (nb >= lim) eval_big();
-      if (ns >= lim) eval_small();
-      if (nm >= lim) eval_masked();
-      if (done) break;
-    }
-    __syncthreads();  // the cell table is rewritten by the next chunk
-  }
+        if constexpr (FAR) nf += __popcll(bf);
+        nb += __popcll(bb);
+        ns += __popcll(bs);
+        nm += __popcll(bm);
+        const int lim = done ? 1 : kWaveFlush;
+        if constexpr (FAR) {
+          if (done && !far_used && nf > 0) {
+            // too few far entries to pay for the tile's interpolation
+            const int n = uniform(nf);
+            const float4 x = lane < n ? L.X[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+            wave_sync();
+            if (lane < n) L.X[kWavePool - 1 - (nb + lane)] = x;
+            nb += n;
+            nf = 0;
+          }
+          if (nf >= lim) eval_far();
+        }
+        if (nb >= lim) eval_big();
+        if (ns >= lim) eval_small();
+        if (nm >= lim) eval_masked();
+      });
   if constexpr (FAR)
     if (far_used && lane == 0) sm.far_used = 1;
 
@@ -1854,23 +1075,273 @@ __global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSum
   }
 }
 
-// Adjoint of the exact-mode gather over one point image (quartic or the
-// tabulated cubic spline).
-template <int TW, int PPT, int KERNEL>
-__global__ __launch_bounds__(kBlock) void k_adjoint(grid_view g, point_view p, uint32_t tiles_x,
-                                                    uint32_t ntiles, adjoint_io io) {
-  __shared__ gather_smem<false, KERNEL, true> sm;
+// ---- the adjoint of the exact-mode gather
+//
+// A workgroup owns a tile of T x T points with their gradients; its waves
+// stream the candidates as the gather does.  A wave lists the kept particles'
+// indices, and with 64 of them gives each lane one: the lane visits the 8x8
+// point blocks that some listed particle's support reaches and sums over
+// their points moments of g = dL/dvalue * s^1.5 (s = 1 - r^2/h^2); the
+// weights are recomputed, not stored.  One atomic add per gradient component,
+// particle and tile:
+//   dL/dw = K/h^2        sum g s
+//   dL/dh = w K/h^3      sum g (7 r^2/h^2 - 2)
+//   dL/dx = -5 w K/h^4   sum g (x - x_point)     (same for y)
+// In 16x16 tiles the far particles (is_far) take the transpose of the
+// gather's interpolation: the tile's gradients are first summed onto the 64
+// nodes, and the particle visits the nodes instead of the 256 points.
+// VALU-bound (16 operations a pair).  Against shared lists of 32x32 tiles,
+// one particle per thread: 4M particles on 1024^2 points 10.8 -> 4.1 ms, 20k on
+// 96^2 (9 workgroups before, 144 now) 1.34 -> 0.06 ms; every component's error
+// against 64 bits is at or below what it was.
+constexpr int kAdjCap = 2 * 63 + 64;  // two index lists from the two ends of one array
+
+template <int T, int KERNEL>
+struct adjoint_smem {
+  static constexpr int NP = T * T;
+  float4 pt[NP];  // tile points (x, y, dL/dvalue, -), 8x8 block after 8x8 block
+  float4 box[NP / 64];  // the blocks' boxes of points with a gradient (x0, y0, x1, y1)
+  alignas(16) float node[KERNEL == 0 && NP > 64 ? 64 : 1];  // the gradients at the nodes
+  union {
+    uint32_t idx[kSumW][kAdjCap];
+    struct {  // while the nodes are summed: the points' Lagrange bases
+      float bx[KERNEL == 0 && NP > 64 ? NP : 1][kNodes];
+      float by[KERNEL == 0 && NP > 64 ? NP : 1][kNodes];
+      double part[KERNEL == 0 && NP > 64 ? kSumW : 1][64];
+    };
+  };
+  cell_table cells;
+  float tab[KERNEL == 2 ? kCubicTable : 1];
+  float dtab[KERNEL == 2 ? kCubicTable : 1];
+};
+
+template <int T, int KERNEL>
+__global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view p,
+                                                        uint32_t tiles_x, uint32_t ntiles,
+                                                        adjoint_io io) {
+  constexpr int NB = 64 * kSumW, NP = T * T, NBLK = NP / 64;
+  constexpr bool FAR = KERNEL == 0 && NP > 64;
+  static_assert(NP <= NB, "one point per thread");
+  __shared__ adjoint_smem<T, KERNEL> sm;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t bid = blockIdx.x;
+  const uint32_t per = ntiles / 8u;
+  const uint32_t tile = bid < per * 8u ? (bid % 8u) * per + bid / 8u : bid;
+  const uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
   if constexpr (KERNEL == 2) {
-    for (int i = threadIdx.x; i < kCubicTable; i += kBlock) {
+    for (int i = t; i < kCubicTable; i += NB) {
       sm.tab[i] = io.ftab[i];
       sm.dtab[i] = io.dtab[i];
     }
   }
-  const uint32_t bid = blockIdx.x;
-  const uint32_t per = ntiles / 8u;
-  const uint32_t tile = bid < per * 8u ? (bid % 8u) * per + bid / 8u : bid;
-  gather_tile<TW, PPT, OP_ADJOINT, KERNEL>(g, p, tile % tiles_x, tile / tiles_x, nullptr, nullptr,
-                                           KERNEL == 2 ? 2.0f : 1.0f, sm, &io);
+  const float support = KERNEL == 2 ? 2.0f : 1.0f;
+
+  // ---- thread t: point t of the blocks' order; the blocks' boxes of the
+  // points with a gradient, and the tile box over them
+  float px = 0.f, py = 0.f, pg = 0.f;
+  if (t < NP) {
+    const int blk = t >> 6, in = t & 63;
+    const uint32_t ix = tx * T + uint32_t((blk % (T / 8)) * 8 + (in & 7));
+    const uint32_t iy = ty * T + uint32_t((blk / (T / 8)) * 8 + (in >> 3));
+    const uint32_t pid = iy * p.lnx + ix;
+    if (ix < p.lnx && iy < p.lny && pid < p.n) {
+      const float4 q = p.gen ? pixel_point(p.pg, ix, iy) : p.pts[pid];
+      px = q.x;
+      py = q.y;
+      pg = io.grad[pid] * io.scale;
+    }
+    sm.pt[t] = make_float4(px, py, pg, 0.0f);
+  }
+  {
+    const bool on = pg != 0.0f;
+    const float x0 = wmin(on ? px : INFINITY), y0 = wmin(on ? py : INFINITY);
+    const float x1 = wmax(on ? px : -INFINITY), y1 = wmax(on ? py : -INFINITY);
+    if (lane == 0 && wave < NBLK) sm.box[wave] = make_float4(x0, y0, x1, y1);
+  }
+  __syncthreads();
+  float tbx0 = INFINITY, tby0 = INFINITY, tbx1 = -INFINITY, tby1 = -INFINITY;
+  for (int b = 0; b < NBLK; ++b) {
+    const float4 x = sm.box[b];
+    tbx0 = fminf(tbx0, x.x);
+    tby0 = fminf(tby0, x.y);
+    tbx1 = fmaxf(tbx1, x.z);
+    tby1 = fmaxf(tby1, x.w);
+  }
+  tbx0 = uniformf(tbx0);
+  tby0 = uniformf(tby0);
+  tbx1 = uniformf(tbx1);
+  tby1 = uniformf(tby1);
+  if (!(tbx0 <= tbx1)) return;  // no gradient in the tile
+  const float tcx = 0.5f * (tbx0 + tbx1), tcy = 0.5f * (tby0 + tby1);
+  const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
+  const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
+
+  // ---- the gradients at the nodes (when any particle is wide enough)
+  const bool nodes = FAR && g.max_h * g.max_h * 0.16f >= hd2;
+  if constexpr (FAR) {
+    if (nodes) {
+      double b[kNodes];
+      node_basis(pg != 0.0f && hd_x > 0.0f ? double(px - tcx) / double(hd_x) : 0.0, b);
+#pragma unroll
+      for (int i = 0; i < kNodes; ++i) sm.bx[t][i] = float(b[i] * double(pg));
+      node_basis(pg != 0.0f && hd_y > 0.0f ? double(py - tcy) / double(hd_y) : 0.0, b);
+#pragma unroll
+      for (int i = 0; i < kNodes; ++i) sm.by[t][i] = float(b[i]);
+      __syncthreads();
+      double sum = 0.0;
+      for (int k = 64 * wave; k < 64 * wave + 64; ++k)
+        sum += double(sm.bx[k][lane & 7]) * double(sm.by[k][lane >> 3]);
+      sm.part[wave][lane] = sum;
+      __syncthreads();
+      if (t < 64) {
+        double n = 0.0;
+        for (int w = 0; w < kSumW; ++w) n += sm.part[w][t];
+        sm.node[t] = float(n);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- candidate cell box (one extra cell on each side absorbs rounding)
+  const float reach = support * g.max_h;
+  const int cx0 = uniform(max(max(cell_of(tbx0, -reach, g.minc[0], g.cs[0]), INT32_MIN + 1) - 1, 0));
+  const int cx1 = uniform(
+      min(min(cell_of(tbx1, reach, g.minc[0], g.cs[0]), INT32_MAX - 1) + 1, g.nc[0] - 1));
+  const int cy0 = uniform(max(max(cell_of(tby0, -reach, g.minc[1], g.cs[1]), INT32_MIN + 1) - 1, 0));
+  const int cy1 = uniform(
+      min(min(cell_of(tby1, reach, g.minc[1], g.cs[1]), INT32_MAX - 1) + 1, g.nc[1] - 1));
+  const float cull2 = support * support;
+
+  uint32_t* const idx = sm.idx[wave];
+  int nf = 0, nn = 0;  // far from the front, near from the back
+
+  // the moments of the particle's lane into the gradients
+  auto add = [&](uint32_t si, const float4& q, float coef, float a0, float a1, float a2,
+                 float a3, float a4) {
+    if constexpr (KERNEL == 2) {
+      // value = w K F(u) / h^2: d/dh = -2 w K / h^3 (F + u F'),
+      // d/dx = 2 w K / h^4 F' (x - x_point)
+      const float c2 = 2.0f * coef * q.w;
+      atomicAdd(io.gw + si, io.norm * q.w * a0);
+      atomicAdd(io.gh + si, -2.0f * coef * __builtin_amdgcn_sqrtf(q.w) * (a0 + a1));
+      atomicAdd(io.gx + si, c2 * a3);
+      atomicAdd(io.gy + si, c2 * a4);
+    } else {
+      const float c5 = -5.0f * coef * q.w;  // -5 w K / h^4
+      atomicAdd(io.gw + si, io.norm * q.w * a0);
+      atomicAdd(io.gh + si, coef * __builtin_amdgcn_sqrtf(q.w) * fmaf(7.0f * q.w, a2, -2.0f * a1));
+      atomicAdd(io.gx + si, c5 * a3);
+      atomicAdd(io.gy + si, c5 * a4);
+    }
+  };
+  auto near_batch = [&]() {
+    const int n = min(uniform(nn), 64);
+    const bool act = lane < n;
+    const uint32_t si = act ? idx[kAdjCap - nn + lane] : 0u;  // the list's last 64
+    float4 q = make_float4(0.f, 0.f, 1.f, 0.f);
+    if (act) q = g.part[si];
+    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, a4 = 0.f;
+    for (int blk = 0; blk < NBLK; ++blk) {
+      const float4 bx = sm.box[blk];
+      const float bdx = fmaxf(fmaxf(bx.x - q.x, q.x - bx.z), 0.0f);
+      const float bdy = fmaxf(fmaxf(bx.y - q.y, q.y - bx.w), 0.0f);
+      if (!__ballot(act && bx.x <= bx.z && fmaf(bdy, bdy, bdx * bdx) * q.w < cull2)) continue;
+#pragma unroll 8
+      for (int k = 0; k < 64; ++k) {
+        const float4 pt = sm.pt[64 * blk + k];
+        const float dx = q.x - pt.x, dy = q.y - pt.y;
+        const float r2 = fmaf(dy, dy, dx * dx);
+        if constexpr (KERNEL == 2) {
+          // F and dF/du at u = r^2/h^2, linear in the tables (0 beyond u = 4)
+          const float uu = r2 * q.w;
+          const float xx = fminf(uu * (float(kCubicTable - 1) / 4.0f), float(kCubicTable - 1));
+          const int ti = min(int(xx), kCubicTable - 2);
+          const float tf = xx - float(ti);
+          const float F = fmaf(tf, sm.tab[ti + 1] - sm.tab[ti], sm.tab[ti]);
+          const float D = fmaf(tf, sm.dtab[ti + 1] - sm.dtab[ti], sm.dtab[ti]);
+          const float gd = pt.z * D;
+          a0 = fmaf(pt.z, F, a0);
+          a1 = fmaf(gd, uu, a1);
+          a3 = fmaf(gd, dx, a3);
+          a4 = fmaf(gd, dy, a4);
+        } else {
+          const float sv = fmaxf(fmaf(-r2, q.w, 1.0f), 0.0f);
+          const float gq = pt.z * (sv * __builtin_amdgcn_sqrtf(sv));
+          a0 = fmaf(gq, sv, a0);
+          a1 += gq;
+          a2 = fmaf(gq, r2, a2);
+          a3 = fmaf(gq, dx, a3);
+          a4 = fmaf(gq, dy, a4);
+        }
+      }
+    }
+    if (act) add(si, q, KERNEL == 2 ? q.z : pow25_pos(q.z), a0, a1, a2, a3, a4);
+    nn -= n;
+  };
+  auto far_batch = [&]() {
+    if constexpr (FAR) {
+      const int n = min(uniform(nf), 64);
+      const bool act = lane < n;
+      const uint32_t si = act ? idx[nf - n + lane] : 0u;
+      float4 q = make_float4(0.f, 0.f, 1.f, 0.f);
+      if (act) q = g.part[si];
+      const float xr = q.x - tcx, yr = q.y - tcy;
+      float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, a4 = 0.f;
+#pragma unroll 1
+      for (int iy = 0; iy < kNodes; ++iy) {
+        float ny = 0.f;
+#pragma unroll
+        for (int i = 0; i < kNodes; ++i)
+          if (iy == i) ny = float(kNodeX[i]);
+        const float dy = fmaf(-hd_y, ny, yr);
+        const float dy2 = dy * dy;
+#pragma unroll
+        for (int ix = 0; ix < kNodes; ++ix) {
+          const float gn = sm.node[8 * iy + ix];
+          const float dx = fmaf(-hd_x, float(kNodeX[ix]), xr);
+          const float r2 = fmaf(dx, dx, dy2);
+          const float sv = fmaxf(fmaf(-r2, q.w, 1.0f), 0.0f);
+          const float gq = gn * (sv * __builtin_amdgcn_sqrtf(sv));
+          a0 = fmaf(gq, sv, a0);
+          a1 += gq;
+          a2 = fmaf(gq, r2, a2);
+          a3 = fmaf(gq, dx, a3);
+          a4 = fmaf(gq, dy, a4);
+        }
+      }
+      if (act) add(si, q, pow25_pos(q.z), a0, a1, a2, a3, a4);
+      nf -= n;
+    }
+  };
+
+  stream_candidates<false>(
+      g, cx0, cx1, cy0, cy1, 0, g.nc[2] - 1, tbx0, tby0, tbx1, tby1, support,
+      [](int, int) { return true; }, sm.cells,
+      [&](bool have, uint32_t sidx, int, bool, bool done) {
+        bool keep = false, far = false;
+        if (have) {
+          const float4 q = g.part[sidx];
+          const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
+          const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
+          keep = fmaf(dy, dy, dx * dx) * q.w < cull2;
+          if constexpr (FAR) {
+            const float xr = q.x - tcx, yr = q.y - tcy;
+            far = keep && nodes && is_far(fmaf(yr, yr, xr * xr), q.w, hd2, 0.16f);
+          }
+        }
+        const uint64_t bf = FAR ? __ballot(far) : 0ull;
+        const uint64_t bn = __ballot(keep && !far);
+        if (far) idx[nf + int(prefix_count(bf))] = sidx;
+        if (keep && !far) idx[kAdjCap - 1 - (nn + int(prefix_count(bn)))] = sidx;
+        nf += __popcll(bf);
+        nn += __popcll(bn);
+        const int lim = done ? 1 : 64;
+        wave_sync();
+        if constexpr (FAR)
+          while (nf >= lim) far_batch();
+        while (nn >= lim) near_batch();
+        wave_sync();
+      });
 }
 
 // gradients in sorted order -> input order
@@ -1948,34 +1419,6 @@ int dispatch(const sum_shape& ts, int op, int kernel, A&&... a) {
 
 }  // namespace
 
-void launch_adjoint(const grid_view& g, const point_view& p, int kernel, const float* grad,
-                    float scale, float norm, const float* ftab, const float* dtab, float* gw,
-                    float* gh, float* gx, float* gy, hipStream_t s) {
-  constexpr int TW = 32, PPT = 4, TH = (kBlock / TW) * PPT;
-  const uint32_t tiles_x = (p.lnx + TW - 1) / TW;
-  const uint32_t ntiles = tiles_x * ((p.lny + TH - 1) / TH);
-  if (!ntiles) return;
-  adjoint_io io{grad, scale, norm, ftab, dtab, gw, gh, gx, gy};
-  if (kernel == ILC_KERNEL_CUBIC) {
-    if (!ftab || !dtab) fail(ILC_EINVAL, "cubic adjoint without its tables");
-    hipLaunchKernelGGL((k_adjoint<TW, PPT, 2>), dim3(ntiles), dim3(kBlock), 0, s, g, p, tiles_x,
-                       ntiles, io);
-  } else {
-    hipLaunchKernelGGL((k_adjoint<TW, PPT, 0>), dim3(ntiles), dim3(kBlock), 0, s, g, p, tiles_x,
-                       ntiles, io);
-  }
-  ILC_HIP(hipGetLastError());
-}
-
-void launch_unpermute4(const uint32_t* perm, uint32_t n, const float* a, const float* b,
-                       const float* c, const float* d, float* oa, float* ob, float* oc, float* od,
-                       hipStream_t s) {
-  if (!n) return;
-  hipLaunchKernelGGL(k_unpermute4, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, perm, n, a,
-                     b, c, d, oa, ob, oc, od);
-  ILC_HIP(hipGetLastError());
-}
-
 // 16x16 tiles list a candidate once per 256 points and sum the far particles
 // at 64 nodes; 8x8 tiles give four times the workgroups and waste fewer pairs
 // at the supports' edges.  Below kPointsFor16 points the launch cannot fill
@@ -2002,6 +1445,38 @@ void tile_grid(const sum_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_
                uint32_t* ntiles) {
   *tiles_x = (lnx + ts.side - 1) / ts.side;
   *ntiles = *tiles_x * ((lny + ts.side - 1) / ts.side);
+}
+
+void launch_adjoint(const grid_view& g, const point_view& p, int kernel, const float* grad,
+                    float scale, float norm, const float* ftab, const float* dtab, float* gw,
+                    float* gh, float* gx, float* gy, hipStream_t s) {
+  uint32_t tiles_x = 0, ntiles = 0;
+  const sum_shape ts{p.n < kPointsFor16 ? 8 : 16};
+  tile_grid(ts, p.lnx, p.lny, &tiles_x, &ntiles);
+  if (!ntiles) return;
+  adjoint_io io{grad, scale, norm, ftab, dtab, gw, gh, gx, gy};
+  const dim3 grid{ntiles}, block{64 * kSumW};
+  if (kernel == ILC_KERNEL_CUBIC) {
+    if (!ftab || !dtab) fail(ILC_EINVAL, "cubic adjoint without its tables");
+    if (ts.side == 8)
+      hipLaunchKernelGGL((k_adjoint<8, 2>), grid, block, 0, s, g, p, tiles_x, ntiles, io);
+    else
+      hipLaunchKernelGGL((k_adjoint<16, 2>), grid, block, 0, s, g, p, tiles_x, ntiles, io);
+  } else if (ts.side == 8) {
+    hipLaunchKernelGGL((k_adjoint<8, 0>), grid, block, 0, s, g, p, tiles_x, ntiles, io);
+  } else {
+    hipLaunchKernelGGL((k_adjoint<16, 0>), grid, block, 0, s, g, p, tiles_x, ntiles, io);
+  }
+  ILC_HIP(hipGetLastError());
+}
+
+void launch_unpermute4(const uint32_t* perm, uint32_t n, const float* a, const float* b,
+                       const float* c, const float* d, float* oa, float* ob, float* oc, float* od,
+                       hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(k_unpermute4, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, perm, n, a,
+                     b, c, d, oa, ob, oc, od);
+  ILC_HIP(hipGetLastError());
 }
 
 int gather_batch_grid(int op, int kernel, const sum_shape& ts) {

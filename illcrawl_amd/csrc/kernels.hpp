@@ -237,7 +237,7 @@ struct point_view {
 };
 
 // OP_CLIP: exact mode with the line-of-sight kernel clip (grid_view::clip)
-enum gather_op { OP_REFERENCE = 0, OP_EXACT = 1, OP_COUNT = 2, OP_ADJOINT = 3, OP_CLIP = 4 };
+enum gather_op { OP_REFERENCE = 0, OP_EXACT = 1, OP_COUNT = 2, OP_CLIP = 3 };
 
 // The caller's tile, as the ABI states it (see sum_shape).
 struct tile_shape {

@@ -139,3 +139,30 @@ def test_coincident_points(B, orc, kernel):
     assert np.all(got == got[0])
     # the cubic kernel is tabulated: the parity tests' 2e-5
     assert abs(got[0] - ref[0]) / ref[0] < (2e-5 if kernel == "cubic" else LINF_TOL)
+
+
+@pytest.mark.parametrize("nx,ny", [(1024, 771), (97, 43), (8, 1)])
+def test_adjoint_tiles(B, orc, nx, ny):
+    """Both tile sides of the adjoint (16x16 from 3 << 18 points), partial
+    tiles, blocks without a gradient, and supports from a fraction of a pixel
+    to most of the image (the nodes of 16x16 tiles).  1e-4 of each component's
+    largest magnitude, as the adjoint tests."""
+    rng = np.random.default_rng(nx)
+    n = 300
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, 0], p4[:, 1] = rng.uniform(-0.6 * nx, 0.6 * nx, n), rng.uniform(-0.6 * ny, 0.6 * ny, n)
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    h = np.exp(rng.uniform(np.log(0.4), np.log(0.4 * max(nx, ny) + 2.0), n)).astype(np.float32)
+    pts = lattice(nx, ny, -0.5 * nx, -0.5 * ny, 1.0)
+    G = rng.normal(size=nx * ny).astype(np.float32)
+    G.reshape(ny, nx)[: ny // 3, : nx // 3] = 0.0
+    b = B.ProjectiveSmoothingGrid(mode="exact", kernel="quartic", target_particles_per_cell=40)
+    b.init_backend(n)
+    b.setup_projected_particles(p4, h)
+    b.setup_evaluation_points(pts, layout_nx=nx)
+    got = [t.cpu().numpy() for t in b.backward(torch.from_numpy(G).cuda(), 1.0)]
+    ref = orc.backward_exact(p4, h, pts, G, kind=1)
+    for name, a, r in zip(("w", "h", "x", "y"), got, ref):
+        e = float(np.max(np.abs(a - r)) / np.max(np.abs(r)))
+        print(f"adjoint {nx}x{ny} dL/d{name}: {e:.2e}", flush=True)
+        assert e < 1e-4

@@ -49,7 +49,7 @@ struct build_lane {
   grid_scratch scratch;
   dbuf<float4> p4tmp;
   dbuf<float> htmp;
-  dbuf<uint32_t> wcounts, woffs;
+  dbuf<uint32_t> wcounts, woffs, scan_temp;
   ~build_lane() {
     if (done) (void)hipEventDestroy(done);
     if (st) (void)hipStreamDestroy(st);
@@ -133,7 +133,7 @@ struct ilc_batch {
   hipEvent_t ev_fork = nullptr;
   std::vector<std::unique_ptr<grid_store>> group_grids;  // per-cell max h per slab group
   std::vector<size_t> group_leader;
-  dbuf<uint32_t> wcounts, woffs, wtotal;
+  dbuf<uint32_t> wcounts, woffs, scan_temp, wtotal;
   pinned<uint32_t> wtotal_host;
   dbuf<float> bbox_parts;
   dbuf<bbox_result> bbox_dev;
@@ -158,7 +158,7 @@ struct ilc_batch {
   // the range relative to the particle in units of h
   int clip = 0;
   dbuf<float2> sh_zc, sh_zcs;
-  dbuf<uint32_t> sh_offs, sh_gkey, sh_orig, sh_key, sh_perm, sh_sk, sh_counts, sh_start, sh_maxh,
+  dbuf<uint32_t> sh_offs, sh_gkey, sh_orig, sh_key, sh_perm, sh_counts, sh_start, sh_maxh,
       sh_temp, sh_cbase;
   pinned<uint32_t> sh_cbase_host;
   dbuf<float> sh_wx, sh_hs;
@@ -548,7 +548,7 @@ void plan(ilc_batch* b, hipStream_t s) {
   b->items_ord.ensure(nitems);
   b->item_keys.ensure(nitems);
   b->item_idx.ensure(nitems);
-  b->item_temp.ensure(radix_temp_words(nitems));
+  b->item_temp.ensure(radix_chain_words(nitems));
   b->desc_dev.ensure(nv);
   b->desc_host.ensure(nv);
   b->counter.ensure(2);
@@ -579,6 +579,7 @@ struct build_ctx {
   dbuf<float>* htmp;
   dbuf<uint32_t>* wcounts;
   dbuf<uint32_t>* woffs;
+  dbuf<uint32_t>* scan_temp;
   hipStream_t st;
 };
 
@@ -610,23 +611,22 @@ void build_view(ilc_batch* b, view_state& vs, const build_ctx& c, bool clear) {
     const uint64_t m = vs.nwin_plain;
     c.woffs->ensure(size_t(nt) + 1);
     c.htmp->ensure(std::max<uint64_t>(m, 1));
-    vs.grid.key.ensure(std::max<uint64_t>(m, 1));
-    vs.grid.perm.ensure(std::max<uint64_t>(m, 1));
-    c.sc->temp.ensure(scan_temp_words(uint64_t(nt) + 1));
+    const radix_chain rc = plan_grid_sort(vs.grid, *c.sc, m, vs.gp);
+    c.scan_temp->ensure(scan_temp_words(uint64_t(nt) + 1));
     // the plan counted the kept particles of every window tile of this view
     launch_exclusive_scan(b->wcounts_all.p + (b->views.size() + view_index(b, vs)) * size_t(nt),
-                          c.woffs->p, nt, c.sc->temp.p, st);
+                          c.woffs->p, nt, c.scan_temp->p, st);
     vs.orig.ensure(std::max<uint64_t>(m, 1));
     launch_window_scatter(b->ps, proj_of(b, vs), gaunt_of(b), vs.win, c.woffs->p, vs.gp,
-                          c.p4tmp->p, c.htmp->p, vs.grid.key.p, vs.grid.perm.p, vs.orig.p,
+                          c.p4tmp->p, c.htmp->p, rc.b[rc.in], rc.a[rc.in], vs.orig.p,
                           b->counter.p + 1, st);
-    enqueue_grid_from_keys(vs.grid, *c.sc, c.p4tmp->p, c.htmp->p, m, vs.gp, vs.kz0, vs.max_h,
+    enqueue_grid_from_keys(vs.grid, *c.sc, rc, c.p4tmp->p, c.htmp->p, m, vs.gp, vs.kz0, vs.max_h,
                            b->kernel, st);
     vs.grid.density_n = vs.windowed ? b->ps.n : 0;
   } else {
     launch_view_project(b->ps, proj_of(b, vs), gaunt_of(b), c.p4tmp->p, st);
     enqueue_grid_build(vs.grid, *c.sc, c.p4tmp->p, b->ps.hsml, b->ps.n, vs.gp, vs.kz0, vs.max_h,
-                       b->kernel, b->counter.p + 1, st);
+                       b->kernel, b->counter.p + 1, false, st);
     vs.grid.density_n = 0;
   }
   own_grid(b, vs);
@@ -640,9 +640,9 @@ void build_shared(ilc_batch* b, hipStream_t s) {
   const uint64_t ntot = b->sh_ntot, nc = b->sh_ncells;
   const uint32_t n32 = static_cast<uint32_t>(ntot);
   b->sh_offs.ensure(nv * size_t(nt) + 1);
-  b->sh_temp.ensure(std::max({radix2_temp_words(ntot), scan_temp_words(nv * uint64_t(nt) + 1),
+  b->sh_temp.ensure(std::max({radix_chain_words(ntot), scan_temp_words(nv * uint64_t(nt) + 1),
                               scan_temp_words(nc + 1)}));
-  for (auto* d : {&b->sh_gkey, &b->sh_orig, &b->sh_key, &b->sh_perm, &b->sh_sk})
+  for (auto* d : {&b->sh_gkey, &b->sh_orig, &b->sh_key, &b->sh_perm})
     d->ensure(ntot);
   b->sh_hs.ensure(ntot);
   b->sh_p4c.ensure(ntot);
@@ -668,26 +668,24 @@ void build_shared(ilc_batch* b, hipStream_t s) {
   bool all_compact = true;
   for (auto& v : b->views) all_compact = all_compact && v->compact;
   uint32_t* const maxh = all_compact ? nullptr : b->sh_maxh.p;
-  if (maxh) launch_fill_u32(maxh, 0u, nc, s);
+  // the rows' sort: by global cell key (view, then cell), biggest h first,
+  // ties in input order
+  const radix_chain rc = plan_radix_chain(b->sh_gkey.p, b->sh_perm.p, ntot, kHKeyBits,
+                                          key_bits_for(b->sh_ncells - 1), b->sh_temp.p);
+  launch_zero({radix_chain_zero(rc), {maxh, maxh ? nc : 0}, {b->sh_counts.p, nc + 1}}, s);
   if (b->clip) {
     b->sh_zc.ensure(ntot);
     b->sh_zcs.ensure(ntot);
   }
   launch_multi_window_scatter(b->ps, any_xray ? b->sh_wx.p : nullptr, b->bdesc_dev.p,
                               b->fviews_dev.p, static_cast<int>(nv), b->sh_offs.p, b->sh_p4c.p,
-                              b->sh_sk.p, b->sh_perm.p, b->sh_gkey.p, b->sh_orig.p,
+                              rc.a[rc.in], rc.b[rc.in], b->sh_orig.p,
                               b->counter.p + 1, b->sh_cbase.p, maxh,
                               b->clip ? b->sh_zc.p : nullptr, b->stack, s);
-  // stable sorts by descending h (each row's global cell key moving with
-  // it), then by global cell key (view, then cell): a view's rows end up in
-  // one range, by cell, biggest h first, ties in input order
-  launch_radix_sort2(b->sh_sk.p, b->sh_perm.p, b->sh_gkey.p, n32, 16, b->sh_temp.p, s);
-  launch_radix_sort(b->sh_gkey.p, b->sh_perm.p, n32, key_bits_for(b->sh_ncells - 1), b->sh_temp.p,
-                    s);
+  launch_radix_chain(rc, true, false, s);
   // view-local cell keys for the gather; the global ones (sh_gkey) give the
   // cell ranges
   launch_local_keys(b->sh_gkey.p, b->sh_cbase.p, static_cast<int>(nv), n32, b->sh_key.p, s);
-  launch_fill_u32(b->sh_counts.p, 0u, nc + 1, s);
   launch_build_soa(b->sh_p4c.p, nullptr, b->sh_perm.p, b->sh_gkey.p, n32, kernel_norm(b->kernel),
                    b->kernel != ILC_KERNEL_CUBIC,
                    b->sh_part.p, b->sh_hs.p, b->sh_counts.p, maxh, s,
@@ -777,7 +775,7 @@ void device_work(ilc_batch* b, bool persistent, hipStream_t s, bool timed = fals
   launch_fill_u32(b->counter.p, 0u, 2, s);
   b->qcounters.ensure(size_t(kQueues) * kQueueStride);
   launch_fill_u32(b->qcounters.p, 0u, uint64_t(kQueues) * kQueueStride, s);
-  const build_ctx main{&b->scratch, &b->p4tmp, &b->htmp, &b->wcounts, &b->woffs, s};
+  const build_ctx main{&b->scratch, &b->p4tmp, &b->htmp, &b->wcounts, &b->woffs, &b->scan_temp, s};
   if (!persistent) {
     for (size_t gi = 0; gi < b->group_leader.size(); ++gi) build_group(b, gi, main);
     for (size_t v = 0; v < nv; ++v) {
@@ -797,7 +795,7 @@ void device_work(ilc_batch* b, bool persistent, hipStream_t s, bool timed = fals
     size_t job = 0;
     auto lane_ctx = [&](size_t j) {
       build_lane& l = *b->lanes[j % b->lanes.size()];
-      return build_ctx{&l.scratch, &l.p4tmp, &l.htmp, &l.wcounts, &l.woffs, l.st};
+      return build_ctx{&l.scratch, &l.p4tmp, &l.htmp, &l.wcounts, &l.woffs, &l.scan_temp, l.st};
     };
     for (size_t gi = 0; gi < b->group_leader.size(); ++gi) build_group(b, gi, lane_ctx(job++));
     if (b->shared) {

@@ -81,75 +81,19 @@ __device__ inline void particle_of(const particle_soa& ps, const view_proj& vp, 
   out[2] = dot3(vp.m + 6, vx, vy, vz);
 }
 
-template <bool WRITE>
 __global__ __launch_bounds__(kBlock) void k_view_pass(particle_soa ps, view_proj vp,
-                                                       gaunt_table gt, float4* __restrict__ out,
-                                                       float* __restrict__ part,
-                                                       uint32_t* __restrict__ bad) {
+                                                       gaunt_table gt, float4* __restrict__ out) {
   __shared__ float tab[kMaxGaunt];
   if (vp.quantity == 1) {
     for (int i = threadIdx.x; i < gt.n; i += kBlock) tab[i] = gt.y[i];
     __syncthreads();
   }
-  float mn0 = INFINITY, mn1 = INFINITY, mx0 = -INFINITY, mx1 = -INFINITY, mh = 0.0f;
-  uint32_t nbad = 0;
   for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < ps.n;
        i += uint64_t(gridDim.x) * kBlock) {
     float pc[3], w;
     particle_of(ps, vp, tab, gt.n, gt.x0, gt.dx, i, pc, &w);
     if (pc[2] < 0.0f || pc[2] > vp.depth) w = 0.0f;
-    if constexpr (WRITE) {
-      out[i] = make_float4(pc[0], pc[1], 0.0f, w);
-    } else {
-      const float hh = ps.hsml[i];
-      const bool ok = isfinite(pc[0]) && isfinite(pc[1]) && isfinite(w) && hh >= 1.1e-19f &&
-                      hh <= 1.8e19f;
-      if (!ok) {
-        ++nbad;
-        continue;
-      }
-      mn0 = fminf(mn0, pc[0]);
-      mx0 = fmaxf(mx0, pc[0]);
-      mn1 = fminf(mn1, pc[1]);
-      mx1 = fmaxf(mx1, pc[1]);
-      mh = fmaxf(mh, hh);
-    }
-  }
-  if constexpr (!WRITE) {
-    __shared__ float red[4][5];
-    __shared__ uint32_t redb[4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const float v[5] = {wmin(mn0), wmin(mn1), wmax(mx0), wmax(mx1), wmax(mh)};
-    uint32_t b = nbad;
-    for (int o = 32; o > 0; o >>= 1) b += __shfl_xor(b, o, 64);
-    if (lane == 0) {
-      for (int k = 0; k < 5; ++k) red[wave][k] = v[k];
-      redb[wave] = b;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      float r[5];
-      for (int k = 0; k < 5; ++k) r[k] = red[0][k];
-      uint32_t bb = redb[0];
-      for (int w = 1; w < 4; ++w) {
-        r[0] = fminf(r[0], red[w][0]);
-        r[1] = fminf(r[1], red[w][1]);
-        r[2] = fmaxf(r[2], red[w][2]);
-        r[3] = fmaxf(r[3], red[w][3]);
-        r[4] = fmaxf(r[4], red[w][4]);
-        bb += redb[w];
-      }
-      // layout of the bbox partials: min x, y, z, max x, y, z, max h
-      float* o = part + blockIdx.x * 8;
-      o[0] = r[0];
-      o[1] = r[1];
-      o[2] = 0.0f;
-      o[3] = r[2];
-      o[4] = r[3];
-      o[5] = 0.0f;
-      o[6] = r[4];
-      if (bb) atomicAdd(bad, bb);
-    }
+    out[i] = make_float4(pc[0], pc[1], 0.0f, w);
   }
 }
 
@@ -654,7 +598,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_window_scatter(
     particle_soa ps, const float* __restrict__ wx, const view_build_desc* __restrict__ vd,
     const int32_t* __restrict__ views, int nviews, uint32_t ntiles,
     const uint32_t* __restrict__ offs, float4* __restrict__ p4c, uint32_t* __restrict__ hqkey,
-    uint32_t* __restrict__ hqval, uint32_t* __restrict__ gkey, uint32_t* __restrict__ orig,
+    uint32_t* __restrict__ gkey, uint32_t* __restrict__ orig,
     uint32_t* __restrict__ err,
     const uint32_t* __restrict__ cbase, uint32_t* __restrict__ maxh_bits,
     float2* __restrict__ zc, slab_stack stack) {
@@ -764,7 +708,6 @@ __global__ __launch_bounds__(kBlock) void k_multi_window_scatter(
     if (zc) zc[j] = make_float2((0.0f - az) / hh, (vp.depth - az) / hh);
     p4c[j] = make_float4(ax, ay, hh, w);
     hqkey[j] = hq_key(hh);
-    hqval[j] = j;
     bool in_grid;
     const uint32_t key = cell_key(g, ax, ay, &in_grid);
     if (!in_grid) atomicAdd(err, 1u);
@@ -921,13 +864,6 @@ __global__ __launch_bounds__(kBlock) void k_multi_window_scatter(
 }
 
 
-__global__ __launch_bounds__(kBlock) void k_gather_u32(const uint32_t* __restrict__ src,
-                                                       const uint32_t* __restrict__ idx,
-                                                       uint32_t n, uint32_t* __restrict__ out) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) out[i] = src[idx[i]];
-}
-
 // Work-item order of the persistent gather.  A tile's cost is dominated by
 // the particles of the grid cells under its points: a tile over a dense core
 // streams and evaluates the most, and started last it runs on alone while
@@ -941,8 +877,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_u32(const uint32_t* __restric
 __global__ __launch_bounds__(kBlock) void k_item_cost(const view_desc* __restrict__ views,
                                                       const uint2* __restrict__ items,
                                                       queue_segs segs, uint32_t n, int side,
-                                                      uint32_t* __restrict__ keys,
-                                                      uint32_t* __restrict__ idx) {
+                                                      uint32_t* __restrict__ keys) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   uint32_t q = 0;
@@ -984,7 +919,6 @@ __global__ __launch_bounds__(kBlock) void k_item_cost(const view_desc* __restric
   const int bits = c32 ? 32 - __clz(c32) : 0;
   const bool heavy = cost >= 16u * uint64_t(vd.cost_unit);
   keys[i] = (q << 5) | (heavy ? uint32_t(31 - min(bits, 31)) : 31u);
-  idx[i] = i;
 }
 
 __global__ __launch_bounds__(kBlock) void k_permute_items(const uint2* __restrict__ items,
@@ -1019,7 +953,7 @@ __global__ __launch_bounds__(kBlock) void k_local_keys(const uint32_t* __restric
 __global__ __launch_bounds__(kBlock) void k_window_scatter(
     particle_soa ps, view_proj vp, gaunt_table gt, window_f win,
     const uint32_t* __restrict__ offsets, grid_params g, float4* __restrict__ p4c,
-    float* __restrict__ hc, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+    float* __restrict__ hc, uint32_t* __restrict__ keys, uint32_t* __restrict__ hkeys,
     uint32_t* __restrict__ orig, uint32_t* __restrict__ err) {
 #pragma clang fp contract(off)
   __shared__ float tab[kMaxGaunt];
@@ -1053,7 +987,8 @@ __global__ __launch_bounds__(kBlock) void k_window_scatter(
       particle_of(ps, vp, tab, gt.n, gt.x0, gt.dx, i, pc, &w);
       if (pc[2] < 0.0f || pc[2] > vp.depth) w = 0.0f;
       p4c[j] = make_float4(pc[0], pc[1], 0.0f, w);
-      hc[j] = ps.hsml[i];
+      const float hh = ps.hsml[i];
+      hc[j] = hh;
       // cell key of (x', y', 0): grid3d_get_cell_indices, particle_grid.cl:45-53
       const float c3[3] = {pc[0], pc[1], 0.0f};
       int32_t idx[3];
@@ -1070,7 +1005,7 @@ __global__ __launch_bounds__(kBlock) void k_window_scatter(
       else
         atomicAdd(err, 1u);
       keys[j] = key;
-      vals[j] = j;
+      hkeys[j] = hq_key(hh);
       orig[j] = uint32_t(i);
     }
     out += tot;
@@ -1137,7 +1072,6 @@ void launch_particle_xray(const particle_soa& ps, const gaunt_table& gt, float* 
 void launch_multi_window_scatter(const particle_soa& ps, const float* wx,
                                  const view_build_desc* vd_dev, const int32_t* views_dev,
                                  int nviews, const uint32_t* offs, float4* p4c, uint32_t* hqkey,
-                                 uint32_t* hqval,
                                  uint32_t* gkey, uint32_t* orig, uint32_t* err,
                                  const uint32_t* cbase, uint32_t* maxh_bits, float2* zc,
                                  const slab_stack& stack, hipStream_t s) {
@@ -1147,16 +1081,8 @@ void launch_multi_window_scatter(const particle_soa& ps, const float* wx,
   ILC_REQUIRE(stack.n == 0 || (stack.n == nviews && stack.n <= kStackMax && zc == nullptr),
               "a slab stack lists every view, at most %d, centre masks only", kStackMax);
   hipLaunchKernelGGL(k_multi_window_scatter, dim3(nb), dim3(kBlock), 0, s, ps, wx, vd_dev,
-                     views_dev, nviews, nb, offs, p4c, hqkey, hqval, gkey, orig, err, cbase,
+                     views_dev, nviews, nb, offs, p4c, hqkey, gkey, orig, err, cbase,
                      maxh_bits, zc, stack);
-  ILC_HIP(hipGetLastError());
-}
-
-void launch_gather_u32(const uint32_t* src, const uint32_t* idx, uint32_t n, uint32_t* out,
-                       hipStream_t s) {
-  if (!n) return;
-  hipLaunchKernelGGL(k_gather_u32, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, src, idx,
-                     n, out);
   ILC_HIP(hipGetLastError());
 }
 
@@ -1173,10 +1099,12 @@ void launch_order_items(const view_desc* views, const uint2* items, const queue_
                         uint32_t n, const sum_shape& ts, uint32_t* keys, uint32_t* idx,
                         uint32_t* radix_temp, uint2* out, hipStream_t s) {
   if (!n) return;
+  const radix_chain c = plan_radix_chain(keys, idx, n, 0, 8, radix_temp);
+  launch_zero({radix_chain_zero(c)}, s);
   hipLaunchKernelGGL(k_item_cost, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, views,
-                     items, segs, n, ts.side, keys, idx);
+                     items, segs, n, ts.side, c.b[c.in]);
   ILC_HIP(hipGetLastError());
-  launch_radix_sort(keys, idx, n, 8, radix_temp, s);
+  launch_radix_chain(c, true, false, s);
   hipLaunchKernelGGL(k_permute_items, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, items,
                      idx, n, out);
   ILC_HIP(hipGetLastError());
@@ -1216,31 +1144,15 @@ void launch_multi_window_count(const float* pos3, const float* hsml, uint64_t n,
 
 void launch_window_scatter(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
                            const window_f& win, const uint32_t* offsets, const grid_params& g,
-                           float4* p4c, float* hc, uint32_t* keys, uint32_t* vals, uint32_t* orig,
+                           float4* p4c, float* hc, uint32_t* keys, uint32_t* hkeys, uint32_t* orig,
                            uint32_t* err, hipStream_t s) {
   if (vp.quantity == 1 && (gt.n < 1 || gt.n > kMaxGaunt || !gt.y))
     fail(ILC_EINVAL, "X-ray view without a Gaunt table (1..%d entries)", kMaxGaunt);
   const uint32_t nb = window_tiles(ps.n);
   if (!nb) return;
   hipLaunchKernelGGL(k_window_scatter, dim3(nb), dim3(kBlock), 0, s, ps, vp, gt, win, offsets, g,
-                     p4c, hc, keys, vals, orig, err);
+                     p4c, hc, keys, hkeys, orig, err);
   ILC_HIP(hipGetLastError());
-}
-
-int view_bbox_parts(uint64_t n) {
-  return static_cast<int>(std::max<uint64_t>(1, std::min<uint64_t>(1024, (n + kBlock - 1) / kBlock)));
-}
-
-void launch_view_bbox(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
-                      float* partial, uint32_t* bad, bbox_result* out, hipStream_t s) {
-  if (vp.quantity == 1 && (gt.n < 1 || gt.n > kMaxGaunt || !gt.y))
-    fail(ILC_EINVAL, "X-ray view without a Gaunt table (1..%d entries)", kMaxGaunt);
-  const int nparts = view_bbox_parts(ps.n);
-  launch_fill_u32(bad, 0u, 1, s);
-  hipLaunchKernelGGL(k_view_pass<false>, dim3(nparts), dim3(kBlock), 0, s, ps, vp, gt, nullptr,
-                     partial, bad);
-  ILC_HIP(hipGetLastError());
-  launch_bbox_final(partial, nparts, bad, out, s);
 }
 
 void launch_view_project(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
@@ -1248,8 +1160,7 @@ void launch_view_project(const particle_soa& ps, const view_proj& vp, const gaun
   uint64_t nb = (ps.n + kBlock - 1) / kBlock;
   if (nb > 16384) nb = 16384;
   if (nb == 0) nb = 1;
-  hipLaunchKernelGGL(k_view_pass<true>, dim3(uint32_t(nb)), dim3(kBlock), 0, s, ps, vp, gt, out,
-                     nullptr, nullptr);
+  hipLaunchKernelGGL(k_view_pass, dim3(uint32_t(nb)), dim3(kBlock), 0, s, ps, vp, gt, out);
   ILC_HIP(hipGetLastError());
 }
 

@@ -186,7 +186,7 @@ ilc_status ilc_psg_setup_projected_particles(ilc_psg* h, const float* particles4
     sc.bbox_partial.ensure(size_t(nparts) * 8);
     sc.bbox_dev.ensure(1);
     sc.flags.ensure(2);
-    launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.flags.p, sc.bbox_dev.p, s);
+    launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.bbox_dev.p, s);
     ILC_HIP(hipMemcpyAsync(h->bbox_host, sc.bbox_dev.p, sizeof(bbox_result),
                            hipMemcpyDeviceToHost, s));
     ILC_HIP(hipStreamSynchronize(s));
@@ -195,8 +195,8 @@ ilc_status ilc_psg_setup_projected_particles(ilc_psg* h, const float* particles4
     int32_t kz0 = 0;
     const grid_params g = plan_grid(bb, n, h->target, h->mode, &kz0);
     // 3. keys, stable sort, SoA, counts, max h, offsets
-    launch_fill_u32(sc.flags.p, 0u, 1, s);
-    enqueue_grid_build(h->grid, sc, p4, hsml_dev, n, g, kz0, bb.max_h, h->kernel, sc.flags.p, s);
+    enqueue_grid_build(h->grid, sc, p4, hsml_dev, n, g, kz0, bb.max_h, h->kernel, sc.flags.p, true,
+                       s);
     ILC_HIP(hipMemcpyAsync(h->flags_host, sc.flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     ILC_HIP(hipStreamSynchronize(s));
     if (h->flags_host[0]) {
@@ -327,7 +327,7 @@ ilc_status ilc_psg_export_grid(const ilc_psg* h, int32_t* cells2_dev, float* max
       const uint64_t n = h->grid.n;
       dbuf<uint32_t> by_index, temp;
       by_index.ensure(n);
-      temp.ensure(radix_temp_words(n));
+      temp.ensure(radix_chain_words(n));
       launch_reference_perm(h->grid.key.p, h->grid.perm.p, static_cast<uint32_t>(n),
                             key_bits_for(h->grid.gp.ncells() - 1), perm_dev, by_index.p, temp.p, s);
       ILC_HIP(hipStreamSynchronize(s));  // the temporaries are freed on return
@@ -491,7 +491,7 @@ ilc_status ilc_grid3d_setup_particles(ilc_grid3d* g3, const float* particles4_de
     sc.bbox_partial.ensure(size_t(nparts) * 8);
     sc.bbox_dev.ensure(1);
     sc.flags.ensure(2);
-    launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.flags.p, sc.bbox_dev.p, s);
+    launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.bbox_dev.p, s);
     ILC_HIP(hipMemcpyAsync(h->bbox_host, sc.bbox_dev.p, sizeof(bbox_result),
                            hipMemcpyDeviceToHost, s));
     ILC_HIP(hipStreamSynchronize(s));
@@ -503,7 +503,6 @@ ilc_status ilc_grid3d_setup_particles(ilc_grid3d* g3, const float* particles4_de
     // the masked list packs a cell's x and y into 16 bits each
     if (h->mode == ILC_MODE_REFERENCE && (g.nc[0] > 65536 || g.nc[1] > 65536))
       fail(ILC_ERANGE, "grid of %d x %d cells in x, y (at most 65536 each)", g.nc[0], g.nc[1]);
-    launch_fill_u32(sc.flags.p, 0u, 1, s);
     enqueue_volumetric_grid(h->grid, sc, p4, hsml_dev, n, g, bb.max_h, h->kernel, sc.flags.p, s);
     ILC_HIP(hipMemcpyAsync(h->flags_host, sc.flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     ILC_HIP(hipStreamSynchronize(s));

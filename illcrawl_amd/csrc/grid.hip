@@ -10,6 +10,8 @@
 // come from a scan of per-cell counts.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -25,6 +27,15 @@ __device__ inline float wave_max(float v) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
 }
+// orders this wave's LDS accesses (lanes read what others of the wave wrote)
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Descending h: the top 16 bits of its float pattern (h > 0, so the pattern
+// orders like the value), reversed.
+__device__ inline uint32_t h_order_key(float h) { return 0x7fffu - (__float_as_uint(h) >> 16); }
 __device__ inline uint32_t wave_sum(uint32_t v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -42,13 +53,26 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
     p[i] = v;
 }
 
+struct fill_regions {
+  uint32_t* p[4];
+  uint64_t n[4];
+};
+
+// zeroes up to four arrays
+__global__ __launch_bounds__(kBlock) void k_zero(fill_regions r) {
+  const uint64_t i0 = blockIdx.x * uint64_t(kBlock) + threadIdx.x;
+  const uint64_t step = uint64_t(gridDim.x) * kBlock;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    for (uint64_t i = i0; i < r.n[k]; i += step) r.p[k][i] = 0u;
+}
+
 // Per-block min/max of x, y, z, max h, and a count of invalid particles.
 // Non-finite coordinates or w, and h that is not a positive normal float
 // whose square stays finite, are invalid.
 __global__ __launch_bounds__(kBlock) void k_bbox_partial(const float4* __restrict__ p4,
                                                           const float* __restrict__ h,
-                                                          uint64_t n, float* __restrict__ part,
-                                                          uint32_t* __restrict__ bad) {
+                                                          uint64_t n, float* __restrict__ part) {
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   float mh = 0.0f;
   uint32_t nbad = 0;
@@ -88,32 +112,42 @@ __global__ __launch_bounds__(kBlock) void k_bbox_partial(const float4* __restric
       bb += redb[w];
     }
     for (int k = 0; k < 7; ++k) part[blockIdx.x * 8 + k] = r[k];
-    if (bb) atomicAdd(bad, bb);
+    part[blockIdx.x * 8 + 7] = __uint_as_float(bb);
   }
 }
 
 __global__ __launch_bounds__(kBlock) void k_bbox_final(const float* __restrict__ part, int nparts,
-                                                        const uint32_t* __restrict__ bad,
                                                         bbox_result* __restrict__ out) {
-  __shared__ float red[kBlock][7];
+  __shared__ float red[4][7];
+  __shared__ uint32_t redb[4];
   float r[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0f};
+  uint32_t bad = 0;
   for (int i = threadIdx.x; i < nparts; i += kBlock) {
     for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], part[i * 8 + k]);
     for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], part[i * 8 + k]);
+    bad += __float_as_uint(part[i * 8 + 7]);
   }
-  for (int k = 0; k < 7; ++k) red[threadIdx.x][k] = r[k];
+  for (int k = 0; k < 3; ++k) r[k] = wave_min(r[k]);
+  for (int k = 3; k < 7; ++k) r[k] = wave_max(r[k]);
+  bad = wave_sum(bad);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane == 0) {
+    for (int k = 0; k < 7; ++k) red[wave][k] = r[k];
+    redb[wave] = bad;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int i = 1; i < kBlock; ++i) {
-      for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], red[i][k]);
-      for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], red[i][k]);
+    for (int w = 1; w < 4; ++w) {
+      for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], red[w][k]);
+      for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], red[w][k]);
+      bad += redb[w];
     }
     for (int k = 0; k < 3; ++k) {
       out->mn[k] = r[k];
       out->mx[k] = r[3 + k];
     }
     out->max_h = r[6];
-    out->bad = *bad;
+    out->bad = bad;
   }
 }
 
@@ -125,35 +159,6 @@ __device__ inline int32_t floor_to_int(float f) {
   if (fl >= 2147483647.0f) return INT32_MAX;
   if (fl <= -2147483648.0f) return INT32_MIN;
   return static_cast<int32_t>(fl);
-}
-
-// keys[i] = cell of particle i (grid3d_generate_sort_keys,
-// particle_grid.cl:96-112), vals[i] = i.  Keys outside the grid (the
-// reference writes out of bounds there) are counted in *err and clamped.
-__global__ __launch_bounds__(kBlock) void k_keys(const float4* __restrict__ p4, uint32_t n,
-                                                  grid_params g, uint32_t* __restrict__ keys,
-                                                  uint32_t* __restrict__ vals,
-                                                  uint32_t* __restrict__ err) {
-#pragma clang fp contract(off)
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const float4 q = p4[i];
-  const float c[3] = {q.x, q.y, q.z};
-  int32_t idx[3];
-  bool ok = true;
-  for (int a = 0; a < 3; ++a) {
-    const float d = c[a] - g.minc[a];
-    idx[a] = floor_to_int(d / g.cs[a]);
-    ok = ok && idx[a] >= 0 && idx[a] < g.nc[a];
-  }
-  uint32_t key = 0;
-  if (ok)
-    key = uint32_t(idx[0]) + uint32_t(idx[1]) * uint32_t(g.nc[0]) +
-          uint32_t(idx[2]) * uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
-  else
-    atomicAdd(err, 1u);
-  keys[i] = key;
-  vals[i] = i;
 }
 
 // exclusive scan over the workgroup (kBlock threads)
@@ -180,120 +185,249 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
 constexpr int kItems = 16;
 constexpr int kTile = kBlock * kItems;  // 4096 keys per workgroup
 
-// The lanes of the wave whose digit equals this lane's (8 ballots), among
-// the valid lanes.
-__device__ inline uint64_t digit_peers(uint32_t d, bool valid) {
+// The active lanes of the wave whose `bits` low bits of d equal this lane's,
+// among the valid ones.
+__device__ inline uint64_t match_peers(uint32_t d, int bits, bool valid) {
   uint64_t peers = __ballot(valid);
-  for (int b = 0; b < 8; ++b) {
+  for (int b = 0; b < bits; ++b) {
     const bool bit = (d >> b) & 1u;
     const uint64_t m = __ballot(bit);
     peers &= bit ? m : ~m;
   }
   return peers;
 }
+__device__ inline uint64_t digit_peers(uint32_t d, bool valid) { return match_peers(d, 8, valid); }
+
+// Counts digit d at position pos into its tile's counts hist[tile][256]
+// (tiles of 1 << tile_log items, tile_bits bits of tile index), one add per
+// distinct (tile, digit) of a wave.
+__device__ inline void count_digit(uint32_t* __restrict__ hist, uint32_t pos, uint32_t d,
+                                   int tile_log, int tile_bits) {
+  const uint32_t bin = (pos >> tile_log) << 8 | d;
+  const uint64_t peers = match_peers(bin, 8 + tile_bits, true);
+  if ((peers & lanes_below()) == 0) atomicAdd(hist + bin, uint32_t(__popcll(peers)));
+}
+
+// keys[i] = cell of particle i (grid3d_generate_sort_keys,
+// particle_grid.cl:96-112), hkeys[i] = its descending-h key (launch of the
+// sort by (cell, descending h)).  Keys outside the grid (the reference writes
+// out of bounds there) are counted in *err and clamped.  hist (may be NULL):
+// the first digit of hkeys is counted into it.
+__global__ __launch_bounds__(kBlock) void k_keys(const float4* __restrict__ p4,
+                                                  const float* __restrict__ h, uint32_t n,
+                                                  grid_params g, uint32_t* __restrict__ hkeys,
+                                                  uint32_t* __restrict__ keys,
+                                                  uint32_t* __restrict__ err,
+                                                  uint32_t* __restrict__ hist, int tile_log,
+                                                  int tile_bits) {
+#pragma clang fp contract(off)
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const float4 q = p4[i];
+  const float c[3] = {q.x, q.y, q.z};
+  int32_t idx[3];
+  bool ok = true;
+  for (int a = 0; a < 3; ++a) {
+    const float d = c[a] - g.minc[a];
+    idx[a] = floor_to_int(d / g.cs[a]);
+    ok = ok && idx[a] >= 0 && idx[a] < g.nc[a];
+  }
+  uint32_t key = 0;
+  if (ok)
+    key = uint32_t(idx[0]) + uint32_t(idx[1]) * uint32_t(g.nc[0]) +
+          uint32_t(idx[2]) * uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
+  else
+    atomicAdd(err, 1u);
+  keys[i] = key;
+  const uint32_t hk = h_order_key(h[i]);
+  hkeys[i] = hk;
+  if (hist) count_digit(hist, i, hk & 255u, tile_log, tile_bits);
+}
 
 // Per-tile digit counts, one LDS add per distinct digit of a wave (a digit
 // with few distinct values would serialise a wave's 64 adds on one word).
+// Layout hist[digit][tile], or hist[tile][digit] (tile_major).
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t* __restrict__ keys,
                                                         uint32_t n, int shift, uint32_t ntiles,
-                                                        uint32_t* __restrict__ hist) {
+                                                        uint32_t* __restrict__ hist,
+                                                        int tile_major) {
   __shared__ uint32_t hh[256];
   hh[threadIdx.x] = 0;
-  const uint32_t base = blockIdx.x * kTile;
-  uint32_t k[kItems];
+  const uint32_t base = blockIdx.x * (kBlock * ITEMS);
+  uint32_t k[ITEMS];
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t i = base + r * kBlock + threadIdx.x;
     k[r] = i < n ? keys[i] : 0u;
   }
   __syncthreads();
   const uint64_t below = lanes_below();
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const bool valid = base + r * kBlock + threadIdx.x < n;
     const uint32_t d = (k[r] >> shift) & 255u;
     const uint64_t peers = digit_peers(d, valid);
     if (valid && (peers & below) == 0) atomicAdd(&hh[d], uint32_t(__popcll(peers)));
   }
   __syncthreads();
-  hist[threadIdx.x * ntiles + blockIdx.x] = hh[threadIdx.x];
+  if (tile_major)
+    hist[blockIdx.x * 256 + threadIdx.x] = hh[threadIdx.x];
+  else
+    hist[threadIdx.x * ntiles + blockIdx.x] = hh[threadIdx.x];
 }
 
-// Stable scatter of one 8-bit digit.  Items of a tile are visited in input
-// order (round r, thread t -> item r*256 + t); within a wave, lanes sharing a
-// digit are found with 8 ballots and ranked by popcount of lower lanes;
-// across waves and rounds, per-digit running counts in LDS keep the order.
-// The tile is first ordered by digit in LDS and then written out in that
-// order, so each digit's items leave as one contiguous run: item i of the
-// ordered tile, of digit d, goes to offs[d, tile] + i - (the tile's items
-// below digit d).
-// V2: a second value array moves with the first.
-template <bool V2>
-__global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t* __restrict__ kin,
-                                                           const uint32_t* __restrict__ vin,
-                                                           uint32_t* __restrict__ kout,
-                                                           uint32_t* __restrict__ vout, uint32_t n,
-                                                           int shift, uint32_t ntiles,
-                                                           const uint32_t* __restrict__ offs,
-                                                           const uint32_t* __restrict__ vin2,
-                                                           uint32_t* __restrict__ vout2) {
-  __shared__ uint32_t sk[kTile];
-  __shared__ uint32_t sv[kTile];
-  __shared__ uint32_t sv2[V2 ? kTile : 1];
+// One stable pass over an 8-bit digit of kin.  A wave ranks its own 64 *
+// ITEMS consecutive items (lanes sharing a digit found with 8 ballots, running
+// counts of its own in LDS: no barrier per row); the waves' counts then give
+// every item its place in the tile ordered by digit, where it goes through
+// LDS, so that each digit's items leave as one contiguous run.  (With shared
+// counts and three barriers per row of 256 items a pass over 8k items took
+// 13.6 us.)
+// vin NULL: the values are the input positions.  kout NULL: the keys are not
+// needed afterwards.  BP: a second value array moves with the first.
+// SMALL: the counts are hist[tile][digit] of every tile, which the workgroup
+// adds up itself (no scan launches); else hist holds the scanned counts
+// hist[digit][tile].  With 4 items a thread the next pass's digit (of the key,
+// or of the second value) is counted into next.hist (NULL: last pass).
+struct radix_next {
+  uint32_t* hist;
+  int shift;
+  int of_second;
+  int tile_bits;
+};
+template <int ITEMS, bool BP, bool SMALL>
+__global__ __launch_bounds__(kBlock) void k_radix_scatter(
+    const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+    const uint32_t* __restrict__ bin, uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+    uint32_t* __restrict__ bout, uint32_t n, int shift, uint32_t ntiles,
+    const uint32_t* __restrict__ hist, radix_next next) {
+  constexpr int TILE = kBlock * ITEMS;
+  constexpr bool COUNTING = ITEMS == 4;
+  // the ordered tile, one array at a time (3 arrays of 4096 words at once
+  // left 3 workgroups per CU: 170 us instead of 97 for a pass over 16M rows
+  // with both values)
+  __shared__ uint32_t so[TILE];
   __shared__ uint32_t gofs[256];
-  __shared__ uint32_t run[256];
   __shared__ uint32_t wc[4][256];
   const uint32_t t = threadIdx.x;
-  const int wave = t >> 6;
-  const uint32_t tile0 = blockIdx.x * kTile;
-  uint32_t k[kItems], v[kItems], v2[V2 ? kItems : 1];
+  const int wave = t >> 6, lane = t & 63;
+  const uint32_t tile0 = blockIdx.x * TILE;
+  const uint32_t w0 = tile0 + uint32_t(wave) * (64 * ITEMS) + uint32_t(lane);
+  uint32_t k[ITEMS], v[ITEMS], b[BP ? ITEMS : 1];
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
-    const uint32_t i = tile0 + r * kBlock + t;
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t i = w0 + r * 64;
     k[r] = i < n ? kin[i] : 0u;
-    v[r] = i < n ? vin[i] : 0u;
-    if constexpr (V2) v2[r] = i < n ? vin2[i] : 0u;
+    v[r] = vin ? (i < n ? vin[i] : 0u) : i;
+    if constexpr (BP) b[r] = i < n ? bin[i] : 0u;
   }
-  // the tile's count of digit t from the scanned counts (the last entry's
-  // successor is the total, n)
-  const uint64_t e = uint64_t(t) * ntiles + blockIdx.x;
-  const uint32_t g0 = offs[e];
-  const uint32_t cnt = (e + 1 < uint64_t(256) * ntiles ? offs[e + 1] : n) - g0;
-  uint32_t tot;
-  const uint32_t ls = block_exclusive_scan(cnt, &tot);
-  run[t] = ls;
-  gofs[t] = g0 - ls;
-  for (int w = 0; w < 4; ++w) wc[w][t] = 0;
-  __syncthreads();
-  const uint64_t below = lanes_below();
+  // digit t's first position in the output
+  uint32_t g0;
+  if constexpr (SMALL) {
+    // wave w adds up the counts of tiles w, w + 4, ..., four digits per lane
+    const uint4* h4 = reinterpret_cast<const uint4*>(hist);
+    uint4 all = make_uint4(0, 0, 0, 0), before = make_uint4(0, 0, 0, 0);
+#pragma unroll 16
+    for (uint32_t j = uint32_t(wave); j < ntiles; j += 4) {
+      const uint4 c = h4[j * 64 + uint32_t(lane)];
+      all.x += c.x;
+      all.y += c.y;
+      all.z += c.z;
+      all.w += c.w;
+      const bool b4 = j < blockIdx.x;
+      before.x += b4 ? c.x : 0u;
+      before.y += b4 ? c.y : 0u;
+      before.z += b4 ? c.z : 0u;
+      before.w += b4 ? c.w : 0u;
+    }
+    uint4* sum4 = reinterpret_cast<uint4*>(so);  // [2][4 waves][64]
+    sum4[wave * 64 + lane] = all;
+    sum4[256 + wave * 64 + lane] = before;
+    __syncthreads();
+    uint32_t a1 = 0, b1 = 0;
+    for (int w = 0; w < 4; ++w) {
+      a1 += so[w * 256 + t];
+      b1 += so[1024 + w * 256 + t];
+    }
+    uint32_t tot;
+    g0 = block_exclusive_scan(a1, &tot) + b1;  // ends with a barrier
+  } else {
+    g0 = hist[uint64_t(t) * ntiles + blockIdx.x];
+  }
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
-    const bool valid = tile0 + r * kBlock + t < n;
+  for (int j = 0; j < 4; ++j) wc[wave][lane + 64 * j] = 0;
+  wave_fence();
+  const uint64_t below = lanes_below();
+  uint32_t rank[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const bool valid = w0 + r * 64 < n;
     const uint32_t d = (k[r] >> shift) & 255u;
     const uint64_t peers = digit_peers(d, valid);
-    const uint32_t rank = __popcll(peers & below);
-    if (valid && rank == 0) wc[wave][d] = __popcll(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = run[d] + rank;
-      for (int w = 0; w < wave; ++w) pos += wc[w][d];
-      sk[pos] = k[r];
-      sv[pos] = v[r];
-      if constexpr (V2) sv2[pos] = v2[r];
+    const uint32_t old = wc[wave][d];
+    rank[r] = old + uint32_t(__popcll(peers & below));
+    wave_fence();
+    if (valid && (peers & below) == 0) wc[wave][d] = old + uint32_t(__popcll(peers));
+    wave_fence();
+  }
+  __syncthreads();
+  {
+    uint32_t c[4], cnt = 0;
+    for (int w = 0; w < 4; ++w) {
+      c[w] = wc[w][t];
+      cnt += c[w];
     }
-    __syncthreads();
-    run[t] += wc[0][t] + wc[1][t] + wc[2][t] + wc[3][t];
-    for (int w = 0; w < 4; ++w) wc[w][t] = 0;
-    __syncthreads();
+    uint32_t tot;
+    uint32_t ls = block_exclusive_scan(cnt, &tot);
+    gofs[t] = g0 - ls;
+    for (int w = 0; w < 4; ++w) {
+      wc[w][t] = ls;
+      ls += c[w];
+    }
   }
-  const uint32_t nv = min(uint32_t(kTile), n - tile0);
-  for (uint32_t i = t; i < nv; i += kBlock) {
-    const uint32_t key = sk[i];
-    const uint32_t pos = gofs[(key >> shift) & 255u] + i;
-    kout[pos] = key;
-    vout[pos] = sv[i];
-    if constexpr (V2) vout2[pos] = sv2[i];
+  __syncthreads();
+  // place in the ordered tile, then the keys: item i of the tile goes to
+  // gofs[digit] + i
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    rank[r] += wc[wave][(k[r] >> shift) & 255u];
+    if (w0 + r * 64 < n) so[rank[r]] = k[r];
   }
+  __syncthreads();
+  const uint32_t nv = min(uint32_t(TILE), n - tile0);
+  uint32_t pos[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t i = t + r * kBlock;
+    if (i < nv) {
+      const uint32_t key = so[i];
+      pos[r] = gofs[(key >> shift) & 255u] + i;
+      if (kout) kout[pos[r]] = key;
+      if constexpr (COUNTING)
+        if (next.hist && !(BP && next.of_second))
+          count_digit(next.hist, pos[r], (key >> next.shift) & 255u, 10, next.tile_bits);
+    }
+  }
+  auto put = [&](const uint32_t* x, uint32_t* __restrict__ out, bool count) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+      if (w0 + r * 64 < n) so[rank[r]] = x[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      const uint32_t i = t + r * kBlock;
+      if (i < nv) {
+        const uint32_t y = so[i];
+        out[pos[r]] = y;
+        if constexpr (COUNTING)
+          if (count) count_digit(next.hist, pos[r], (y >> next.shift) & 255u, 10, next.tile_bits);
+      }
+    }
+  };
+  put(v, vout, false);
+  if constexpr (BP) put(b, bout, COUNTING && next.hist && next.of_second);
 }
 
 // ---- exclusive scan of uint32 (reduce, scan of block sums, apply)
@@ -396,6 +530,39 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const uint32_t* __restric
   }
 }
 
+// A scan of at most 1024 * ITEMS words in one workgroup of 16 waves (one
+// launch, not three).
+constexpr uint64_t kOneScanMax = 1 << 15;
+template <int ITEMS>
+__global__ __launch_bounds__(1024) void k_scan_one(const uint32_t* in, uint32_t* out,
+                                                    uint32_t n) {
+  __shared__ uint32_t ws[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // word r of the thread: 64 lanes side by side, row r of the wave's block
+  const uint32_t base = uint32_t(wave) * (64 * ITEMS) + uint32_t(lane);
+  uint32_t v[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) v[r] = base + r * 64 < n ? in[base + r * 64] : 0u;
+  uint32_t carry = 0;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    uint32_t incl = v[r];
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    v[r] = carry + incl - v[r];
+    carry += uint32_t(__builtin_amdgcn_readlane(int(incl), 63));
+  }
+  if (lane == 0) ws[wave] = carry;
+  __syncthreads();
+  uint32_t off = 0;
+  for (int w = 0; w < wave; ++w) off += ws[w];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r)
+    if (base + r * 64 < n) out[base + r * 64] = off + v[r];
+}
+
 // Sorted SoA: part[s] = (x, y, coef, 1/h^2) of particle perm[s], hs[s] = h.
 // coef = w * C / h^2 with C the kernel's normalisation, so that the kernel
 // value is coef * shape(r^2 / h^2).  For the projected quartic (shape
@@ -455,47 +622,15 @@ __global__ __launch_bounds__(kBlock) void k_build_soa(const float4* __restrict__
   }
 }
 
-// Within-cell order for the gather: descending h, to the top 16 bits of its
-// float pattern (h > 0, so the pattern orders like the value).  A stable sort
-// of positions by this key, then the stable sort by cell key, leaves every
-// cell's particles biggest first (ties in input order); a tile then only
-// needs the prefix of a cell whose h can reach it.
-__global__ __launch_bounds__(kBlock) void k_h_order_keys(const float* __restrict__ h,
-                                                         const uint32_t* __restrict__ perm,
-                                                         uint32_t n, uint32_t* __restrict__ hk,
-                                                         uint32_t* __restrict__ hv) {
-  const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
-  if (j >= n) return;
-  hk[j] = 0x7fffu - (__float_as_uint(h[perm[j]]) >> 16);
-  hv[j] = j;
-}
-
-// out_key[i] = key[order[i]], out_perm[i] = perm[order[i]]
-__global__ __launch_bounds__(kBlock) void k_permute_pairs(const uint32_t* __restrict__ order,
-                                                          const uint32_t* __restrict__ key,
-                                                          const uint32_t* __restrict__ perm,
-                                                          uint32_t n,
-                                                          uint32_t* __restrict__ out_key,
-                                                          uint32_t* __restrict__ out_perm) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t j = order[i];
-  out_key[i] = key[j];
-  out_perm[i] = perm[j];
-}
-
-// Cell key of every input index (by_index[perm[j]] = key[j]) and the
-// identity, the input of a stable sort by cell key that gives the
-// reference's order (stable by input index within a cell).
+// Cell key of every input index (by_index[perm[j]] = key[j]), the input of a
+// stable sort by cell key that gives the reference's order (stable by input
+// index within a cell).
 __global__ __launch_bounds__(kBlock) void k_keys_by_index(const uint32_t* __restrict__ key,
                                                           const uint32_t* __restrict__ perm,
                                                           uint32_t n,
-                                                          uint32_t* __restrict__ by_index,
-                                                          uint32_t* __restrict__ iota) {
+                                                          uint32_t* __restrict__ by_index) {
   const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
-  if (j >= n) return;
-  by_index[perm[j]] = key[j];
-  iota[j] = j;
+  if (j < n) by_index[perm[j]] = key[j];
 }
 
 // Reference layout of the grid for parity checks.
@@ -557,18 +692,29 @@ void launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s) {
   ILC_HIP(hipGetLastError());
 }
 
-void launch_bbox(const float4* p4, const float* h, uint64_t n, float* partial, int nparts,
-                 uint32_t* bad, bbox_result* out, hipStream_t s) {
-  launch_fill_u32(bad, 0u, 1, s);
-  hipLaunchKernelGGL(k_bbox_partial, dim3(nparts), dim3(kBlock), 0, s, p4, h, n, partial, bad);
-  ILC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, s, partial, nparts, bad, out);
+void launch_zero(std::initializer_list<std::pair<uint32_t*, uint64_t>> regions, hipStream_t s) {
+  fill_regions r{};
+  uint64_t most = 0;
+  int k = 0;
+  for (const auto& x : regions) {
+    ILC_REQUIRE(k < 4, "at most four regions");
+    if (!x.second) continue;
+    r.p[k] = x.first;
+    r.n[k++] = x.second;
+    most = std::max(most, x.second);
+  }
+  if (!k) return;
+  uint32_t nb = blocks_for(most, kBlock);
+  if (nb > 65536) nb = 65536;
+  hipLaunchKernelGGL(k_zero, dim3(nb), dim3(kBlock), 0, s, r);
   ILC_HIP(hipGetLastError());
 }
 
-void launch_bbox_final(const float* partial, int nparts, const uint32_t* bad, bbox_result* out,
-                       hipStream_t s) {
-  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, s, partial, nparts, bad, out);
+void launch_bbox(const float4* p4, const float* h, uint64_t n, float* partial, int nparts,
+                 bbox_result* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_bbox_partial, dim3(nparts), dim3(kBlock), 0, s, p4, h, n, partial);
+  ILC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, s, partial, nparts, out);
   ILC_HIP(hipGetLastError());
 }
 
@@ -580,11 +726,12 @@ void launch_cell_maxh(const float4* p4, const float* h, uint32_t n, const grid_p
   ILC_HIP(hipGetLastError());
 }
 
-void launch_keys(const float4* p4, uint32_t n, const grid_params& g, uint32_t* keys,
-                 uint32_t* vals, uint32_t* err, hipStream_t s) {
+void launch_keys(const float4* p4, const float* h, uint32_t n, const grid_params& g,
+                 const radix_chain& c, uint32_t* err, hipStream_t s) {
   if (!n) return;
-  hipLaunchKernelGGL(k_keys, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, p4, n, g, keys,
-                     vals, err);
+  hipLaunchKernelGGL(k_keys, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, p4, h, n, g,
+                     c.a[c.in], c.b[c.in], err, c.counting ? c.hist : nullptr, c.tile_log,
+                     c.tile_bits);
   ILC_HIP(hipGetLastError());
 }
 
@@ -593,6 +740,14 @@ uint64_t scan_temp_words(uint64_t n) { return blocks_for(n, kTile) + 1; }
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* temp,
                            hipStream_t s) {
   if (!n) return;
+  if (n <= kOneScanMax) {
+    if (n <= 8192)
+      hipLaunchKernelGGL(k_scan_one<8>, dim3(1), dim3(1024), 0, s, in, out, uint32_t(n));
+    else
+      hipLaunchKernelGGL(k_scan_one<32>, dim3(1), dim3(1024), 0, s, in, out, uint32_t(n));
+    ILC_HIP(hipGetLastError());
+    return;
+  }
   const uint32_t nb = blocks_for(n, kTile);
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kBlock), 0, s, in, n, temp);
   ILC_HIP(hipGetLastError());
@@ -602,59 +757,113 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32
   ILC_HIP(hipGetLastError());
 }
 
-uint64_t radix_temp_words(uint64_t n) {
-  const uint64_t ntiles = blocks_for(n, kTile);
-  return 2 * n + 256 * ntiles + scan_temp_words(256 * ntiles);
-}
+// Arrays of up to kSmallTiles tiles are sorted without scan launches: every
+// workgroup adds up all tiles' counts itself (256 KB at most, from L2).  Up
+// to kCountingRows rows (tiles of 1024 items) the passes also count each
+// other's digits with global atomics, one launch a pass: 8k rows 25 us a pass
+// with count, scan and scatter launches, 7 now.  Above, a million atomics
+// cost more than the count launch (1M rows: 33 us a pass against 27).
+constexpr uint32_t kSmallTiles = 256;
+constexpr uint64_t kCountingRows = 128u << 10;
 
 namespace {
-void radix_sort_impl(uint32_t* keys, uint32_t* vals, uint32_t* vals2, uint32_t n, int key_bits,
-                     uint32_t* temp, hipStream_t s) {
-  if (n <= 1 || key_bits <= 0) return;
-  const uint32_t ntiles = blocks_for(n, kTile);
-  uint32_t* k2 = temp;
-  uint32_t* v2 = temp + n;
-  uint32_t* hist = temp + 2 * uint64_t(n);
-  uint32_t* stemp = hist + 256 * uint64_t(ntiles);
-  uint32_t* w2 = temp + radix_temp_words(n);  // the second values' other half (vals2 only)
-  uint32_t *ka = keys, *va = vals, *kb = k2, *vb = v2, *wa = vals2, *wb = w2;
-  int passes = (key_bits + 7) / 8;
-  for (int p = 0; p < passes; ++p) {
-    const int shift = 8 * p;
-    hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(kBlock), 0, s, ka, n, shift, ntiles, hist);
-    ILC_HIP(hipGetLastError());
-    launch_exclusive_scan(hist, hist, uint64_t(256) * ntiles, stemp, s);
-    if (vals2)
-      hipLaunchKernelGGL(k_radix_scatter<true>, dim3(ntiles), dim3(kBlock), 0, s, ka, va, kb, vb, n,
-                         shift, ntiles, hist, wa, wb);
-    else
-      hipLaunchKernelGGL(k_radix_scatter<false>, dim3(ntiles), dim3(kBlock), 0, s, ka, va, kb, vb,
-                         n, shift, ntiles, hist, nullptr, nullptr);
-    ILC_HIP(hipGetLastError());
-    std::swap(ka, kb);
-    std::swap(va, vb);
-    std::swap(wa, wb);
-  }
-  if (ka != keys) {
-    ILC_HIP(hipMemcpyAsync(keys, ka, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-    ILC_HIP(hipMemcpyAsync(vals, va, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-    if (vals2)
-      ILC_HIP(hipMemcpyAsync(vals2, wa, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-  }
+void radix_shape(uint64_t n, radix_chain* c) {
+  c->counting = n <= kCountingRows;
+  c->tile_log = c->counting ? 10 : 12;
+  c->ntiles = static_cast<uint32_t>((n + (uint64_t(1) << c->tile_log) - 1) >> c->tile_log);
+  c->small = c->ntiles <= kSmallTiles;
+  c->tile_bits = 0;
+  while ((1u << c->tile_bits) < c->ntiles && c->tile_bits < 31) ++c->tile_bits;
 }
+uint64_t radix_hist_words(const radix_chain& c, int passes) {
+  if (c.counting) return uint64_t(passes) * c.ntiles * 256;
+  return 256 * uint64_t(c.ntiles) + scan_temp_words(256 * uint64_t(c.ntiles));
+}
+constexpr int kMaxPasses = 8;
 }  // namespace
 
-void launch_radix_sort(uint32_t* keys, uint32_t* vals, uint32_t n, int key_bits, uint32_t* temp,
-                       hipStream_t s) {
-  radix_sort_impl(keys, vals, nullptr, n, key_bits, temp, s);
+uint64_t radix_chain_words(uint64_t n) {
+  radix_chain c{};
+  radix_shape(n, &c);
+  return 4 * n + radix_hist_words(c, kMaxPasses);
 }
 
-uint64_t radix2_temp_words(uint64_t n) { return radix_temp_words(n) + n; }
+radix_chain plan_radix_chain(uint32_t* b_out, uint32_t* v_out, uint64_t n, int bits_a, int bits_b,
+                             uint32_t* temp) {
+  radix_chain c{};
+  c.n = static_cast<uint32_t>(n);
+  c.pa = (bits_a + 7) / 8;
+  c.pb = (bits_b + 7) / 8;
+  ILC_REQUIRE(c.pa + c.pb <= kMaxPasses, "radix chain of %d passes", c.pa + c.pb);
+  radix_shape(n, &c);
+  c.b[0] = b_out;
+  c.v[0] = v_out;
+  c.a[0] = temp;
+  c.a[1] = temp + n;
+  c.b[1] = temp + 2 * n;
+  c.v[1] = temp + 3 * n;
+  c.hist = temp + 4 * n;
+  c.hist_words = radix_hist_words(c, c.pa + c.pb);
+  c.in = (c.pa + c.pb) & 1;
+  return c;
+}
 
-void launch_radix_sort2(uint32_t* keys, uint32_t* vals, uint32_t* vals2, uint32_t n, int key_bits,
-                        uint32_t* temp, hipStream_t s) {
-  ILC_REQUIRE(vals2 != nullptr, "second value array");
-  radix_sort_impl(keys, vals, vals2, n, key_bits, temp, s);
+std::pair<uint32_t*, uint64_t> radix_chain_zero(const radix_chain& c) {
+  return {c.hist, c.counting ? c.hist_words : 0};
+}
+
+void launch_radix_chain(const radix_chain& c, bool iota, bool counted, hipStream_t s) {
+  if (!c.n) return;
+  const int passes = c.pa + c.pb;
+  int cur = c.in;
+  const dim3 grid{c.ntiles}, block{kBlock};
+  auto key_of = [&](int p, int set) { return p < c.pa ? c.a[set] : c.b[set]; };
+  auto shift_of = [&](int p) { return 8 * (p < c.pa ? p : p - c.pa); };
+  if (c.counting && !counted && passes) {
+    hipLaunchKernelGGL(k_radix_hist<4>, grid, block, 0, s, key_of(0, cur), c.n, 0, c.ntiles,
+                       c.hist, 1);
+    ILC_HIP(hipGetLastError());
+  }
+  for (int p = 0; p < passes; ++p) {
+    const bool in_a = p < c.pa, last_a = p + 1 == c.pa, last = p + 1 == passes;
+    const uint32_t* kin = key_of(p, cur);
+    const uint32_t* vin = p == 0 && iota ? nullptr : c.v[cur];
+    const uint32_t* bin = in_a ? c.b[cur] : nullptr;
+    // the first keys are not read again once their passes are done
+    uint32_t* kout = last_a ? nullptr : key_of(p, cur ^ 1);
+    uint32_t* vout = c.v[cur ^ 1];
+    uint32_t* bout = in_a ? c.b[cur ^ 1] : nullptr;
+    const int shift = shift_of(p);
+    uint32_t* hist = c.counting ? c.hist + uint64_t(p) * c.ntiles * 256 : c.hist;
+    radix_next next{nullptr, 0, 0, c.tile_bits};
+    if (c.counting) {
+      if (!last) {
+        next.hist = c.hist + uint64_t(p + 1) * c.ntiles * 256;
+        next.shift = shift_of(p + 1);
+        next.of_second = last_a ? 1 : 0;
+      }
+    } else {
+      hipLaunchKernelGGL(k_radix_hist<16>, grid, block, 0, s, kin, c.n, shift, c.ntiles, hist,
+                         c.small ? 1 : 0);
+      ILC_HIP(hipGetLastError());
+    }
+    if (!c.small) {
+      launch_exclusive_scan(hist, hist, uint64_t(256) * c.ntiles,
+                            hist + 256 * uint64_t(c.ntiles), s);
+    }
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, kin, vin, bin, kout, vout, bout, c.n, shift,
+                         c.ntiles, hist, next);
+    };
+    if (!c.small)
+      in_a ? go(k_radix_scatter<16, true, false>) : go(k_radix_scatter<16, false, false>);
+    else if (c.counting)
+      in_a ? go(k_radix_scatter<4, true, true>) : go(k_radix_scatter<4, false, true>);
+    else
+      in_a ? go(k_radix_scatter<16, true, true>) : go(k_radix_scatter<16, false, true>);
+    ILC_HIP(hipGetLastError());
+    cur ^= 1;
+  }
 }
 
 void launch_build_soa(const float4* p4, const float* h, const uint32_t* perm,
@@ -668,29 +877,15 @@ void launch_build_soa(const float4* p4, const float* h, const uint32_t* perm,
   ILC_HIP(hipGetLastError());
 }
 
-void launch_h_order(const float* h, uint32_t* key, uint32_t* perm, uint32_t n, uint32_t* horder,
-                    uint32_t* temp, hipStream_t s) {
-  if (n <= 1) return;
-  uint32_t* hk = horder;
-  uint32_t* hv = horder + n;
-  hipLaunchKernelGGL(k_h_order_keys, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, h, perm, n,
-                     hk, hv);
-  ILC_HIP(hipGetLastError());
-  launch_radix_sort(hk, hv, n, 16, temp, s);
-  hipLaunchKernelGGL(k_permute_pairs, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, hv, key,
-                     perm, n, temp, temp + n);
-  ILC_HIP(hipGetLastError());
-  ILC_HIP(hipMemcpyAsync(key, temp, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-  ILC_HIP(hipMemcpyAsync(perm, temp + n, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-}
-
 void launch_reference_perm(const uint32_t* key, const uint32_t* perm, uint32_t n, int key_bits,
                            uint32_t* out_perm, uint32_t* by_index, uint32_t* temp, hipStream_t s) {
   if (!n) return;
+  const radix_chain c = plan_radix_chain(by_index, out_perm, n, 0, std::max(key_bits, 1), temp);
+  launch_zero({radix_chain_zero(c)}, s);
   hipLaunchKernelGGL(k_keys_by_index, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, key, perm,
-                     n, by_index, out_perm);
+                     n, c.b[c.in]);
   ILC_HIP(hipGetLastError());
-  launch_radix_sort(by_index, out_perm, n, key_bits, temp, s);
+  launch_radix_chain(c, true, false, s);
 }
 
 void launch_export_cells(const uint32_t* start, const uint32_t* maxh_bits, uint32_t ncells,

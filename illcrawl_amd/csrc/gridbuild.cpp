@@ -109,13 +109,44 @@ grid_params plan_grid(const bbox_result& bb, uint64_t n, uint64_t target, int mo
   return g;
 }
 
-void enqueue_grid_build(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
-                        uint64_t n, const grid_params& g, int32_t kz0, float max_h, int kernel,
-                        uint32_t* err, hipStream_t s) {
+radix_chain plan_grid_sort(grid_store& gs, grid_scratch& sc, uint64_t n, const grid_params& g) {
+  const uint64_t ncells = g.ncells();
+  gs.ready = false;
   gs.key.ensure(n);
   gs.perm.ensure(n);
-  launch_keys(p4, uint32_t(n), g, gs.key.p, gs.perm.p, err, s);
-  enqueue_grid_from_keys(gs, sc, p4, h, n, g, kz0, max_h, kernel, s);
+  sc.temp.ensure(std::max(radix_chain_words(n), scan_temp_words(ncells + 1)));
+  return plan_radix_chain(gs.key.p, gs.perm.p, n, kHKeyBits, key_bits_for(ncells - 1), sc.temp.p);
+}
+
+namespace {
+// per-cell arrays cleared with the sort's counts, in one launch
+void zero_cells(grid_store& gs, grid_scratch& sc, const radix_chain& c, const grid_params& g,
+                uint32_t* err, hipStream_t s) {
+  const uint64_t ncells = g.ncells();
+  sc.counts.ensure(ncells + 1);
+  gs.maxh_bits.ensure(ncells);
+  launch_zero({radix_chain_zero(c),
+               {sc.counts.p, ncells + 1},
+               {gs.maxh_bits.p, ncells},
+               {err, err ? 1 : 0}},
+              s);
+}
+}  // namespace
+
+void enqueue_grid_build(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
+                        uint64_t n, const grid_params& g, int32_t kz0, float max_h, int kernel,
+                        uint32_t* err, bool clear_err, hipStream_t s) {
+  const radix_chain c = plan_grid_sort(gs, sc, n, g);
+  zero_cells(gs, sc, c, g, clear_err ? err : nullptr, s);
+  launch_keys(p4, h, uint32_t(n), g, c, err, s);
+  enqueue_grid_sorted(gs, sc, c, true, p4, h, n, g, kz0, max_h, kernel, s);
+}
+
+void enqueue_grid_from_keys(grid_store& gs, grid_scratch& sc, const radix_chain& c,
+                            const float4* p4, const float* h, uint64_t n, const grid_params& g,
+                            int32_t kz0, float max_h, int kernel, hipStream_t s) {
+  zero_cells(gs, sc, c, g, nullptr, s);
+  enqueue_grid_sorted(gs, sc, c, false, p4, h, n, g, kz0, max_h, kernel, s);
 }
 
 void enqueue_grid_maxh(grid_store& gs, const float4* p4, const float* h, uint64_t n,
@@ -138,24 +169,14 @@ void enqueue_grid_maxh(grid_store& gs, const float4* p4, const float* h, uint64_
   gs.ready = true;
 }
 
-void enqueue_grid_from_keys(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
-                            uint64_t n, const grid_params& g, int32_t kz0, float max_h,
-                            int kernel, hipStream_t s) {
+void enqueue_grid_sorted(grid_store& gs, grid_scratch& sc, const radix_chain& c, bool counted,
+                         const float4* p4, const float* h, uint64_t n, const grid_params& g,
+                         int32_t kz0, float max_h, int kernel, hipStream_t s) {
   const uint64_t ncells = g.ncells();
-  gs.ready = false;
-  gs.key.ensure(n);
-  gs.perm.ensure(n);
   gs.start.ensure(ncells + 1);
-  gs.maxh_bits.ensure(ncells);
   gs.part.ensure(n);
   gs.hs.ensure(n);
-  sc.counts.ensure(ncells + 1);
-  sc.temp.ensure(std::max(radix_temp_words(n), scan_temp_words(ncells + 1)));
-  sc.horder.ensure(2 * std::max<uint64_t>(n, 1));
-  launch_h_order(h, gs.key.p, gs.perm.p, uint32_t(n), sc.horder.p, sc.temp.p, s);
-  launch_radix_sort(gs.key.p, gs.perm.p, uint32_t(n), key_bits_for(ncells - 1), sc.temp.p, s);
-  launch_fill_u32(sc.counts.p, 0u, ncells + 1, s);
-  launch_fill_u32(gs.maxh_bits.p, 0u, ncells, s);
+  launch_radix_chain(c, true, counted, s);
   gs.volumetric = false;
   launch_build_soa(p4, h, gs.perm.p, gs.key.p, uint32_t(n), kernel_norm(kernel),
                    kernel != ILC_KERNEL_CUBIC, gs.part.p,
@@ -182,8 +203,8 @@ void enqueue_volumetric_grid(grid_store& gs, grid_scratch& sc, const float4* p4,
   gs.lv_w.ensure(n);
   gs.lv_cell.ensure(n);
   gs.lv_meta.ensure(kLvMetaWords);
-  sc.lv_tmp.ensure(11 * std::max<uint64_t>(n, 1));
-  sc.temp.ensure(radix_temp_words(n));
+  sc.lv_tmp.ensure(10 * std::max<uint64_t>(n, 1));
+  sc.temp.ensure(radix_chain_words(n));
   level_cell_sizes(g, max_h, gs.lv_cs);
   level_planes(g, gs.lv_cs, gs.lv_poff);
   gs.lv_pdir.ensure(gs.lv_poff[kLevels3]);

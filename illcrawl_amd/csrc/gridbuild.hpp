@@ -45,7 +45,7 @@ struct grid_store {
 
 // Scratch shared by successive builds on one stream.
 struct grid_scratch {
-  dbuf<uint32_t> temp, counts, flags, horder, lv_tmp;
+  dbuf<uint32_t> temp, counts, flags, lv_tmp;
   dbuf<float> bbox_partial;
   dbuf<bbox_result> bbox_dev;
 };
@@ -57,10 +57,19 @@ grid_params plan_grid(const bbox_result& bb, uint64_t n, uint64_t target, int mo
 
 // Enqueue keys, stable sort, sorted SoA, per-cell counts / max h and cell
 // offsets for n float4 particles p4 with smoothing lengths h.  Out-of-grid
-// keys are counted into err (device uint32, not cleared here).
+// keys are counted into err (device uint32, cleared here with clear_err).
 void enqueue_grid_build(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
                         uint64_t n, const grid_params& g, int32_t kz0, float max_h, int kernel,
-                        uint32_t* err, hipStream_t s);
+                        uint32_t* err, bool clear_err, hipStream_t s);
+
+// The sort of a grid's n particles: by cell key (b), biggest h first (a).
+radix_chain plan_grid_sort(grid_store& gs, grid_scratch& sc, uint64_t n, const grid_params& g);
+
+// The rest of a build, once the keys of plan_grid_sort's chain are written
+// (counted: with their first digit).
+void enqueue_grid_sorted(grid_store& gs, grid_scratch& sc, const radix_chain& c, bool counted,
+                         const float4* p4, const float* h, uint64_t n, const grid_params& g,
+                         int32_t kz0, float max_h, int kernel, hipStream_t s);
 
 // Only the per-cell max h (gs.maxh_bits) and the grid parameters of n
 // particles, no sorted arrays (gs.part, key, hs, perm and start stay as they
@@ -69,11 +78,11 @@ void enqueue_grid_maxh(grid_store& gs, const float4* p4, const float* h, uint64_
                        const grid_params& g, int32_t kz0, float max_h, uint32_t* err,
                        hipStream_t s);
 
-// The same from keys already in gs.key (cell keys) and gs.perm (indices into
-// p4 / h), n of them, in the order the within-cell order must follow.
-void enqueue_grid_from_keys(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
-                            uint64_t n, const grid_params& g, int32_t kz0, float max_h,
-                            int kernel, hipStream_t s);
+// The same from keys already written to the chain of plan_grid_sort, in the
+// order the within-cell order must follow (row j is p4[j], h[j]).
+void enqueue_grid_from_keys(grid_store& gs, grid_scratch& sc, const radix_chain& c,
+                            const float4* p4, const float* h, uint64_t n, const grid_params& g,
+                            int32_t kz0, float max_h, int kernel, hipStream_t s);
 
 // The grid of the 3-D smoothing: the reference grid's parameters and per-cell
 // max h, and the level index (coef = w K / h^3) the volumetric gather

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
+#include <utility>
 
 #include "common.hpp"
 
@@ -11,10 +13,43 @@ namespace ilc {
 
 // ---- grid.hip
 void launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
+// zeroes up to four arrays (pointer, words) in one launch
+void launch_zero(std::initializer_list<std::pair<uint32_t*, uint64_t>> regions, hipStream_t s);
 void launch_bbox(const float4* p4, const float* h, uint64_t n, float* partial, int nparts,
-                 uint32_t* bad, bbox_result* out, hipStream_t s);
-void launch_keys(const float4* p4, uint32_t n, const grid_params& g, uint32_t* keys,
-                 uint32_t* vals, uint32_t* err, hipStream_t s);
+                 bbox_result* out, hipStream_t s);
+
+// A stable sort of n rows by key b, rows of equal b by key a (ascending),
+// rows of equal keys in input order: LSD radix passes over a's digits, then
+// over b's, the row's value (and b, while a's digits are sorted) moving
+// along.  The producer writes the keys to a[in] and b[in] (and the values to
+// v[in], unless they are the input positions); the sorted b and values end
+// in b_out and v_out.  bits_a may be 0 (no first key).
+struct radix_chain {
+  uint32_t n;
+  int pa, pb;        // passes over a and over b
+  uint32_t *a[2], *b[2], *v[2];
+  int in;
+  uint32_t* hist;    // digit counts
+  uint64_t hist_words;
+  uint32_t ntiles;
+  int tile_log, tile_bits;
+  bool small;        // the passes add up the tiles' counts themselves
+  bool counting;     // and count the next pass's digits (the producer the first's)
+};
+uint64_t radix_chain_words(uint64_t n);
+// temp: radix_chain_words(n)
+radix_chain plan_radix_chain(uint32_t* b_out, uint32_t* v_out, uint64_t n, int bits_a, int bits_b,
+                             uint32_t* temp);
+// what has to be zeroed before the keys are written (and counted)
+std::pair<uint32_t*, uint64_t> radix_chain_zero(const radix_chain& c);
+// iota: the values are the input positions; counted: the producer counted
+// the first digit into hist when c.counting
+void launch_radix_chain(const radix_chain& c, bool iota, bool counted, hipStream_t s);
+// Cell keys (b) and descending-h keys (a) of n particles, the first digit
+// counted.
+void launch_keys(const float4* p4, const float* h, uint32_t n, const grid_params& g,
+                 const radix_chain& c, uint32_t* err, hipStream_t s);
+constexpr int kHKeyBits = 16;
 // Per-cell max h (float bits, atomic max; maxh_bits cleared by the caller)
 // of n particles, without sorting them; out-of-grid particles count in err.
 void launch_cell_maxh(const float4* p4, const float* h, uint32_t n, const grid_params& g,
@@ -22,32 +57,19 @@ void launch_cell_maxh(const float4* p4, const float* h, uint32_t n, const grid_p
 uint64_t scan_temp_words(uint64_t n);
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* temp,
                            hipStream_t s);
-uint64_t radix_temp_words(uint64_t n);
-void launch_radix_sort(uint32_t* keys, uint32_t* vals, uint32_t n, int key_bits, uint32_t* temp,
-                       hipStream_t s);
-// The same sort with a second value array moved alongside; temp holds
-// radix2_temp_words(n).
-uint64_t radix2_temp_words(uint64_t n);
-void launch_radix_sort2(uint32_t* keys, uint32_t* vals, uint32_t* vals2, uint32_t n, int key_bits,
-                        uint32_t* temp, hipStream_t s);
 // coef = w norm / h^2 (pow04: coef^0.4, the projected quartic's form); h
 // NULL: each particle's h is the z of its p4
 void launch_build_soa(const float4* p4, const float* h, const uint32_t* perm,
                       const uint32_t* skeys, uint32_t n, float norm, bool pow04, float4* part,
                       float* hs, uint32_t* count, uint32_t* maxh_bits, hipStream_t s,
                       const float2* zc_in = nullptr, float2* zc_out = nullptr);
-// Reorder (key, perm) pairs, n of them, by descending h[perm] (top 16 bits,
-// stable); horder holds 2n words, temp radix_temp_words(n).
-void launch_h_order(const float* h, uint32_t* key, uint32_t* perm, uint32_t n, uint32_t* horder,
-                    uint32_t* temp, hipStream_t s);
 // The reference's within-cell order (stable by input index) of a grid whose
-// sorted keys and perm are given; by_index holds n words.
+// sorted keys and perm are given; by_index holds n words, temp
+// radix_chain_words(n).
 void launch_reference_perm(const uint32_t* key, const uint32_t* perm, uint32_t n, int key_bits,
                            uint32_t* out_perm, uint32_t* by_index, uint32_t* temp, hipStream_t s);
 void launch_export_cells(const uint32_t* start, const uint32_t* maxh_bits, uint32_t ncells,
                          int32_t* cells2, float* maxh, hipStream_t s);
-void launch_bbox_final(const float* partial, int nparts, const uint32_t* bad, bbox_result* out,
-                       hipStream_t s);
 
 // ---- batch.hip
 // Per-view particle pass: quantity functor (mass or bolometric X-ray), camera
@@ -119,7 +141,8 @@ struct view_build_desc {
   grid_params g;  // the view's grid (cell keys of the scatter)
 };
 // Bounding boxes of every view in one read of the snapshot: out[v] as
-// launch_view_bbox would give it (every view's vp.scale must be 1).  partial
+// launch_bbox would give it from the view's projected particles (every view's
+// vp.scale must be 1).  partial
 // holds multi_bbox_parts(n) * 8 * nv floats, bad nv words.  one_group: every
 // view is a slab of one slab group (the same x', y' projection bit for bit,
 // the same quantity).
@@ -160,7 +183,7 @@ void launch_particle_xray(const particle_soa& ps, const gaunt_table& gt, float* 
 // The kept particles of every listed view, in input order, at the global
 // positions offs[v * ntiles + t] (exclusive scan of the multi-window counts):
 // projected float4 (x', y', h, w with the depth mask), the descending-h sort
-// key (as launch_h_order) and the row index as its value, the global cell key
+// key (launch_keys), the global cell key
 // (the view's first cell cbase[v] + the cell key in the view's grid, so that
 // it orders rows by view, then cell) and the snapshot index.
 // wx: launch_particle_xray.  maxh_bits: the per-cell max h of the shared cell
@@ -169,19 +192,16 @@ void launch_particle_xray(const particle_soa& ps, const gaunt_table& gt, float* 
 void launch_multi_window_scatter(const particle_soa& ps, const float* wx,
                                  const view_build_desc* vd_dev, const int32_t* views_dev,
                                  int nviews, const uint32_t* offs, float4* p4c, uint32_t* hqkey,
-                                 uint32_t* hqval, uint32_t* gkey, uint32_t* orig, uint32_t* err,
+                                 uint32_t* gkey, uint32_t* orig, uint32_t* err,
                                  const uint32_t* cbase, uint32_t* maxh_bits, float2* zc,
                                  const slab_stack& stack, hipStream_t s);
-// out[i] = src[idx[i]]
-void launch_gather_u32(const uint32_t* src, const uint32_t* idx, uint32_t n, uint32_t* out,
-                       hipStream_t s);
 // lkey[i] = gkey[i] - cbase[v], v the view whose cells hold gkey[i] (cbase:
 // the nv views' first cells, rising strictly)
 void launch_local_keys(const uint32_t* gkey, const uint32_t* cbase, int nv, uint32_t n,
                        uint32_t* lkey, hipStream_t s);
 void launch_window_scatter(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
                            const window_f& win, const uint32_t* offsets, const grid_params& g,
-                           float4* p4c, float* hc, uint32_t* keys, uint32_t* vals, uint32_t* orig,
+                           float4* p4c, float* hc, uint32_t* keys, uint32_t* hkeys, uint32_t* orig,
                            uint32_t* err, hipStream_t s);
 // one view's adjoint (sorted order, projected frame) into snapshot gradients;
 // orig (may be NULL): the snapshot index of each grid input row
@@ -189,9 +209,6 @@ void launch_scatter_grads(const uint32_t* perm, const uint32_t* orig, uint32_t n
                           const float* gw, const float* gh, const float* gx, const float* gy,
                           const float* pos3, const view_proj& vp, float* out_w, float* out_h,
                           float* out_pos3, hipStream_t s);
-int view_bbox_parts(uint64_t n);
-void launch_view_bbox(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
-                      float* partial, uint32_t* bad, bbox_result* out, hipStream_t s);
 void launch_view_project(const particle_soa& ps, const view_proj& vp, const gaunt_table& gt,
                          float4* out, hipStream_t s);
 
@@ -303,7 +320,7 @@ struct queue_segs {
 };
 // The persistent gather's items reordered inside every queue: tiles with the
 // most particles under them first (stable inside a cost class).  keys, idx:
-// n words each; radix_temp: radix_temp_words(n); out: n items.
+// n words each; radix_temp: radix_chain_words(n); out: n items.
 void launch_order_items(const view_desc* views, const uint2* items, const queue_segs& segs,
                         uint32_t n, const sum_shape& ts, uint32_t* keys, uint32_t* idx,
                         uint32_t* radix_temp, uint2* out, hipStream_t s);
@@ -353,8 +370,8 @@ void level_planes(const grid_params& g, const float cs[kLevels3], uint32_t poff[
 // Builds the level index of particles p4 (x, y, z, w) with smoothing lengths
 // h on grid g, and the grid's per-cell max h (maxh_bits, ncells words); err
 // counts particles outside the grid.  norm: the kernel's 3-D normalisation
-// (coef = w norm / h^3).  tmp: 11 n words, 16-byte aligned; radix_temp:
-// radix_temp_words(n).
+// (coef = w norm / h^3).  tmp: 10 n words, 16-byte aligned; radix_temp:
+// radix_chain_words(n).
 void launch_volumetric_index(const float4* p4, const float* h, uint32_t n, const grid_params& g,
                              float max_h, float norm, const level_view& lv,
                              unsigned long long* key, float4* pos, float* w, int2* cell,

@@ -545,7 +545,6 @@ __global__ __launch_bounds__(kBlock) void k_vol_keys(const float4* __restrict__ 
                                                       float4* __restrict__ rec,
                                                       uint32_t* __restrict__ lo,
                                                       uint32_t* __restrict__ hi,
-                                                      uint32_t* __restrict__ idx,
                                                       uint32_t* __restrict__ meta,
                                                       uint32_t* __restrict__ maxh_bits,
                                                       uint32_t* __restrict__ err) {
@@ -593,7 +592,6 @@ __global__ __launch_bounds__(kBlock) void k_vol_keys(const float4* __restrict__ 
                                             fine_of(q.z, g.minc[2], cs));
       lo[i] = uint32_t(k);
       hi[i] = uint32_t(k >> 32);
-      idx[i] = i;
       atomicAdd(&cnt[l], 1u);
       if (__float_as_uint(h) > mh[l]) atomicMax(&mh[l], __float_as_uint(h));
     }
@@ -683,23 +681,20 @@ void launch_volumetric_index(const float4* p4, const float* h, uint32_t n, const
                              unsigned long long* key, float4* pos, float* w, int2* cell,
                              uint32_t* meta, uint32_t* pdir, uint32_t* maxh_bits, uint32_t* err,
                              uint32_t* tmp, uint32_t* radix_temp, hipStream_t s) {
-  launch_fill_u32(meta, 0u, kLvMetaWords, s);
-  launch_fill_u32(maxh_bits, 0u, g.ncells(), s);
+  // the sort by the 62-bit level key: its high word (30 bits), then its low
+  uint32_t* hi_out = tmp + 8 * uint64_t(n);
+  uint32_t* idx = hi_out + n;
+  const radix_chain c = plan_radix_chain(hi_out, idx, n, 32, 30, radix_temp);
+  launch_zero({radix_chain_zero(c), {meta, kLvMetaWords}, {maxh_bits, g.ncells()}, {err, 1}}, s);
   if (n) {
     float4* rec = reinterpret_cast<float4*>(tmp);
-    uint32_t* lo = tmp + 8 * uint64_t(n);
-    uint32_t* hi = lo + n;
-    uint32_t* idx = hi + n;
     // a capped grid: each workgroup adds its level counts to the same few
     // global words once
     const uint32_t nb = std::min<uint32_t>((n + kBlock - 1) / kBlock, 2048u);
-    hipLaunchKernelGGL(k_vol_keys, dim3(nb), dim3(kBlock), 0, s, p4, h, n, g, max_h, lv, rec, lo,
-                       hi, idx, meta, maxh_bits, err);
+    hipLaunchKernelGGL(k_vol_keys, dim3(nb), dim3(kBlock), 0, s, p4, h, n, g, max_h, lv, rec,
+                       c.a[c.in], c.b[c.in], meta, maxh_bits, err);
     ILC_HIP(hipGetLastError());
-    // (hi, lo) order by two stable sorts: low word, then high word
-    launch_radix_sort(lo, idx, n, 32, radix_temp, s);
-    launch_gather_u32(hi, idx, n, lo, s);
-    launch_radix_sort(lo, idx, n, 30, radix_temp, s);
+    launch_radix_chain(c, true, false, s);
     const dim3 grid{(n + kBlock - 1) / kBlock}, block{kBlock};
     hipLaunchKernelGGL(k_vol_soa, grid, block, 0, s, rec, n, g, max_h, norm, lv, idx, key, pos, w,
                        cell);

@@ -166,3 +166,26 @@ def test_adjoint_tiles(B, orc, nx, ny):
         e = float(np.max(np.abs(a - r)) / np.max(np.abs(r)))
         print(f"adjoint {nx}x{ny} dL/d{name}: {e:.2e}", flush=True)
         assert e < 1e-4
+
+
+@pytest.mark.parametrize("n", [1, 2, 1024, 1025, 131072, 131073, 1 << 20, (1 << 20) + 1])
+def test_grid_sort_at_the_tile_and_path_limits(B, orc, n):
+    """The sort's tiles of 1024 and 4096 rows and its three paths (digit counts
+    by the passes, by a count launch, scanned): cells, ranges, max h and order
+    equal the oracle's bit for bit, and every cell holds its particles by
+    descending h (top 16 bits), ties in input order."""
+    rng = np.random.default_rng(n)
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :2] = rng.normal(0, 30.0, (n, 2))
+    p4[:, 3] = 1.0
+    h = np.exp(rng.uniform(-8, 8, n)).astype(np.float32)
+    h[rng.random(n) < 0.5] = 1.5
+    b = B.ProjectiveSmoothingGrid(target_particles_per_cell=40)
+    b.init_backend(n)
+    b.setup_projected_particles(p4, h)
+    g = orc.Grid(p4, h, target=40)
+    cells, maxh, perm = b.export_grid()
+    assert np.array_equal(cells.cpu().numpy(), g.cells)
+    assert np.array_equal(maxh.cpu().numpy(), g.maxh_cell)
+    assert np.array_equal(perm.cpu().numpy().astype(np.uint32), g.perm)
+    print(f"sort n={n}: {g.ncells} cells", flush=True)

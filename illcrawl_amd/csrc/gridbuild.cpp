@@ -46,13 +46,16 @@ level_view grid_store::levels() const {
 }
 
 void level_cell_sizes(const grid_params& g, float max_h, float cs[kLevels3]) {
-  // level L: h <= H_L = max_h 2^(L - 23), cells of H_L, at least the grid
-  // extent over the 19-bit fine coordinate range
+  // level L: h <= H_L = max_h 2^(L - 23), cells of 0.7 H_L, at least the grid
+  // extent over the 19-bit fine coordinate range.  Smaller cells fit the
+  // support spheres better, larger ones make fewer key rows: 8 slices of
+  // 2048^2 through 16M particles 6.21 ms with H_L, 6.00 with 0.7, 6.35 with
+  // 0.5; a 250 x 180 slice through 60k 293, 285 and 271 us.
   double ext = 0.0;
   for (int a = 0; a < 3; ++a) ext = std::max(ext, double(g.nc[a]) * double(g.cs[a]));
   const float floor_cs = static_cast<float>(ext / 524000.0);
   for (int l = 0; l < kLevels3; ++l) {
-    const float hl = std::ldexp(max_h, l - (kLevels3 - 1));
+    const float hl = 0.7f * std::ldexp(max_h, l - (kLevels3 - 1));
     cs[l] = std::max(hl, floor_cs);
     if (!(cs[l] > 0.0f) || !std::isfinite(cs[l])) cs[l] = std::max(max_h, 1e-30f);
   }

@@ -345,7 +345,7 @@ void launch_retrieve(const double* acc, uint64_t n, float scale, float* out, hip
 //
 // The level index of a volumetric grid: particles binned by h into levels
 // (level L holds h <= max_h 2^(L - 23)), each level sorted by a fine cell key
-// (L << 57 | z << 38 | y << 19 | x) of cell size cs[L] ~ the level's h.
+// (L << 57 | z << 38 | y << 19 | x) of cell size cs[L], 0.7 of the level's h.
 constexpr int kLevels3 = 24;
 constexpr uint32_t kFineMax3 = (1u << 19) - 1;
 // meta layout: count[24], max h bits[24], start[25]

@@ -1,0 +1,87 @@
+"""The volumetric gather at the edges of its tiles, against the FP64 sums.
+
+The bound is the rounding of the FP32 pair w/h^3 s^2, s = 1 - r^2/h^2, with
+u = 2^-24: r^2 is off by 5 u (a subtraction counts twice, three roundings), 1/h^2
+by 2 u and s, one rounding more, by 7 u in all; the coefficient by 6 u, the
+square and the product by 2 u, a partial sum of 32 pairs by 32 u.  So a point
+may be off by u sum(coef (14 s + 40 s^2)), and by (7 u)^2 coef for a pair at
+the edge of its support."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+U = 2.0 ** -24
+SUM_TOL = 1e-6
+
+
+def bound(p4, h, pts):
+    coef = 1.05 * p4[:, 3].astype(np.float64) / h.astype(np.float64) ** 3
+    xyz, h2 = p4[:, :3].astype(np.float64), h.astype(np.float64) ** 2
+    out = np.empty(pts.shape[0])
+    for i in range(0, pts.shape[0], 2048):
+        q = pts[i:i + 2048, :3].astype(np.float64)
+        r2 = sum((q[:, a, None] - xyz[None, :, a]) ** 2 for a in range(3))
+        s = np.maximum(1.0 - r2 / h2, 0.0)
+        out[i:i + 2048] = ((14 * U * s + 40 * U * s * s + (7 * U) ** 2) * coef).sum(1)
+    return out
+
+
+@pytest.fixture(scope="module")
+def B():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from illcrawl_amd import backend
+    return backend
+
+
+@pytest.fixture(scope="module")
+def orc():
+    import oracle
+    return oracle
+
+
+@pytest.mark.parametrize("nx,ny,step,bend,hmax", [
+    (1, 1, 1.0, 0.0, 30.0),        # one point
+    (1, 300, 0.2, 0.0, 20.0),      # one column: no plane through the tile's corners
+    (300, 1, 0.2, 0.0, 20.0),      # one row
+    (17, 9, 1.0, 0.0, 60.0),       # a column and a row beyond a tile; cover particles
+    (16, 16, 0.0, 0.0, 20.0),      # every point the same
+    (40, 33, 1.0, 6.0, 12.0),      # points off their tile's plane
+    (23, 48, 1.0, 1e9, 12.0),      # rows of far-apart slices in one tile
+    (1024, 513, 0.1, 0.0, 12.0),   # 16 x 16 tiles, the last row of points alone
+    (1000, 525, 0.1, 0.7, 12.0),   # the same, off their plane and a partial column
+])
+@pytest.mark.parametrize("mode,kernel", [("reference", "quartic_ref"), ("exact", "quartic")])
+def test_tiles_match_the_sums(B, orc, nx, ny, step, bend, hmax, mode, kernel):
+    rng = np.random.default_rng(nx * 1000 + ny)
+    n = 3000
+    p4 = np.concatenate([rng.uniform(0, 100, (n, 3)), rng.lognormal(0, 0.3, (n, 1))],
+                        1).astype(np.float32)
+    h = np.exp(rng.uniform(np.log(1.0), np.log(hmax), n)).astype(np.float32)
+    u, v = np.meshgrid((np.arange(nx) - 0.5 * nx) * step, (np.arange(ny) - 0.5 * ny) * step)
+    z = 30.0 * (np.arange(ny)[:, None] % 3 - 1.0) + 0 * u if bend > 1e8 else bend * np.sin(u + v)
+    pts = np.zeros((nx * ny, 4), np.float32)
+    pts[:, 0] = (50.0 + u).ravel()
+    pts[:, 1] = (50.0 + 0.8 * v - 0.6 * z).ravel()
+    pts[:, 2] = (50.0 + 0.6 * v + 0.8 * z).ravel()
+    # past 20000 points, some of them (stride coprime to the tile side, both ends)
+    some = np.unique(np.r_[0:pts.shape[0]:max(1, pts.shape[0] // 20000) | 1, pts.shape[0] - 1])
+    print(f"tiles {nx} x {ny} step {step} bend {bend} {mode}", flush=True)
+    g = B.GridSmoothing(mode=mode, kernel=kernel, target_particles_per_cell=64)
+    g.init_backend(n)
+    g.setup_particles(p4, [h])
+    g.setup_evaluation_points(pts, layout_nx=nx)
+    g.run()
+    got = g.retrieve_results_f64().cpu().numpy()[some]
+    if mode == "reference":
+        ref = orc.Grid(p4, h, target=64).smooth3d_ref(pts[some], form=1)
+    else:
+        ref = orc.smooth3d_exact(p4, h, pts[some])
+    assert ref.max() > 0
+    off = np.abs(got - ref) / bound(p4, h, pts[some])
+    print(f"  largest error {off.max():.3f} of its bound", flush=True)
+    assert off.max() < 1.0
+    assert abs(got.sum() - ref.sum()) < SUM_TOL * ref.sum()

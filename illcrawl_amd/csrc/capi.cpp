@@ -183,7 +183,7 @@ ilc_status ilc_psg_setup_projected_particles(ilc_psg* h, const float* particles4
     grid_scratch& sc = h->scratch;
     // 1. bounding box (the host scan of particle_grid.cpp:43-67)
     const int nparts = static_cast<int>(std::min<uint64_t>(1024, (n + kBlock - 1) / kBlock));
-    sc.bbox_partial.ensure(size_t(nparts) * 8);
+    sc.bbox_partial.ensure(size_t(nparts) * kBboxWords);
     sc.bbox_dev.ensure(1);
     sc.flags.ensure(2);
     launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.bbox_dev.p, s);
@@ -488,7 +488,7 @@ ilc_status ilc_grid3d_setup_particles(ilc_grid3d* g3, const float* particles4_de
     grid_scratch& sc = h->scratch;
     // bounding box (particle_grid.cpp:43-67), then the grid parameters
     const int nparts = static_cast<int>(std::min<uint64_t>(1024, (n + kBlock - 1) / kBlock));
-    sc.bbox_partial.ensure(size_t(nparts) * 8);
+    sc.bbox_partial.ensure(size_t(nparts) * kBboxWords);
     sc.bbox_dev.ensure(1);
     sc.flags.ensure(2);
     launch_bbox(p4, hsml_dev, n, sc.bbox_partial.p, nparts, sc.bbox_dev.p, s);
@@ -503,7 +503,8 @@ ilc_status ilc_grid3d_setup_particles(ilc_grid3d* g3, const float* particles4_de
     // the masked list packs a cell's x and y into 16 bits each
     if (h->mode == ILC_MODE_REFERENCE && (g.nc[0] > 65536 || g.nc[1] > 65536))
       fail(ILC_ERANGE, "grid of %d x %d cells in x, y (at most 65536 each)", g.nc[0], g.nc[1]);
-    enqueue_volumetric_grid(h->grid, sc, p4, hsml_dev, n, g, bb.max_h, h->kernel, sc.flags.p, s);
+    enqueue_volumetric_grid(h->grid, sc, p4, hsml_dev, n, g, bb.max_h, bb.min_h, h->kernel,
+                            sc.flags.p, s);
     ILC_HIP(hipMemcpyAsync(h->flags_host, sc.flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     ILC_HIP(hipStreamSynchronize(s));
     if (h->flags_host[0]) {

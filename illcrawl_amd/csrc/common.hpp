@@ -77,6 +77,7 @@ struct bbox_result {
   float mx[3];
   float max_h;
   uint32_t bad;  // count of particles with non-finite coordinates or h <= 0 / NaN
+  float min_h;   // of launch_bbox only
 };
 
 // Host part of the grid construction, in double exactly as the reference.

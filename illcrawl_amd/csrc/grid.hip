@@ -13,7 +13,9 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "cellmax.hpp"
 #include "kernels.hpp"
+#include "wave.hpp"
 
 namespace ilc {
 
@@ -67,14 +69,14 @@ __global__ __launch_bounds__(kBlock) void k_zero(fill_regions r) {
     for (uint64_t i = i0; i < r.n[k]; i += step) r.p[k][i] = 0u;
 }
 
-// Per-block min/max of x, y, z, max h, and a count of invalid particles.
+// Per-block min/max of x, y, z, max h, max -h, and a count of invalid particles.
 // Non-finite coordinates or w, and h that is not a positive normal float
 // whose square stays finite, are invalid.
 __global__ __launch_bounds__(kBlock) void k_bbox_partial(const float4* __restrict__ p4,
                                                           const float* __restrict__ h,
                                                           uint64_t n, float* __restrict__ part) {
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  float mh = 0.0f;
+  float mh = 0.0f, lh = -INFINITY;
   uint32_t nbad = 0;
   for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n;
        i += uint64_t(gridDim.x) * kBlock) {
@@ -90,56 +92,59 @@ __global__ __launch_bounds__(kBlock) void k_bbox_partial(const float4* __restric
     mn[1] = fminf(mn[1], q.y); mx[1] = fmaxf(mx[1], q.y);
     mn[2] = fminf(mn[2], q.z); mx[2] = fmaxf(mx[2], q.z);
     mh = fmaxf(mh, hh);
+    lh = fmaxf(lh, -hh);
   }
-  __shared__ float red[4][7];
+  __shared__ float red[4][8];
   __shared__ uint32_t redb[4];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  float v[7] = {wave_min(mn[0]), wave_min(mn[1]), wave_min(mn[2]), wave_max(mx[0]),
-                wave_max(mx[1]), wave_max(mx[2]), wave_max(mh)};
+  float v[8] = {wave_min(mn[0]), wave_min(mn[1]), wave_min(mn[2]), wave_max(mx[0]),
+                wave_max(mx[1]), wave_max(mx[2]), wave_max(mh), wave_max(lh)};
   uint32_t b = wave_sum(nbad);
   if (lane == 0) {
-    for (int k = 0; k < 7; ++k) red[wave][k] = v[k];
+    for (int k = 0; k < 8; ++k) red[wave][k] = v[k];
     redb[wave] = b;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    float r[7];
-    for (int k = 0; k < 7; ++k) r[k] = red[0][k];
+    float r[8];
+    for (int k = 0; k < 8; ++k) r[k] = red[0][k];
     uint32_t bb = redb[0];
     for (int w = 1; w < 4; ++w) {
       for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], red[w][k]);
-      for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], red[w][k]);
+      for (int k = 3; k < 8; ++k) r[k] = fmaxf(r[k], red[w][k]);
       bb += redb[w];
     }
-    for (int k = 0; k < 7; ++k) part[blockIdx.x * 8 + k] = r[k];
-    part[blockIdx.x * 8 + 7] = __uint_as_float(bb);
+    float* out = part + blockIdx.x * kBboxWords;
+    for (int k = 0; k < 8; ++k) out[k] = r[k];
+    out[8] = __uint_as_float(bb);
   }
 }
 
 __global__ __launch_bounds__(kBlock) void k_bbox_final(const float* __restrict__ part, int nparts,
                                                         bbox_result* __restrict__ out) {
-  __shared__ float red[4][7];
+  __shared__ float red[4][8];
   __shared__ uint32_t redb[4];
-  float r[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0f};
+  float r[8] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0f, -INFINITY};
   uint32_t bad = 0;
   for (int i = threadIdx.x; i < nparts; i += kBlock) {
-    for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], part[i * 8 + k]);
-    for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], part[i * 8 + k]);
-    bad += __float_as_uint(part[i * 8 + 7]);
+    const float* p = part + i * kBboxWords;
+    for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], p[k]);
+    for (int k = 3; k < 8; ++k) r[k] = fmaxf(r[k], p[k]);
+    bad += __float_as_uint(p[8]);
   }
   for (int k = 0; k < 3; ++k) r[k] = wave_min(r[k]);
-  for (int k = 3; k < 7; ++k) r[k] = wave_max(r[k]);
+  for (int k = 3; k < 8; ++k) r[k] = wave_max(r[k]);
   bad = wave_sum(bad);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) {
-    for (int k = 0; k < 7; ++k) red[wave][k] = r[k];
+    for (int k = 0; k < 8; ++k) red[wave][k] = r[k];
     redb[wave] = bad;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 4; ++w) {
       for (int k = 0; k < 3; ++k) r[k] = fminf(r[k], red[w][k]);
-      for (int k = 3; k < 7; ++k) r[k] = fmaxf(r[k], red[w][k]);
+      for (int k = 3; k < 8; ++k) r[k] = fmaxf(r[k], red[w][k]);
       bad += redb[w];
     }
     for (int k = 0; k < 3; ++k) {
@@ -147,18 +152,9 @@ __global__ __launch_bounds__(kBlock) void k_bbox_final(const float* __restrict__
       out->mx[k] = r[3 + k];
     }
     out->max_h = r[6];
+    out->min_h = -r[7];
     out->bad = bad;
   }
-}
-
-// Cell indices exactly as grid3d_get_cell_indices (particle_grid.cl:45-53):
-// floor((p - min) / size) in FP32 with a correctly rounded division.
-__device__ inline int32_t floor_to_int(float f) {
-  const float fl = floorf(f);
-  if (!(fl == fl)) return 0;
-  if (fl >= 2147483647.0f) return INT32_MAX;
-  if (fl <= -2147483648.0f) return INT32_MIN;
-  return static_cast<int32_t>(fl);
 }
 
 // exclusive scan over the workgroup (kBlock threads)
@@ -650,36 +646,37 @@ inline uint32_t blocks_for(uint64_t n, uint64_t per) {
 }
 
 // Per-cell max h without the sort (a slab group's shared grid: its views
-// read only the per-cell max h and the grid parameters): each particle's cell
-// as k_keys computes it, and an atomic max that is only issued when the cell's
-// current max is smaller (clustered cells hold many particles).  maxh_bits
-// starts at 0; particles outside the grid count in err.
+// read only the per-cell max h and the grid parameters) of particles i0 .. i1 - 1:
+// each particle's cell as k_keys computes it.  maxh_bits starts at 0;
+// particles outside the grid count in err.
 __global__ __launch_bounds__(kBlock) void k_cell_maxh(const float4* __restrict__ p4,
-                                                      const float* __restrict__ h, uint32_t n,
-                                                      grid_params g,
+                                                      const float* __restrict__ h, uint32_t i0,
+                                                      uint32_t i1, grid_params g,
                                                       uint32_t* __restrict__ maxh_bits,
                                                       uint32_t* __restrict__ err) {
 #pragma clang fp contract(off)
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const float4 q = p4[i];
-  const float c[3] = {q.x, q.y, q.z};
-  int32_t idx[3];
-  bool ok = true;
-  for (int a = 0; a < 3; ++a) {
-    const float d = c[a] - g.minc[a];
-    idx[a] = floor_to_int(d / g.cs[a]);
-    ok = ok && idx[a] >= 0 && idx[a] < g.nc[a];
+  __shared__ unsigned long long slots[kMaxSlots];
+  const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
+  bool ok = i < i1;
+  uint32_t key = 0, hb = 0;
+  if (ok) {
+    const float4 q = p4[i];
+    const float c[3] = {q.x, q.y, q.z};
+    int32_t idx[3];
+    for (int a = 0; a < 3; ++a) {
+      const float d = c[a] - g.minc[a];
+      idx[a] = floor_to_int(d / g.cs[a]);
+      ok = ok && idx[a] >= 0 && idx[a] < g.nc[a];
+    }
+    if (ok) {
+      key = uint32_t(idx[0]) + uint32_t(idx[1]) * uint32_t(g.nc[0]) +
+            uint32_t(idx[2]) * uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
+      hb = __float_as_uint(h[i]);
+    } else {
+      atomicAdd(err, 1u);
+    }
   }
-  if (!ok) {
-    atomicAdd(err, 1u);
-    return;
-  }
-  const uint32_t key = uint32_t(idx[0]) + uint32_t(idx[1]) * uint32_t(g.nc[0]) +
-                       uint32_t(idx[2]) * uint32_t(g.nc[0]) * uint32_t(g.nc[1]);
-  const uint32_t hb = __float_as_uint(h[i]);
-  uint32_t* m = maxh_bits + key;
-  if (hb > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m, hb);
+  block_raise_max(maxh_bits, key, hb, ok, slots);
 }
 
 }  // namespace
@@ -721,9 +718,11 @@ void launch_bbox(const float4* p4, const float* h, uint64_t n, float* partial, i
 void launch_cell_maxh(const float4* p4, const float* h, uint32_t n, const grid_params& g,
                       uint32_t* maxh_bits, uint32_t* err, hipStream_t s) {
   if (!n) return;
-  hipLaunchKernelGGL(k_cell_maxh, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, p4, h, n, g,
-                     maxh_bits, err);
-  ILC_HIP(hipGetLastError());
+  for_ranges(n, [&](uint32_t i0, uint32_t i1) {
+    hipLaunchKernelGGL(k_cell_maxh, dim3(blocks_for(i1 - i0, kBlock)), dim3(kBlock), 0, s, p4, h,
+                       i0, i1, g, maxh_bits, err);
+    ILC_HIP(hipGetLastError());
+  });
 }
 
 void launch_keys(const float4* p4, const float* h, uint32_t n, const grid_params& g,

@@ -40,6 +40,7 @@ level_view grid_store::levels() const {
   lv.cell = lv_cell.p;
   lv.meta = lv_meta.p;
   lv.pdir = lv_pdir.p;
+  lv.bits = lv_bits;
   for (int l = 0; l <= kLevels3; ++l) lv.poff[l] = lv_poff[l];
   for (int l = 0; l < kLevels3; ++l) lv.cs[l] = lv_cs[l];
   return lv;
@@ -61,14 +62,41 @@ void level_cell_sizes(const grid_params& g, float max_h, float cs[kLevels3]) {
   }
 }
 
-void level_planes(const grid_params& g, const float cs[kLevels3], uint32_t poff[kLevels3 + 1]) {
-  // a particle's fine z is at most floor(extent / cs) (one more by rounding)
-  const double ext = double(g.nc[2]) * double(g.cs[2]);
+namespace {
+// a particle's fine coordinate is at most floor(extent / cs) (one more by
+// rounding)
+uint32_t fine_count(const grid_params& g, int a, float cs) {
+  const double ext = double(g.nc[a]) * double(g.cs[a]);
+  return static_cast<uint32_t>(
+      std::min(std::floor(ext / double(cs)) + 2.0, double(kFineMax3) + 1.0));
+}
+}  // namespace
+
+level_key level_key_for(const grid_params& g, const float cs[kLevels3], float max_h, float min_h) {
+  level_key k;
+  // the level of the smallest h, as the device takes it (the exponent of the
+  // FP32 quotient)
+  const float r = max_h / min_h;
+  const int e = r >= 1.0f && std::isfinite(r) ? std::ilogb(r) : kLevels3;
+  k.lmin = std::min(std::max(kLevels3 - 1 - e, 0), kLevels3 - 1);
+  int b = 0;
+  for (int a = 0; a < 3; ++a) {
+    const int bits = key_bits_for(fine_count(g, a, cs[k.lmin]) - 1);
+    k.fmax[a] = (1u << bits) - 1u;
+    k.shift[a] = b;
+    b += bits;
+  }
+  k.shift[3] = b;
+  k.bits = b + key_bits_for(uint64_t(kLevels3 - 1 - k.lmin));
+  return k;
+}
+
+void level_planes(const grid_params& g, const float cs[kLevels3], int lmin,
+                  uint32_t poff[kLevels3 + 1]) {
   uint32_t off = 0;
   for (int l = 0; l < kLevels3; ++l) {
     poff[l] = off;
-    const double np = std::floor(ext / double(cs[l])) + 2.0;
-    off += static_cast<uint32_t>(std::min(np, double(kFineMax3) + 1.0)) + 1u;
+    if (l >= lmin) off += fine_count(g, 2, cs[l]) + 1u;
   }
   poff[kLevels3] = off;
 }
@@ -197,8 +225,8 @@ void enqueue_grid_sorted(grid_store& gs, grid_scratch& sc, const radix_chain& c,
 }
 
 void enqueue_volumetric_grid(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
-                             uint64_t n, const grid_params& g, float max_h, int kernel,
-                             uint32_t* err, hipStream_t s) {
+                             uint64_t n, const grid_params& g, float max_h, float min_h,
+                             int kernel, uint32_t* err, hipStream_t s) {
   gs.ready = false;
   gs.maxh_bits.ensure(g.ncells());
   gs.lv_key.ensure(n);
@@ -209,7 +237,8 @@ void enqueue_volumetric_grid(grid_store& gs, grid_scratch& sc, const float4* p4,
   sc.lv_tmp.ensure(10 * std::max<uint64_t>(n, 1));
   sc.temp.ensure(radix_chain_words(n));
   level_cell_sizes(g, max_h, gs.lv_cs);
-  level_planes(g, gs.lv_cs, gs.lv_poff);
+  gs.lv_bits = level_key_for(g, gs.lv_cs, max_h, min_h);
+  level_planes(g, gs.lv_cs, gs.lv_bits.lmin, gs.lv_poff);
   gs.lv_pdir.ensure(gs.lv_poff[kLevels3]);
   launch_volumetric_index(p4, h, uint32_t(n), g, max_h, kernel_norm_3d(kernel), gs.levels(),
                           gs.lv_key.p, gs.lv_pos.p, gs.lv_w.p, gs.lv_cell.p, gs.lv_meta.p,

@@ -27,6 +27,7 @@ struct grid_store {
   dbuf<int2> lv_cell;
   dbuf<uint32_t> lv_meta;
   dbuf<uint32_t> lv_pdir;
+  level_key lv_bits;
   uint32_t lv_poff[kLevels3 + 1] = {};
   float lv_cs[kLevels3] = {};
   grid_params gp{};
@@ -88,8 +89,8 @@ void enqueue_grid_from_keys(grid_store& gs, grid_scratch& sc, const radix_chain&
 // max h, and the level index (coef = w K / h^3) the volumetric gather
 // searches.  Out-of-grid particles are counted into err.
 void enqueue_volumetric_grid(grid_store& gs, grid_scratch& sc, const float4* p4, const float* h,
-                             uint64_t n, const grid_params& g, float max_h, int kernel,
-                             uint32_t* err, hipStream_t s);
+                             uint64_t n, const grid_params& g, float max_h, float min_h,
+                             int kernel, uint32_t* err, hipStream_t s);
 
 float kernel_norm(int kernel);
 // the 3-D quartic's normalisation: the reference's 1.04445f (ILC_KERNEL_QUARTIC_REF)

@@ -15,6 +15,7 @@ namespace ilc {
 void launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 // zeroes up to four arrays (pointer, words) in one launch
 void launch_zero(std::initializer_list<std::pair<uint32_t*, uint64_t>> regions, hipStream_t s);
+constexpr int kBboxWords = 9;  // words of partial per part
 void launch_bbox(const float4* p4, const float* h, uint64_t n, float* partial, int nparts,
                  bbox_result* out, hipStream_t s);
 
@@ -345,11 +346,19 @@ void launch_retrieve(const double* acc, uint64_t n, float scale, float* out, hip
 //
 // The level index of a volumetric grid: particles binned by h into levels
 // (level L holds h <= max_h 2^(L - 23)), each level sorted by a fine cell key
-// (L << 57 | z << 38 | y << 19 | x) of cell size cs[L], 0.7 of the level's h.
+// (level, z, y, x) of cell size cs[L], 0.7 of the level's h.
 constexpr int kLevels3 = 24;
 constexpr uint32_t kFineMax3 = (1u << 19) - 1;
-// meta layout: count[24], max h bits[24], start[25]
-constexpr int kLvMetaWords = 3 * kLevels3 + 1;
+// The key's bits, as many as the finest level in use needs: x | y << shift[1]
+// | z << shift[2] | (L - lmin) << shift[3].
+struct level_key {
+  int lmin = 0;  // level of the smallest h
+  int shift[4] = {};
+  uint32_t fmax[3] = {};  // the largest coordinate the bits hold
+  int bits = 0;
+};
+// meta: the levels' starts
+constexpr int kLvMetaWords = kLevels3 + 1;
 struct level_view {
   const unsigned long long* key;  // sorted fine keys
   const float4* pos;              // (x, y, z, 1/h^2)
@@ -359,14 +368,18 @@ struct level_view {
   // plane directory: pdir[poff[L] + z] = first index of level L whose fine z
   // is >= z, for z = 0 .. poff[L + 1] - poff[L] - 1 (the last: the level's end)
   const uint32_t* pdir;
+  level_key bits;
   uint32_t poff[kLevels3 + 1];
   float cs[kLevels3];
 };
 // Fine cell sizes of the levels for a grid of that extent and max h (host).
 void level_cell_sizes(const grid_params& g, float max_h, float cs[kLevels3]);
-// Offsets of the levels' plane directories (host): every fine z a particle
-// can have, plus one entry for the level's end.
-void level_planes(const grid_params& g, const float cs[kLevels3], uint32_t poff[kLevels3 + 1]);
+// The key's bits for h in [min_h, max_h] (host).
+level_key level_key_for(const grid_params& g, const float cs[kLevels3], float max_h, float min_h);
+// Offsets of the plane directories of levels lmin and up (host): every fine z
+// a particle can have, plus one entry for the level's end.
+void level_planes(const grid_params& g, const float cs[kLevels3], int lmin,
+                  uint32_t poff[kLevels3 + 1]);
 // Builds the level index of particles p4 (x, y, z, w) with smoothing lengths
 // h on grid g, and the grid's per-cell max h (maxh_bits, ncells words); err
 // counts particles outside the grid.  norm: the kernel's 3-D normalisation

@@ -49,6 +49,7 @@
 
 #include <algorithm>
 
+#include "cellmax.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "wave.hpp"
@@ -126,26 +127,28 @@ struct smem3 {
 };
 
 // level of a particle: the smallest L with h <= max_h 2^(L - 23) (by the
-// exponent of max_h / h; any assignment is correct, the gather searches
-// each level with its particles' largest h)
-__device__ inline int level_of(float h, float max_h) {
+// exponent of max_h / h; a level may also hold smaller h: the gather
+// searches it with its largest possible h)
+__device__ inline int level_of(float h, float max_h, int lmin) {
   const float r = max_h / h;
   const int e = int((__float_as_uint(r) >> 23) & 0xffu) - 127;
-  return min(max(kLevels3 - 1 - e, 0), kLevels3 - 1);
+  return min(max(kLevels3 - 1 - e, lmin), kLevels3 - 1);
 }
 
-// fine cell coordinate, clamped to [0, kFineMax3]; monotone in x
-__device__ inline uint32_t fine_of(float x, float mn, float cs) {
+// fine cell coordinate, clamped to [0, fmax]; monotone in x
+__device__ inline uint32_t fine_of(float x, float mn, float cs, uint32_t fmax) {
 #pragma clang fp contract(off)
   const float f = floorf((x - mn) / cs);
   if (!(f >= 0.0f)) return 0u;
-  if (f >= float(kFineMax3)) return kFineMax3;
+  if (f >= float(fmax)) return fmax;
   return uint32_t(f);
 }
 
-__device__ inline unsigned long long fine_key(int l, uint32_t fx, uint32_t fy, uint32_t fz) {
-  return (static_cast<unsigned long long>(l) << 57) | (static_cast<unsigned long long>(fz) << 38) |
-         (static_cast<unsigned long long>(fy) << 19) | static_cast<unsigned long long>(fx);
+__device__ inline unsigned long long fine_key(const level_key& b, int l, uint32_t fx, uint32_t fy,
+                                              uint32_t fz) {
+  using u64 = unsigned long long;
+  return (u64(l - b.lmin) << b.shift[3]) | (u64(fz) << b.shift[2]) | (u64(fy) << b.shift[1]) |
+         u64(fx);
 }
 
 // first index in [a, b) whose key is >= k (keys sorted ascending)
@@ -521,15 +524,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       int f0[3] = {0, 0, 0}, f1[3] = {-1, -1, -1};
       int mode = 0;
       float R = 0.0f;
-      if (lv.meta[l] != 0u) {
+      if (lv.meta[l + 1] != lv.meta[l]) {
         // every particle whose support reaches a point of the tile lies within
         // the level's largest h of the tile box; the margin covers rounding
-        R = __uint_as_float(lv.meta[kLevels3 + l]);
+        R = ldexpf(g.max_h, l - (kLevels3 - 1));
         const float c = lv.cs[l];
         for (int a = 0; a < 3; ++a) {
           const float m = R + 1e-5f * (fabsf(bmin[a]) + fabsf(bmax[a]) + R + fabsf(g.minc[a]));
-          f0[a] = int(fine_of(bmin[a] - m, g.minc[a], c));
-          f1[a] = int(fine_of(bmax[a] + m, g.minc[a], c));
+          f0[a] = int(fine_of(bmin[a] - m, g.minc[a], c, lv.bits.fmax[a]));
+          f1[a] = int(fine_of(bmax[a] + m, g.minc[a], c, lv.bits.fmax[a]));
         }
         const uint32_t ny = uint32_t(f1[1] - f0[1] + 1), nz = uint32_t(f1[2] - f0[2] + 1);
         if (ny <= kRowCap3 && nz <= kRowCap3 && ny * nz <= kRowCap3) {
@@ -549,10 +552,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       }
       sm.lv_mode[l] = mode;
       sm.lv_r[l] = R;
-      sm.lv_s[l] = lv.meta[2 * kLevels3 + l];
+      sm.lv_s[l] = lv.meta[l];
       sm.lv_p[l] = lv.poff[l];
       if (l == kLevels3 - 1) {
-        sm.lv_s[kLevels3] = lv.meta[3 * kLevels3];
+        sm.lv_s[kLevels3] = lv.meta[kLevels3];
         sm.lv_p[kLevels3] = lv.poff[kLevels3];
       }
     }
@@ -594,7 +597,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
         // box, and of the points' extent along the plane's normal.  A fine
         // cell's particles lie inside it up to a few ulps of the
         // coordinates; the outermost cells also hold what was clamped.
-        if (y0 > 0 && y0 < int(kFineMax3) && z0 > 0 && z0 < int(kFineMax3)) {
+        if (y0 > 0 && y0 < int(lv.bits.fmax[1]) && z0 > 0 && z0 < int(lv.bits.fmax[2])) {
           const float c = lv.cs[l];
           const float mg = 1e-3f * c + 5e-7f * at + 1e-5f * hd;
           const float R = sm.lv_r[l] * 1.00002f + mg;
@@ -623,8 +626,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
             }
           }
           if (xa <= xb) {
-            x0 = max(x0, int(fine_of(tc[0] + xa - mg, g.minc[0], c)));
-            x1 = min(x1, int(fine_of(tc[0] + xb + mg, g.minc[0], c)));
+            x0 = max(x0, int(fine_of(tc[0] + xa - mg, g.minc[0], c, lv.bits.fmax[0])));
+            x1 = min(x1, int(fine_of(tc[0] + xb + mg, g.minc[0], c, lv.bits.fmax[0])));
           } else {
             x1 = x0 - 1;
           }
@@ -633,8 +636,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
         z0 = z1 = f0[2] + int(k);
       }
       if (x0 <= x1) {
-        const unsigned long long klo = fine_key(l, uint32_t(x0), uint32_t(y0), uint32_t(z0));
-        const unsigned long long khi = fine_key(l, uint32_t(x1), uint32_t(y1), uint32_t(z1));
+        const auto klo = fine_key(lv.bits, l, uint32_t(x0), uint32_t(y0), uint32_t(z0));
+        const auto khi = fine_key(lv.bits, l, uint32_t(x1), uint32_t(y1), uint32_t(z1));
         // the keys of planes z0 .. z1 from the plane directory (a plane
         // beyond the level's last holds no particle)
         const uint32_t planes = sm.lv_p[l + 1] - sm.lv_p[l] - 1;
@@ -800,76 +803,90 @@ __device__ inline bool cell_index_3d(const float4& q, const grid_params& g, int3
   return ok;
 }
 
-// per particle: the reference cell's max h (atomic max), the level and its
-// fine key (lo, hi words), the level counts and max h, and a 32-byte record
-// (x, y, z, h | w, cell xy, cell z, 0) in input order, so that the sorted
-// gather reads one line per particle instead of one from p4 and one from h
+__device__ inline unsigned long long particle_key(const float4& q, float h, float max_h,
+                                                  const grid_params& g, const level_view& lv,
+                                                  const float* scs) {
+  const int l = level_of(h, max_h, lv.bits.lmin);
+  const float cs = scs[l];
+  return fine_key(lv.bits, l, fine_of(q.x, g.minc[0], cs, lv.bits.fmax[0]),
+                  fine_of(q.y, g.minc[1], cs, lv.bits.fmax[1]),
+                  fine_of(q.z, g.minc[2], cs, lv.bits.fmax[2]));
+}
+
+// particles i0 .. i1 - 1: the reference cell's max h, the particle's fine key
+// (low and high words; the low one alone in hi when the key has no more than 32
+// bits), and a 32-byte record (x, y, z, h | w, cell xy, cell z, 0) in input
+// order, so that the sorted gather reads one line per particle instead of one
+// from p4 and one from h.  Bound by memory (60 bytes a particle): 16M particles
+// 471 us, 867 with the levels counted here on a few common words and the
+// maxima read past the caches.
 __global__ __launch_bounds__(kBlock) void k_vol_keys(const float4* __restrict__ p4,
-                                                      const float* __restrict__ hsml, uint32_t n,
-                                                      grid_params g, float max_h, level_view lv,
-                                                      float4* __restrict__ rec,
+                                                      const float* __restrict__ hsml, uint32_t i0,
+                                                      uint32_t i1, grid_params g, float max_h,
+                                                      level_view lv, float4* __restrict__ rec,
                                                       uint32_t* __restrict__ lo,
                                                       uint32_t* __restrict__ hi,
-                                                      uint32_t* __restrict__ meta,
                                                       uint32_t* __restrict__ maxh_bits,
                                                       uint32_t* __restrict__ err) {
-  __shared__ uint32_t cnt[kLevels3], mh[kLevels3];
   __shared__ float scs[kLevels3];
   __shared__ float4 srec[2 * kBlock];
+  __shared__ unsigned long long slots[kMaxSlots];
   const int t = threadIdx.x;
   if (t == 0) {
 #pragma unroll
-    for (int l = 0; l < kLevels3; ++l) {
-      cnt[l] = 0u;
-      mh[l] = 0u;
-      scs[l] = lv.cs[l];
-    }
+    for (int l = 0; l < kLevels3; ++l) scs[l] = lv.cs[l];
   }
   __syncthreads();
   const uint32_t nx = uint32_t(g.nc[0]), nxy = nx * uint32_t(g.nc[1]);
-  // the whole block runs every round (the records go out through LDS)
-  for (uint64_t base = uint64_t(blockIdx.x) * kBlock; base < n;
-       base += uint64_t(gridDim.x) * kBlock) {
-    const uint32_t i = uint32_t(base) + uint32_t(t);
-    if (i < n) {
-      const float4 q = p4[i];
-      const float h = hsml[i];
-      int32_t c[3];
-      if (cell_index_3d(q, g, c)) {
-        // clustered cells hold millions of particles: read the running max
-        // first and go to the atomic unit only with a larger h (a stale read
-        // is never above the true max, so nothing is skipped wrongly)
-        uint32_t* m = &maxh_bits[uint32_t(c[0]) + uint32_t(c[1]) * nx + uint32_t(c[2]) * nxy];
-        const uint32_t hb = __float_as_uint(h);
-        if (hb > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-          atomicMax(m, hb);
-      } else {
-        atomicAdd(err, 1u);
-        c[0] = c[1] = c[2] = 0;
-      }
-      srec[2 * t] = make_float4(q.x, q.y, q.z, h);
-      srec[2 * t + 1] = make_float4(q.w, __uint_as_float(uint32_t(c[0]) | (uint32_t(c[1]) << 16)),
-                                    __uint_as_float(uint32_t(c[2])), 0.0f);
-      const int l = level_of(h, max_h);
-      const float cs = scs[l];
-      const unsigned long long k = fine_key(l, fine_of(q.x, g.minc[0], cs),
-                                            fine_of(q.y, g.minc[1], cs),
-                                            fine_of(q.z, g.minc[2], cs));
+  const uint32_t base = i0 + blockIdx.x * kBlock, i = base + uint32_t(t);
+  bool ok = false;
+  uint32_t cell = 0, hb = 0;
+  if (i < i1) {
+    const float4 q = p4[i];
+    const float h = hsml[i];
+    int32_t c[3];
+    ok = cell_index_3d(q, g, c);
+    if (ok) {
+      cell = uint32_t(c[0]) + uint32_t(c[1]) * nx + uint32_t(c[2]) * nxy;
+      hb = __float_as_uint(h);
+    } else {
+      atomicAdd(err, 1u);
+      c[0] = c[1] = c[2] = 0;
+    }
+    srec[2 * t] = make_float4(q.x, q.y, q.z, h);
+    srec[2 * t + 1] = make_float4(q.w, __uint_as_float(uint32_t(c[0]) | (uint32_t(c[1]) << 16)),
+                                  __uint_as_float(uint32_t(c[2])), 0.0f);
+    const auto k = particle_key(q, h, max_h, g, lv, scs);
+    if (lv.bits.bits > 32) {
       lo[i] = uint32_t(k);
       hi[i] = uint32_t(k >> 32);
-      atomicAdd(&cnt[l], 1u);
-      if (__float_as_uint(h) > mh[l]) atomicMax(&mh[l], __float_as_uint(h));
+    } else {
+      hi[i] = uint32_t(k);
     }
-    __syncthreads();
-    // the round's records are contiguous: whole 16-byte words per lane
-    const uint32_t m2 = 2u * uint32_t(min(uint64_t(kBlock), uint64_t(n) - base));
-    for (uint32_t k = uint32_t(t); k < m2; k += kBlock) rec[2 * base + k] = srec[k];
-    __syncthreads();
   }
-  if (t < kLevels3 && cnt[t]) {
-    atomicAdd(&meta[t], cnt[t]);
-    atomicMax(&meta[kLevels3 + t], mh[t]);
+  block_raise_max(maxh_bits, cell, hb, ok, slots);  // has a barrier
+  // the block's records are contiguous: whole 16-byte words per lane
+  const uint32_t m2 = 2u * min(uint32_t(kBlock), i1 - base);
+  for (uint32_t k = uint32_t(t); k < m2; k += kBlock) rec[2 * uint64_t(base) + k] = srec[k];
+}
+
+// lower_bound_u64 in few rounds of 15 independent loads: a search has nothing
+// else to wait for (60k particles: 20 us a launch with dependent loads, 8 now)
+__device__ inline uint32_t wide_lower_bound_u64(const unsigned long long* __restrict__ key,
+                                                uint32_t a, uint32_t b, unsigned long long k) {
+  while (b - a >= 16u) {
+    const uint32_t step = (b - a) >> 4;  // a + 15 step < b
+    uint32_t below = 0;
+#pragma unroll
+    for (uint32_t j = 1; j <= 15; ++j) below += key[a + j * step] < k ? 1u : 0u;
+    if (below < 15u) b = a + (below + 1) * step;
+    if (below) a += below * step + 1;
   }
+  uint32_t below = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < 15; ++j)
+    if (a + j < b) below += key[a + j] < k ? 1u : 0u;
+  return a + below;
 }
 
 // pdir[poff[L] + z]: first index of level L whose fine z is >= z; the last
@@ -880,7 +897,7 @@ __global__ __launch_bounds__(kBlock) void k_lv_planes(level_view lv, uint32_t* _
 #pragma unroll
     for (int l = 0; l <= kLevels3; ++l) {
       sp[l] = lv.poff[l];
-      ss[l] = lv.meta[2 * kLevels3 + l];
+      ss[l] = lv.meta[l];
     }
   }
   __syncthreads();
@@ -891,22 +908,13 @@ __global__ __launch_bounds__(kBlock) void k_lv_planes(level_view lv, uint32_t* _
   const uint32_t z = e - sp[l];
   const uint32_t last = sp[l + 1] - sp[l] - 1;
   pdir[e] = z == last ? ss[l + 1]
-                      : lower_bound_u64(lv.key, ss[l], ss[l + 1],
-                                        fine_key(l, 0u, 0u, min(z, kFineMax3)));
-}
-
-__global__ void k_lv_starts(uint32_t* __restrict__ meta) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  uint32_t s = 0;
-  for (int l = 0; l < kLevels3; ++l) {
-    meta[2 * kLevels3 + l] = s;
-    s += meta[l];
-  }
-  meta[3 * kLevels3] = s;
+                      : wide_lower_bound_u64(lv.key, ss[l], ss[l + 1],
+                                             fine_key(lv.bits, l, 0u, 0u,
+                                                      min(z, lv.bits.fmax[2])));
 }
 
 // the level-ordered arrays: key, (x, y, z, 1/h^2), coef = w norm / h^3 and
-// the reference cell
+// the reference cell; and the levels' starts, where the level changes
 __global__ __launch_bounds__(kBlock) void k_vol_soa(const float4* __restrict__ rec, uint32_t n,
                                                      grid_params g, float max_h, float norm,
                                                      level_view lv,
@@ -914,7 +922,8 @@ __global__ __launch_bounds__(kBlock) void k_vol_soa(const float4* __restrict__ r
                                                      unsigned long long* __restrict__ key,
                                                      float4* __restrict__ pos,
                                                      float* __restrict__ w,
-                                                     int2* __restrict__ cell) {
+                                                     int2* __restrict__ cell,
+                                                     uint32_t* __restrict__ start) {
   __shared__ float scs[kLevels3];
   const int t = threadIdx.x;
   if (t == 0) {
@@ -925,14 +934,21 @@ __global__ __launch_bounds__(kBlock) void k_vol_soa(const float4* __restrict__ r
   const uint32_t j = blockIdx.x * kBlock + uint32_t(t);
   if (j >= n) return;
   const uint32_t i = order[j];
+  // the particle before the wave's first one
+  float h0 = 0.0f;
+  if ((t & 63) == 0 && j > 0) h0 = rec[2 * uint64_t(order[j - 1])].w;
   const float4 r0 = rec[2 * uint64_t(i)];
   const float4 r1 = rec[2 * uint64_t(i) + 1];
   const float4 q = make_float4(r0.x, r0.y, r0.z, r1.x);
   const float h = r0.w;
-  const int l = level_of(h, max_h);
-  const float cs = scs[l];
-  key[j] = fine_key(l, fine_of(q.x, g.minc[0], cs), fine_of(q.y, g.minc[1], cs),
-                    fine_of(q.z, g.minc[2], cs));
+  const auto k = particle_key(q, h, max_h, g, lv, scs);
+  key[j] = k;
+  const int l = lv.bits.lmin + int(k >> lv.bits.shift[3]);
+  int before = __shfl_up(l, 1, 64);
+  if ((t & 63) == 0) before = j > 0 ? level_of(h0, max_h, lv.bits.lmin) : -1;
+  for (int m = before + 1; m <= l; ++m) start[m] = j;
+  if (j == n - 1)
+    for (int m = l + 1; m <= kLevels3; ++m) start[m] = n;
   const float ih2 = 1.0f / (h * h);
   pos[j] = make_float4(q.x, q.y, q.z, ih2);
   w[j] = q.w * (norm * (ih2 / h));
@@ -946,27 +962,26 @@ void launch_volumetric_index(const float4* p4, const float* h, uint32_t n, const
                              unsigned long long* key, float4* pos, float* w, int2* cell,
                              uint32_t* meta, uint32_t* pdir, uint32_t* maxh_bits, uint32_t* err,
                              uint32_t* tmp, uint32_t* radix_temp, hipStream_t s) {
-  // the sort by the 62-bit level key: its high word (30 bits), then its low
+  // the sort by the level key: its low word, if it has two, then its high
   uint32_t* hi_out = tmp + 8 * uint64_t(n);
   uint32_t* idx = hi_out + n;
-  const radix_chain c = plan_radix_chain(hi_out, idx, n, 32, 30, radix_temp);
+  const int bits = std::max(lv.bits.bits, 1);
+  const radix_chain c = plan_radix_chain(hi_out, idx, n, bits > 32 ? 32 : 0,
+                                         bits > 32 ? bits - 32 : bits, radix_temp);
   launch_zero({radix_chain_zero(c), {meta, kLvMetaWords}, {maxh_bits, g.ncells()}, {err, 1}}, s);
   if (n) {
     float4* rec = reinterpret_cast<float4*>(tmp);
-    // a capped grid: each workgroup adds its level counts to the same few
-    // global words once
-    const uint32_t nb = std::min<uint32_t>((n + kBlock - 1) / kBlock, 2048u);
-    hipLaunchKernelGGL(k_vol_keys, dim3(nb), dim3(kBlock), 0, s, p4, h, n, g, max_h, lv, rec,
-                       c.a[c.in], c.b[c.in], meta, maxh_bits, err);
-    ILC_HIP(hipGetLastError());
-    launch_radix_chain(c, true, false, s);
     const dim3 grid{(n + kBlock - 1) / kBlock}, block{kBlock};
+    for_ranges(n, [&](uint32_t i0, uint32_t i1) {
+      hipLaunchKernelGGL(k_vol_keys, dim3((i1 - i0 + kBlock - 1) / kBlock), block, 0, s, p4, h, i0,
+                         i1, g, max_h, lv, rec, c.a[c.in], c.b[c.in], maxh_bits, err);
+      ILC_HIP(hipGetLastError());
+    });
+    launch_radix_chain(c, true, false, s);
     hipLaunchKernelGGL(k_vol_soa, grid, block, 0, s, rec, n, g, max_h, norm, lv, idx, key, pos, w,
-                       cell);
+                       cell, meta);
     ILC_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_lv_starts, dim3(1), dim3(64), 0, s, meta);
-  ILC_HIP(hipGetLastError());
   // the directory searches the sorted keys (lv.key is key, lv.meta is meta)
   const uint32_t nd = lv.poff[kLevels3];
   ILC_REQUIRE(lv.key == key && lv.meta == meta && lv.pdir == pdir, "level index buffers");

@@ -85,3 +85,33 @@ def test_tiles_match_the_sums(B, orc, nx, ny, step, bend, hmax, mode, kernel):
     print(f"  largest error {off.max():.3f} of its bound", flush=True)
     assert off.max() < 1.0
     assert abs(got.sum() - ref.sum()) < SUM_TOL * ref.sum()
+
+
+@pytest.mark.parametrize("n,span,cluster", [
+    (1, 0.0, False),               # one particle
+    (700, 0.0, False),             # one h: one level, no level bits
+    (257, 40.0, False),            # levels that the clamp at level 0 shares; a two-word key
+    (20000, 6.0, True),            # most particles in one cell
+    ((1 << 20) + 77, 3.0, True),   # cell maxima in ranges, the last workgroup partial
+])
+def test_level_index_matches_the_sums(B, orc, n, span, cluster):
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(0, 100, (n, 3))
+    if cluster:
+        xyz[: 3 * n // 4] = 50.0 + rng.normal(0, 0.4, (3 * n // 4, 3))
+    w = rng.lognormal(0, 0.3, (n, 1))
+    p4 = np.concatenate([xyz, w], 1).astype(np.float32)
+    h = (20.0 * (n ** -0.3) * 2.0 ** (-span * rng.uniform(0, 1, n))).astype(np.float32)
+    pts = np.zeros((96, 4), np.float32)
+    pts[:, :3] = rng.uniform(0, 100, (96, 3))
+    pts[48:, :3] = p4[rng.integers(0, n, 48), :3] + rng.normal(0, 0.05, (48, 3))
+    print(f"level index n={n} span={span}", flush=True)
+    g = B.GridSmoothing(mode="reference", kernel="quartic_ref", target_particles_per_cell=64)
+    g.init_backend(n)
+    g.setup_particles(p4, [h])
+    g.setup_evaluation_points(pts)
+    g.run()
+    got = g.retrieve_results_f64().cpu().numpy()
+    ref = orc.Grid(p4, h, target=64).smooth3d_ref(pts, form=1)
+    assert ref.max() > 0
+    assert np.all(np.abs(got - ref) <= bound(p4, h, pts))

@@ -52,4 +52,16 @@ __device__ inline float wave_maxf(float v) {
   }));
 }
 
+// the inclusive sum of v over the lanes up to this one
+__device__ inline uint32_t wave_scan(uint32_t v) {
+  int s = int(v);
+  s += dpp_from<0x111, 0xf>(0, s);
+  s += dpp_from<0x112, 0xf>(0, s);
+  s += dpp_from<0x114, 0xf>(0, s);
+  s += dpp_from<0x118, 0xf>(0, s);
+  s += dpp_from<0x142, 0xa>(0, s);
+  s += dpp_from<0x143, 0xc>(0, s);
+  return uint32_t(s);
+}
+
 }  // namespace ilc

@@ -47,31 +47,23 @@ PEAK_FP32_TFLOPS = 157.3  # MI355X vector FP32 (the spec figure counts packed FP
 FLOP_PER_EVAL = 12
 # 3-D pair: dx, dy, dz; r^2 (mul + 2 FMA); s = 1 - r^2/h^2 (FMA); s^2; w s^2 + a (FMA)
 FLOP_PER_EVAL_3D = 13
-# HBM bytes per k_gather_batch launch, from rocprofv3 FETCH_SIZE / WRITE_SIZE
-# runs of this workload scaled by a 1 GiB copy (profiles/k_gather_batch_xray_16M_64views.md);
-# keyed by (workload, mode, tile)
-MEASURED_TRAFFIC = {("c3", "reference", (16, 16, 256)): dict(read=22.63e9, write=3.250e9),
-                    # profiles/k_gather_batch_xray_64M_32slabs.md
-                    ("c5", "reference", (16, 16, 256)): dict(read=21.15e9, write=19.59e9),
-                    # profiles/k_gather_batch_colden_1M_512_and_xray_16M_2048.md
-                    ("c1", "reference", (8, 8, 64)): dict(read=28.80e6, write=10.97e6),
-                    ("c2", "reference", (16, 16, 256)): dict(read=252.97e6, write=161.38e6),
-                    # k_smooth3d, profiles/k_smooth3d_slices_16M.md
-                    ("v1", "reference", (16, 16)): dict(read=1.244e9, write=0.461e9)}
+# HBM bytes per k_gather_batch launch (v1: k_smooth3d), from rocprofv3 FETCH_SIZE /
+# WRITE_SIZE runs of this workload scaled by a 1 GiB copy; keyed by
+# (workload, mode, tile).  None is recorded for the current kernels.
+MEASURED_TRAFFIC = {}
 
 
 def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-# every gather tile shape (w, h, threads per workgroup)
-PLAIN_TILES = [(16, 16, 256), (32, 16, 256), (32, 32, 256), (64, 16, 256), (8, 8, 64),
-               (16, 16, 64)]
+# the gather's two tiles, as exact requests (w, h, threads per workgroup)
+PLAIN_TILES = [(16, 16, 64), (8, 8, 64)]
 
 
 def parse_tile(text):
-    """'WxH' (one tile per 256-thread workgroup) or 'WxH/G' (G threads per
-    workgroup: 256, or 64 for one-wave 16x16 tiles) -> (W, H, G)."""
+    """'WxH' or 'WxH/G' -> (W, H, G): a shape of G = 256 threads leaves the tile side
+    to the number of points, '16x16/64' and '8x8/64' ask for that side."""
     shape, _, wg = text.partition("/")
     w, h = (int(x) for x in shape.split("x"))
     return w, h, int(wg) if wg else 256

@@ -302,8 +302,12 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(
   constexpr bool COUNTING = ITEMS == 4;
   // the ordered tile, one array at a time (3 arrays of 4096 words at once
   // left 3 workgroups per CU: 170 us instead of 97 for a pass over 16M rows
-  // with both values)
-  __shared__ uint32_t so[TILE];
+  // with both values); before that, the sums of the tiles' counts
+  __shared__ union {
+    alignas(16) uint32_t so[TILE];
+    uint32_t sum[SMALL ? 2 : 1][SMALL ? 4 : 1][256];  // each wave's sums, all tiles and those before
+  } sm;
+  auto& so = sm.so;
   __shared__ uint32_t gofs[256];
   __shared__ uint32_t wc[4][256];
   const uint32_t t = threadIdx.x;
@@ -337,14 +341,13 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(
       before.z += b4 ? c.z : 0u;
       before.w += b4 ? c.w : 0u;
     }
-    uint4* sum4 = reinterpret_cast<uint4*>(so);  // [2][4 waves][64]
-    sum4[wave * 64 + lane] = all;
-    sum4[256 + wave * 64 + lane] = before;
+    reinterpret_cast<uint4*>(sm.sum[0][wave])[lane] = all;
+    reinterpret_cast<uint4*>(sm.sum[1][wave])[lane] = before;
     __syncthreads();
     uint32_t a1 = 0, b1 = 0;
     for (int w = 0; w < 4; ++w) {
-      a1 += so[w * 256 + t];
-      b1 += so[1024 + w * 256 + t];
+      a1 += sm.sum[0][w][t];
+      b1 += sm.sum[1][w][t];
     }
     uint32_t tot;
     g0 = block_exclusive_scan(a1, &tot) + b1;  // ends with a barrier

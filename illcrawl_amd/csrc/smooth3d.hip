@@ -218,7 +218,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
 
   // ---- thread t: point t, its search box (reference mode)
   float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
-  bool pv = false;
+  // a point with an infinite or NaN coordinate is out of every particle's
+  // reach: it has no part in the tile's box, plane and search boxes, which
+  // would lose the other points their particles
+  bool pv = false, on = false;
   int lo[3] = {0, 0, 0}, hi[3] = {-1, -1, -1};
   float minr = INFINITY;  // the search radius (the smallest of the tile's is wanted)
   if (t < NP) {
@@ -226,10 +229,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     const uint32_t pid = py * p.lnx + px;
     pv = px < p.lnx && py < p.lny && pid < p.n;
     if (pv) q = p.pts[pid];
-    sm.pt[t] = make_float4(q.x, q.y, q.z, pv ? 1.0f : 0.0f);
+    on = pv && isfinite(q.x) && isfinite(q.y) && isfinite(q.z);
+    sm.pt[t] = make_float4(q.x, q.y, q.z, on ? 1.0f : 0.0f);
   }
   const float qc[3] = {q.x, q.y, q.z};
-  if (REF && pv) {
+  if (REF && on) {
     int32_t c[3];
     for (int a = 0; a < 3; ++a) c[a] = cell_of(qc[a], 0.0f, g.minc[a], g.cs[a]);
     const uint64_t nx = uint64_t(int64_t(g.nc[0])), ny = uint64_t(int64_t(g.nc[1]));
@@ -255,7 +259,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       const int x0 = max(lo[0], 0), x1 = min(hi[0], 65535);
       const int y0 = max(lo[1], 0), y1 = min(hi[1], 65535);
       const int z0 = max(lo[2], 0), z1 = min(hi[2], INT32_MAX - 1);
-      if (pv && x0 <= x1 && y0 <= y1 && z0 <= z1)
+      if (on && x0 <= x1 && y0 <= y1 && z0 <= z1)
         b = make_uint4(uint32_t(x0) | uint32_t(x1 - x0) << 16,
                        uint32_t(y0) | uint32_t(y1 - y0) << 16, uint32_t(z0), uint32_t(z1 - z0));
       sm.box[t] = b;
@@ -268,17 +272,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
   {
     const bool some = wave * 64 < NP;
     for (int a = 0; a < 3; ++a) {
-      const float f0 = some ? wave_minf(pv ? qc[a] : INFINITY) : INFINITY;
-      const float f1 = some ? wave_maxf(pv ? qc[a] : -INFINITY) : -INFINITY;
+      const float f0 = some ? wave_minf(on ? qc[a] : INFINITY) : INFINITY;
+      const float f1 = some ? wave_maxf(on ? qc[a] : -INFINITY) : -INFINITY;
       if (lane == 0) {
         sm.redf[wave][a] = f0;
         sm.redf[wave][3 + a] = f1;
       }
       if constexpr (REF) {
-        const int i0 = some ? wave_mini(pv ? lo[a] : INT32_MAX) : INT32_MAX;  // union
-        const int i1 = some ? wave_maxi(pv ? hi[a] : INT32_MIN) : INT32_MIN;
-        const int i2 = some ? wave_maxi(pv ? lo[a] : INT32_MIN) : INT32_MIN;  // intersection
-        const int i3 = some ? wave_mini(pv ? hi[a] : INT32_MAX) : INT32_MAX;
+        const int i0 = some ? wave_mini(on ? lo[a] : INT32_MAX) : INT32_MAX;  // union
+        const int i1 = some ? wave_maxi(on ? hi[a] : INT32_MIN) : INT32_MIN;
+        const int i2 = some ? wave_maxi(on ? lo[a] : INT32_MIN) : INT32_MIN;  // intersection
+        const int i3 = some ? wave_mini(on ? hi[a] : INT32_MAX) : INT32_MAX;
         if (lane == 0) {
           sm.redi[wave][a] = i0;
           sm.redi[wave][3 + a] = i1;
@@ -291,7 +295,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       const float r = some ? wave_minf(minr) : INFINITY;
       if (lane == 0) sm.minr[wave] = r;
     }
-    const uint64_t any = __ballot(pv);
+    const uint64_t any = __ballot(on);
     if (lane == 0) sm.redi[wave][12] = any ? 1 : 0;
   }
   __syncthreads();
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     }
     for (int k = 0; k < 3; ++k) n[k] = __int_as_float(uniform(__float_as_int(n[k])));
     const float d = n[0] * (q.x - tc[0]) + n[1] * (q.y - tc[1]) + n[2] * (q.z - tc[2]);
-    const float d0 = wave_minf(pv ? d : INFINITY), d1 = wave_maxf(pv ? d : -INFINITY);
+    const float d0 = wave_minf(on ? d : INFINITY), d1 = wave_maxf(on ? d : -INFINITY);
     if (lane == 0) {
       sm.redf[wave][6] = d0;
       sm.redf[wave][7] = d1;

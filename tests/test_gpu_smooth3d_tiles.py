@@ -115,3 +115,43 @@ def test_level_index_matches_the_sums(B, orc, n, span, cluster):
     ref = orc.Grid(p4, h, target=64).smooth3d_ref(pts, form=1)
     assert ref.max() > 0
     assert np.all(np.abs(got - ref) <= bound(p4, h, pts))
+
+
+def with_odd_points(nx, ny, value, axes):
+    """A tilted lattice whose points `odd` have `value` as their coordinates `axes`."""
+    u, v = np.meshgrid((np.arange(nx) - 0.5 * nx) * 0.2, (np.arange(ny) - 0.5 * ny) * 0.2)
+    pts = np.zeros((nx * ny, 4), np.float32)
+    pts[:, 0], pts[:, 1], pts[:, 2] = (50.0 + u).ravel(), (50.0 + v).ravel(), (50.0 + 0.3 * u).ravel()
+    odd = np.array([0, nx * (ny // 2) + nx // 2, nx * ny - 1])
+    pts[np.ix_(odd, axes)] = value
+    return pts, odd
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e25])
+@pytest.mark.parametrize("axes", [[0], [2], [0, 1, 2]])
+@pytest.mark.parametrize("nx,ny", [(40, 33), (1024, 513)])
+@pytest.mark.parametrize("mode,kernel", [("reference", "quartic_ref"), ("exact", "quartic")])
+def test_a_point_out_of_reach_takes_nothing_from_its_tile(B, orc, mode, kernel, nx, ny, axes,
+                                                          value):
+    rng = np.random.default_rng(nx)
+    n = 2000
+    p4 = np.concatenate([rng.uniform(30, 70, (n, 3)), rng.lognormal(0, 0.3, (n, 1))],
+                        1).astype(np.float32)
+    h = np.exp(rng.uniform(np.log(1.0), np.log(15.0), n)).astype(np.float32)
+    pts, odd = with_odd_points(nx, ny, value, axes)
+    print(f"odd points {value} {axes} {nx} x {ny} {mode}", flush=True)
+    g = B.GridSmoothing(mode=mode, kernel=kernel, target_particles_per_cell=64)
+    g.init_backend(n)
+    g.setup_particles(p4, [h])
+    g.setup_evaluation_points(pts, layout_nx=nx)
+    g.run()
+    got = g.retrieve_results_f64().cpu().numpy()
+    # the odd points' neighbours (a tile's side away at most) and some others
+    x, y = odd % nx, odd // nx
+    near = [(b, a) for px, py in zip(x, y) for b in range(max(py - 16, 0), min(py + 17, ny), 3)
+            for a in range(max(px - 16, 0), min(px + 17, nx), 3)]
+    some = np.setdiff1d(np.unique([b * nx + a for b, a in near]), odd)
+    ref = orc.Grid(p4, h, target=64).smooth3d_ref(pts[some], form=1) if mode == "reference" else \
+        orc.smooth3d_exact(p4, h, pts[some])
+    assert ref.max() > 0
+    assert np.all(np.abs(got[some] - ref) <= bound(p4, h, pts[some]))

@@ -773,7 +773,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
   if constexpr (COUNT) {
     cnt[pid] += static_cast<unsigned long long>(v);
   } else {
-    if (sm.covered) {
+    if (sm.covered && on) {
       const double x = double(q.x) - double(tc[0]), y = double(q.y) - double(tc[1]),
                    z = double(q.z) - double(tc[2]);
       const double b[5] = {1.0, x, y, z, x * x + y * y + z * z};

@@ -155,3 +155,4 @@ def test_a_point_out_of_reach_takes_nothing_from_its_tile(B, orc, mode, kernel, 
         orc.smooth3d_exact(p4, h, pts[some])
     assert ref.max() > 0
     assert np.all(np.abs(got[some] - ref) <= bound(p4, h, pts[some]))
+    assert np.all(got[odd] == 0.0)

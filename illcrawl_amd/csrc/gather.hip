@@ -963,9 +963,9 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     double v = sm.sum[0][pt];
     for (int w = 1; w < W; ++w) v += sm.sum[w][pt];
     if constexpr (FAR) {
-      if (interp) {
-        // the far field at the point
-        const float2 e = sm.pt[pt];
+      // the far field at the point (a NaN coordinate is in no support)
+      const float2 e = sm.pt[pt];
+      if (interp && e.x == e.x && e.y == e.y) {
         double bx[kNodes], by[kNodes];
         node_basis(hd_x > 0.0f ? double(e.x - tcx) / double(hd_x) : 0.0, bx);
         node_basis(hd_y > 0.0f ? double(e.y - tcy) / double(hd_y) : 0.0, by);

@@ -189,3 +189,41 @@ def test_grid_sort_at_the_tile_and_path_limits(B, orc, n):
     assert np.array_equal(maxh.cpu().numpy(), g.maxh_cell)
     assert np.array_equal(perm.cpu().numpy().astype(np.uint32), g.perm)
     print(f"sort n={n}: {g.ncells} cells", flush=True)
+
+
+def odd_lattice(value, axes):
+    """1024 x 771 points (16x16 tiles), three of them with `value` as `axes`."""
+    nx, ny = 1024, 771
+    pts = lattice(nx, ny, -0.05 * nx, -0.05 * ny, 0.1)
+    odd = np.array([0, 385 * nx + 512, nx * ny - 1])
+    pts[np.ix_(odd, axes)] = value
+    near = [b * nx + a for c in odd for b in range(max(c // nx - 16, 0), min(c // nx + 17, ny), 3)
+            for a in range(max(c % nx - 16, 0), min(c % nx + 17, nx), 3)]
+    return pts, nx, odd, np.setdiff1d(np.unique(near), odd)
+
+
+def wide_particles(n, seed):
+    rng = np.random.default_rng(seed)
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, 0], p4[:, 1] = rng.uniform(-70, 70, n), rng.uniform(-60, 60, n)
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    return p4, np.exp(rng.uniform(np.log(0.5), np.log(60.0), n)).astype(np.float32)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("axes", [[0], [0, 1]])
+@pytest.mark.parametrize("mode,kernel", [("reference", "quartic_ref"), ("exact", "quartic"),
+                                         ("exact", "cubic")])
+def test_points_out_of_reach(B, orc, mode, kernel, axes, value):
+    """A point with an infinite or NaN coordinate is worth 0, as the oracle has
+    it, and its tile's other points lose nothing."""
+    p4, h = wide_particles(2000, 7)
+    pts, nx, odd, some = odd_lattice(value, axes)
+    print(f"points out of reach: {mode} {kernel} {axes} {value}", flush=True)
+    got = render(B, p4, h, pts, nx, mode=mode, kernel=kernel)
+    ref = orc.Grid(p4, h).gather_ref(pts[some], acc_mode=1) if mode == "reference" else \
+        orc.gather_exact(p4, h, pts[some], kind={"quartic": 1, "cubic": 2}[kernel])
+    linf, s = rel_errors(got[some], ref)
+    # the cubic kernel is tabulated: the parity tests' 2e-5
+    assert linf < (2e-5 if kernel == "cubic" else LINF_TOL) and s < SUM_TOL
+    assert np.all(got[odd] == 0.0)

@@ -1122,9 +1122,13 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
     const uint32_t pid = iy * p.lnx + ix;
     if (ix < p.lnx && iy < p.lny && pid < p.n) {
       const float4 q = p.gen ? pixel_point(p.pg, ix, iy) : p.pts[pid];
-      px = q.x;
-      py = q.y;
-      pg = io.grad[pid] * io.scale;
+      // a point with an infinite or NaN coordinate is in no support (its
+      // moments would be 0 times that)
+      if (isfinite(q.x) && isfinite(q.y)) {
+        px = q.x;
+        py = q.y;
+        pg = io.grad[pid] * io.scale;
+      }
     }
     sm.pt[t] = make_float4(px, py, pg, 0.0f);
   }

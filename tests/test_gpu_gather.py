@@ -227,3 +227,26 @@ def test_points_out_of_reach(B, orc, mode, kernel, axes, value):
     # the cubic kernel is tabulated: the parity tests' 2e-5
     assert linf < (2e-5 if kernel == "cubic" else LINF_TOL) and s < SUM_TOL
     assert np.all(got[odd] == 0.0)
+
+
+def adjoint(B, p4, h, pts, nx, G):
+    b = B.ProjectiveSmoothingGrid(mode="exact", kernel="quartic", target_particles_per_cell=40)
+    b.init_backend(p4.shape[0])
+    b.setup_projected_particles(p4, h)
+    b.setup_evaluation_points(pts, layout_nx=nx)
+    return [t.cpu().numpy() for t in b.backward(torch.from_numpy(G).cuda(), 1.0)]
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("axes", [[0], [0, 1]])
+def test_adjoint_of_points_out_of_reach(B, orc, axes, value):
+    """They add nothing to any particle's gradient."""
+    p4, h = wide_particles(300, 8)
+    pts, nx, odd, _ = odd_lattice(value, axes)
+    G = np.random.default_rng(8).normal(size=pts.shape[0]).astype(np.float32)
+    got = adjoint(B, p4, h, pts, nx, G)
+    ref = orc.backward_exact(p4, h, pts, G, kind=1)
+    for name, a, r in zip(("w", "h", "x", "y"), got, ref):
+        e = float(np.max(np.abs(a - r)) / np.max(np.abs(r)))
+        print(f"adjoint with points at {value} {axes} dL/d{name}: {e:.2e}", flush=True)
+        assert e < 1e-4

@@ -1077,6 +1077,7 @@ struct adjoint_smem {
   static constexpr int NP = T * T;
   float4 pt[NP];  // tile points (x, y, dL/dvalue, -), 8x8 block after 8x8 block
   float4 box[NP / 64];  // the blocks' boxes of points with a gradient (x0, y0, x1, y1)
+  int wild[NP / 64];    // whether a block's gradients are infinite or NaN somewhere
   alignas(16) float node[KERNEL == 0 && NP > 64 ? 64 : 1];  // the gradients at the nodes
   union {
     uint32_t idx[kSumW][kAdjCap];
@@ -1136,11 +1137,17 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
     const bool on = pg != 0.0f;
     const float x0 = wave_minf(on ? px : INFINITY), y0 = wave_minf(on ? py : INFINITY);
     const float x1 = wave_maxf(on ? px : -INFINITY), y1 = wave_maxf(on ? py : -INFINITY);
-    if (lane == 0 && wave < NBLK) sm.box[wave] = make_float4(x0, y0, x1, y1);
+    const bool wild = __ballot(!isfinite(pg)) != 0;
+    if (lane == 0 && wave < NBLK) {
+      sm.box[wave] = make_float4(x0, y0, x1, y1);
+      sm.wild[wave] = wild;
+    }
   }
   __syncthreads();
   float tbx0 = INFINITY, tby0 = INFINITY, tbx1 = -INFINITY, tby1 = -INFINITY;
+  int wild = 0;
   for (int b = 0; b < NBLK; ++b) {
+    wild |= sm.wild[b];
     const float4 x = sm.box[b];
     tbx0 = fminf(tbx0, x.x);
     tby0 = fminf(tby0, x.y);
@@ -1156,8 +1163,9 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
   const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
   const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
 
-  // ---- the gradients at the nodes (when any particle is wide enough)
-  const bool nodes = FAR && g.max_h * g.max_h * 0.16f >= hd2;
+  // ---- the gradients at the nodes (when any particle is wide enough; an
+  // infinite one would meet weights of either sign there)
+  const bool nodes = FAR && !uniform(wild) && g.max_h * g.max_h * 0.16f >= hd2;
   if constexpr (FAR) {
     if (nodes) {
       double b[kNodes];

@@ -250,3 +250,26 @@ def test_adjoint_of_points_out_of_reach(B, orc, axes, value):
         e = float(np.max(np.abs(a - r)) / np.max(np.abs(r)))
         print(f"adjoint with points at {value} {axes} dL/d{name}: {e:.2e}", flush=True)
         assert e < 1e-4
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_adjoint_of_a_point_without_a_finite_gradient(B, orc, value):
+    """dL/dw of the particles that cover the point is that value (at the nodes
+    of a tile it would meet weights of either sign); those a tile's diagonal
+    beyond their support have the other points' gradient."""
+    p4, h = wide_particles(300, 9)
+    pts, nx, odd, _ = odd_lattice(0.0, [2])
+    G = np.random.default_rng(9).normal(size=pts.shape[0]).astype(np.float32)
+    c = odd[1]
+    G[c] = 0.0
+    ref = orc.backward_exact(p4, h, pts, G, kind=1)
+    G[c] = value
+    got = adjoint(B, p4, h, pts, nx, G)
+    r = np.hypot(p4[:, 0] - pts[c, 0], p4[:, 1] - pts[c, 1])
+    covers, clear = r < 0.999 * h, r > h + 0.1 * 16 * 1.5
+    assert covers.sum() > 20 and clear.sum() > 20
+    assert np.array_equal(got[0][covers], np.full(covers.sum(), value, np.float32), equal_nan=True)
+    for name, a, x in zip(("w", "h", "x", "y"), got, ref):
+        e = float(np.max(np.abs(a[clear] - x[clear])) / np.max(np.abs(x)))
+        print(f"adjoint with a gradient of {value} dL/d{name}: {e:.2e}", flush=True)
+        assert e < 1e-4

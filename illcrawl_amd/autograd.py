@@ -28,11 +28,12 @@ from .backend import (ProjectiveSmoothingGrid, camera_pixel_points, camera_proje
 # for the device: a forward and backward of 20k particles on 96^2 pixels takes
 # 0.70 ms with a handle of its own, 0.47 with one taken over.  Handles of up to
 # _POOL_ROWS particles, pixels and grid cells are kept (at most some 60 MB each; a
-# larger pass takes longer than the allocations), _POOL_SIZE per device and
-# configuration: two alternate while the image of the pass before is alive.
+# larger pass takes longer than the allocations), _POOL_SIZE per device over all
+# configurations, the newest (two alternate while the image of the pass before
+# is alive).  They are not torch's memory: release_handles() gives it back.
 _POOL_ROWS = 1 << 18
-_POOL_SIZE = 2
-_pool = collections.defaultdict(collections.deque)
+_POOL_SIZE = 4
+_pool = collections.defaultdict(collections.deque)   # device: (target, kernel), handle, event
 _pool_lock = threading.RLock()   # a lease may end inside the collector, on any thread
 
 
@@ -53,15 +54,18 @@ class _Lease:
     an event behind its last work, which its next holder's stream waits for."""
 
     def __init__(self, device, target, kernel, rows):
-        self.key = (device, target, kernel)
+        self.device, self.config = device, (target, kernel)
         self.event = None        # None: not to be pooled
         self.small = rows <= _POOL_ROWS
         self.psg = None
         if self.small:
             with _pool_lock:
-                free = _pool.get(self.key)
-                if free:
-                    self.psg, event = free.pop()
+                free = _pool[device]
+                for k in range(len(free) - 1, -1, -1):   # the newest
+                    if free[k][0] == self.config:
+                        _, self.psg, event = free[k]
+                        del free[k]
+                        break
             if self.psg is not None:
                 torch.cuda.current_stream(device).wait_event(event)
         if self.psg is None:
@@ -69,8 +73,8 @@ class _Lease:
 
     def used(self):
         """Marks the end of the work enqueued so far on the current stream."""
-        stream = torch.cuda.current_stream(self.key[0])
-        with torch.cuda.device(self.key[0]):
+        stream = torch.cuda.current_stream(self.device)
+        with torch.cuda.device(self.device):
             if not self.small or torch.cuda.is_current_stream_capturing():
                 # a captured graph keeps reading the handle's buffers
                 self.small, self.event = False, None
@@ -88,10 +92,14 @@ class _Lease:
     def __del__(self):
         if getattr(self, "event", None) is None or _pool_lock is None:
             return
+        self.psg._keep = []   # the next holder sets its own points
+        oldest = None
         with _pool_lock:
-            free = _pool[self.key]
-            if len(free) < _POOL_SIZE:
-                free.append((self.psg, self.event))
+            free = _pool[self.device]
+            free.append((self.config, self.psg, self.event))
+            if len(free) > _POOL_SIZE:
+                oldest = free.popleft()
+        del oldest   # destroyed outside the lock
 
 
 class ProjectedImage(torch.autograd.Function):

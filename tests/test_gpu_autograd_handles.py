@@ -106,3 +106,22 @@ def test_large_passes_keep_nothing(A):
     A.release_handles()
     run(A, inputs(A._POOL_ROWS + 1, 16, 5))
     assert not any(A._pool.values())
+
+
+def test_kept_handles_are_bounded_over_all_configurations(A):
+    """Passes of many configurations leave no more handles than passes of one,
+    the newest, and none of their points."""
+    A.release_handles()
+    case = inputs(500, 20, 1)
+    x, cam, g = case
+    fresh = run(A, case)
+    for target in (8, 20, 50, 120, 300, 700, 900, 2000):
+        for kernel in ("quartic", "cubic"):
+            img = A.projected_image(*x, cam, kernel=kernel, target_particles_per_cell=target)
+            torch.autograd.grad(img, x, g)
+            del img
+    kept = [e for q in A._pool.values() for e in q]
+    print(f"handles kept: {len(kept)}", flush=True)
+    assert 0 < len(kept) <= A._POOL_SIZE
+    assert not any(p._keep for e in kept for p in e if hasattr(p, "_keep"))
+    same(run(A, case), fresh)

@@ -246,10 +246,10 @@ struct cell_table {
 
 // Streams the candidate particles of the cell box [cx0, cx1] x [cy0, cy1] x
 // [cz0, cz1] for the tile box (tbx0, tby0, tbx1, tby1): calls batch(have,
-// sorted index, packed cell, in_all(cell), done) on the waves, 64 candidates
-// at a time dealt to the waves in turn, and once per wave at the end with
-// done set and no candidate.  Every thread of the workgroup takes part.
-template <bool REF, class InAll, class Batch>
+// sorted index, packed cell, in_all(cell), done) on the waves, up to 64
+// candidates at a time dealt to the waves in turn, and once per wave at the end
+// with done set and no candidate.  Every thread of the workgroup takes part.
+template <bool REF, bool EVEN, class InAll, class Batch>
 __device__ __attribute__((always_inline)) inline void stream_candidates(
     const grid_view& g, int cx0, int cx1, int cy0, int cy1, int cz0, int cz1, float tbx0,
     float tby0, float tbx1, float tby1, float support, InAll&& in_all, cell_table& ct,
@@ -356,16 +356,25 @@ __device__ __attribute__((always_inline)) inline void stream_candidates(
     __syncthreads();
     // the chunk's particles, 64 at a time, dealt to the waves in turn; after
     // the last of them the wave's lists are evaluated whatever their size
-    // (here and not behind the loop: one copy of the evaluation code)
+    // (here and not behind the loop: one copy of the evaluation code).
+    // EVEN: a chunk of less than 64 for each wave is dealt evenly, for the sums
+    // of 16x16 tiles: a candidate is work for the whole wave, and in sparse
+    // tiles (100 candidates) two waves had all the pairs and two had none (16
+    // slabs of 4096^2 through 32M particles, gather 13.6 -> 12.1 ms; a cubic
+    // 2048^2 view of 1M 13.5 -> 12.7).  With one pair a lane and candidate (8x8
+    // tiles) the half-empty culls cost as much (24 views of 200^2 of 1M 3.9 ->
+    // 4.06); in the adjoint a candidate is a lane's.
     const bool last_chunk = c0 + NB >= nitems;
-    for (uint32_t v0 = uint32_t(wave) * 64u;; v0 += NB) {
+    const uint32_t deal =
+        EVEN && tot < uint32_t(NB) ? max(1u, (tot + kSumW - 1) / kSumW) : 64u;
+    for (uint32_t v0 = uint32_t(wave) * deal;; v0 += deal * kSumW) {
       const bool done = v0 >= tot;
       if (done && !last_chunk) break;
       const uint32_t v = v0 + uint32_t(lane);
       bool have = false;
       uint32_t sidx = 0;
       int cinf = 0, cf = 0;
-      if (v < tot) {
+      if (v < tot && uint32_t(lane) < deal) {
         // last cell whose offset is <= v (it has a nonzero count)
         int lo = 0;
 #pragma unroll
@@ -835,7 +844,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     nm = 0;
   };
 
-  stream_candidates<REF>(
+  stream_candidates<REF, (PPT > 1)>(
       g, cx0, cx1, cy0, cy1, cz0, cz1, tbx0, tby0, tbx1, tby1, support,
       [&](int cx, int cy) {
         return allz_u && cy >= r_ily && cy <= r_ihy && cx >= r_ilx && cx <= r_ihx;
@@ -1302,7 +1311,7 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
     }
   };
 
-  stream_candidates<false>(
+  stream_candidates<false, false>(
       g, cx0, cx1, cy0, cy1, 0, g.nc[2] - 1, tbx0, tby0, tbx1, tby1, support,
       [](int, int) { return true; }, sm.cells,
       [&](bool have, uint32_t sidx, int, bool, bool done) {

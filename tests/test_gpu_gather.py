@@ -273,3 +273,46 @@ def test_adjoint_of_a_point_without_a_finite_gradient(B, orc, value):
         e = float(np.max(np.abs(a[clear] - x[clear])) / np.max(np.abs(x)))
         print(f"adjoint with a gradient of {value} dL/d{name}: {e:.2e}", flush=True)
         assert e < 1e-4
+
+
+def pair_bound(pp, h, pts, kernel):
+    """Rounding of the FP32 pairs (c s)^2.5, s = 1 - r^2/h^2, per point, with
+    u = 2^-24.  The argument c s is a sum of terms of at most 1.5 c, each off by
+    some 6 u: 24 u c in all, the value by 2.5 coef s^1.5 24 u; the power, the
+    coefficient and a partial sum of 32 pairs by 50 u of it."""
+    u = 2.0 ** -24
+    norm = 3.5 / np.pi if kernel == "quartic" else 2.0 * 1.04445 * 1.066667
+    h2 = h.astype(np.float64) ** 2
+    coef = norm * np.abs(pp[:, 3].astype(np.float64)) / h2
+    r2 = sum((pts[:, None, a].astype(np.float64) - pp[None, :, a].astype(np.float64)) ** 2
+             for a in range(2))
+    s = np.maximum(1.0 - r2 / h2, 0.0)
+    return ((60 * u * s ** 1.5 + 50 * u * s ** 2.5 + (24 * u) ** 2.5) * coef).sum(1)
+
+
+@pytest.mark.parametrize("mode,kernel", [("reference", "quartic_ref"), ("exact", "quartic"),
+                                         ("exact", "cubic")])
+@pytest.mark.parametrize("n", [1, 3, 5, 63, 66, 255, 256, 257])
+def test_few_candidates_for_a_tile(B, orc, n, mode, kernel):
+    """A 16x16 tile with fewer candidates than its four waves take at a time."""
+    rng = np.random.default_rng(n)
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :2] = rng.uniform(-7, 7, (n, 2))
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    h = np.exp(rng.uniform(np.log(0.8), np.log(30.0), n)).astype(np.float32)
+    view = dict(position=np.array([0.0, 0.0, -20.0]), look_at=np.array([0.0, 0.0, 1.0]),
+                roll=0.0, width=16.0, nx=16, ny=16, depth=40.0)
+    cam = orc.Camera(view["position"], view["look_at"], view["roll"], view["width"], 16, 16)
+    pp, pts = cam.project_particles(p4, view["depth"]), cam.pixel_points()
+    ref = orc.Grid(pp, h).gather_ref(pts, acc_mode=1) if mode == "reference" else \
+        orc.gather_exact(pp, h, pts, kind={"quartic": 1, "cubic": 2}[kernel])
+    r = B.BatchRenderer(mode=mode, kernel=kernel, tile=(16, 16, 64))
+    r.set_particles(p4[:, :3].copy(), p4[:, 3].copy(), h)
+    r.set_views([view])
+    r.render()
+    got = r.image_f64(0).cpu().numpy().reshape(-1)
+    print(f"few candidates n={n} {mode} {kernel}", flush=True)
+    if kernel == "cubic":  # tabulated: the parity tests' 2e-5, of the largest value
+        assert np.max(np.abs(got - ref)) < 2e-5 * ref.max()
+    else:
+        assert np.all(np.abs(got - ref) <= pair_bound(pp, h, pts, kernel))

@@ -530,6 +530,10 @@ void plan(ilc_batch* b, hipStream_t s) {
     nitems += vs.ntiles;
   }
   ILC_REQUIRE(nitems < (uint64_t(1) << 32), "too many work items");
+  bool slabs = true;
+  for (auto& v : b->views) slabs = slabs && v->compact;
+  b->ss.quad = slabs && !b->clip && b->kernel != ILC_KERNEL_CUBIC && b->ss.side == 16 &&
+               quarter_tiles(nitems, ntot);
   // queue q: the q-th eighth (contiguous tiles, image order) of every view,
   // largest views first
   uint2* it = b->items_host.ensure(nitems);

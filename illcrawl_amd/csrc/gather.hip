@@ -212,27 +212,32 @@ __device__ inline bool is_far(float r2, float ih2, float a2, float slope = 0.22f
 // workgroup barriers, and a tile of 64 points had one wave: one wave per tile
 // takes 1.25 ms for a 512^2 view of 1M particles, four 0.80, eight 0.79, at
 // 8x8 points; 6 frames of 160x120 1.12, 0.71, 0.73.)
+//
+// QUAD: in a 16x16 tile every wave works on one 8x8 quarter, one point a lane,
+// with all of the tile's candidates.  Nothing is added up at the end, a lane
+// needs 64 registers (8 waves a SIMD, not 5), and a particle smaller than the
+// tile costs only the quarters that it reaches; but a candidate is culled four
+// times, and wide particles have no nodes.  Taken where quarter_tiles says.
 constexpr int kSumW = 4;
 
-// a wave evaluates a list when it reaches kWaveFlush entries; a batch of 64
-// candidates lands on a list of at most kWaveFlush - 1
-constexpr int kWaveFlush = 32;
-// one list, and two lists sharing an array from its two ends, with room to
-// pad either to a multiple of 4 entries
-constexpr int kWaveCap = kWaveFlush - 1 + 64 + 1;
-constexpr int kWavePool = 2 * (kWaveFlush - 1) + 64 + 6;
-static_assert(kWaveCap % 4 == 0 && kWavePool % 4 == 0, "whole groups of 4 entries");
-
-template <bool REF, int KERNEL, bool CLIP, bool COUNT>
+// A wave's lists.  It evaluates one when it reaches FLUSH entries; a batch of 64
+// candidates lands on a list of at most FLUSH - 1.
+template <bool REF, int KERNEL, bool CLIP, bool COUNT, bool QUAD>
 struct wave_lists {
+  static constexpr int FLUSH = QUAD ? 16 : 32;
+  // one list, and two lists sharing an array from its two ends, with room to
+  // pad either to a multiple of 4 entries
+  static constexpr int CAP = FLUSH - 1 + 64 + 1;
+  static constexpr int POOL = 2 * (FLUSH - 1) + 64 + 6;
+  static_assert(CAP % 4 == 0 && POOL % 4 == 0, "whole groups of 4 entries");
   static constexpr bool QUARTIC = KERNEL == 0 && !COUNT;
-  alignas(16) float4 X[QUARTIC ? kWavePool : 1];  // expansion form: far from the front, big from the back
-  float4 S[REF ? kWavePool : kWaveCap];  // position form: small from the front, masked from the back
-  alignas(16) int M[REF ? kWaveCap : 1];  // masked: packed cell (cx | cy << 16)
+  alignas(16) float4 X[QUARTIC ? POOL : 1];  // expansion form: far from the front, big from the back
+  float4 S[REF ? POOL : CAP];  // position form: small from the front, masked from the back
+  alignas(16) int M[REF ? CAP : 1];  // masked: packed cell (cx | cy << 16)
   // line-of-sight clip: per entry, the depth range relative to the particle
   // in units of h, times c^(1/2) (see clip_pow)
-  float2 Xz[CLIP ? kWavePool : 1];
-  float2 Sz[CLIP ? kWaveCap : 1];
+  float2 Xz[CLIP ? POOL : 1];
+  float2 Sz[CLIP ? CAP : 1];
 };
 
 // The workgroup's chunk of candidate cells (or of rows of them).
@@ -247,9 +252,11 @@ struct cell_table {
 // Streams the candidate particles of the cell box [cx0, cx1] x [cy0, cy1] x
 // [cz0, cz1] for the tile box (tbx0, tby0, tbx1, tby1): calls batch(have,
 // sorted index, packed cell, in_all(cell), done) on the waves, up to 64
-// candidates at a time dealt to the waves in turn, and once per wave at the end
-// with done set and no candidate.  Every thread of the workgroup takes part.
-template <bool REF, bool EVEN, class InAll, class Batch>
+// candidates at a time, and once per wave at the end with done set and no
+// candidate.  The candidates are dealt to the waves in turn, or every wave takes
+// all of them (DEAL_ALL).  Every thread of the workgroup takes part.
+enum deal_kind { DEAL_64, DEAL_EVEN, DEAL_ALL };
+template <bool REF, deal_kind DEAL, class InAll, class Batch>
 __device__ __attribute__((always_inline)) inline void stream_candidates(
     const grid_view& g, int cx0, int cx1, int cy0, int cy1, int cz0, int cz1, float tbx0,
     float tby0, float tbx1, float tby1, float support, InAll&& in_all, cell_table& ct,
@@ -357,7 +364,7 @@ __device__ __attribute__((always_inline)) inline void stream_candidates(
     // the chunk's particles, 64 at a time, dealt to the waves in turn; after
     // the last of them the wave's lists are evaluated whatever their size
     // (here and not behind the loop: one copy of the evaluation code).
-    // EVEN: a chunk of less than 64 for each wave is dealt evenly, for the sums
+    // DEAL_EVEN: a chunk of less than 64 for each wave is dealt evenly, for the sums
     // of 16x16 tiles: a candidate is work for the whole wave, and in sparse
     // tiles (100 candidates) two waves had all the pairs and two had none (16
     // slabs of 4096^2 through 32M particles, gather 13.6 -> 12.1 ms; a cubic
@@ -366,8 +373,9 @@ __device__ __attribute__((always_inline)) inline void stream_candidates(
     // 4.06); in the adjoint a candidate is a lane's.
     const bool last_chunk = c0 + NB >= nitems;
     const uint32_t deal =
-        EVEN && tot < uint32_t(NB) ? max(1u, (tot + kSumW - 1) / kSumW) : 64u;
-    for (uint32_t v0 = uint32_t(wave) * deal;; v0 += deal * kSumW) {
+        DEAL == DEAL_EVEN && tot < uint32_t(NB) ? max(1u, (tot + kSumW - 1) / kSumW) : 64u;
+    constexpr uint32_t TURNS = DEAL == DEAL_ALL ? 1 : kSumW;
+    for (uint32_t v0 = uint32_t(wave) % TURNS * deal;; v0 += deal * TURNS) {
       const bool done = v0 >= tot;
       if (done && !last_chunk) break;
       const uint32_t v = v0 + uint32_t(lane);
@@ -401,19 +409,19 @@ __device__ __attribute__((always_inline)) inline void stream_candidates(
   }
 }
 
-template <int T, bool REF, int KERNEL, bool CLIP, bool COUNT>
+template <int T, bool REF, int KERNEL, bool CLIP, bool COUNT, bool QUAD>
 struct tile_smem {
   static constexpr int W = kSumW, NB = 64 * W;
   union {
-    wave_lists<REF, KERNEL, CLIP, COUNT> L[W];
+    wave_lists<REF, KERNEL, CLIP, COUNT, QUAD> L[W];
     struct {                      // at the end of the tile: the waves' sums
-      double sum[W][T * T];
-      double node[KERNEL == 0 && !CLIP && !COUNT && T * T > 64 ? W : 1][64];
+      double sum[QUAD ? 1 : W][QUAD ? 1 : T * T];
+      double node[KERNEL == 0 && !CLIP && !COUNT && !QUAD && T * T > 64 ? W : 1][64];
     };
   };
   int far_used;
-  float2 pt[T * T];          // the tile's points
-  uint2 box[REF ? T * T : 1];  // their search boxes: (x0 | xw << 16, y0 | yw << 16)
+  float2 pt[QUAD ? 1 : T * T];          // the tile's points
+  uint2 box[REF && !QUAD ? T * T : 1];  // their search boxes: (x0 | xw << 16, y0 | yw << 16)
   float tab[KERNEL == 2 ? kCubicTable : 1];
   cell_table cells;
   float redf[W][5];
@@ -431,13 +439,13 @@ __device__ inline void wave_sync() {
 // One tile (tx, ty) of the point image: everything between the point loads
 // and the accumulator update.  All threads of the workgroup call it with the
 // same arguments.
-template <int T, int OP, int KERNEL>
+template <int T, int OP, int KERNEL, bool QUAD>
 __device__ __attribute__((always_inline)) inline void sum_tile(
     const grid_view& g, const point_view& p, uint32_t tx, uint32_t ty, double* __restrict__ acc_out,
     unsigned long long* __restrict__ counts, float support,
-    tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT>& sm,
+    tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT, QUAD>& sm,
     float* __restrict__ img_out = nullptr, float img_scale = 1.0f, int fused = 0) {
-  constexpr int W = kSumW, NB = 64 * W, NP = T * T, PPT = NP / 64;
+  constexpr int W = kSumW, NB = 64 * W, NP = T * T, PPT = QUAD ? 1 : NP / 64;
   constexpr bool REF = OP == OP_REFERENCE;
   constexpr bool COUNT = OP == OP_COUNT;
   constexpr bool CLIP = OP == OP_CLIP;
@@ -446,9 +454,19 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   constexpr bool FAR = QUARTIC && !CLIP && PPT > 1;
   static_assert(!CLIP || KERNEL == 0, "the line-of-sight clip is the quartic's");
   static_assert(NP % 64 == 0, "whole points per lane");
+  static_assert(!QUAD || (T == 16 && W == 4), "a wave for each 8x8 quarter");
+  using lists = wave_lists<REF, KERNEL, CLIP, COUNT, QUAD>;
+  constexpr int POOL = lists::POOL, FLUSH = lists::FLUSH;
 
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
+
+  // point pt's column and row in the tile
+  auto col_of = [](int pt) { return QUAD ? (pt >> 6 & 1) * 8 + (pt & 7) : pt % T; };
+  auto row_of = [](int pt) { return QUAD ? (pt >> 7) * 8 + (pt >> 3 & 7) : pt / T; };
+  // QUAD: the lane's point and its search box
+  float2 my_pt = make_float2(0.f, 0.f);
+  uint2 my_box = make_uint2(0xffffu, 0xffffu);
 
   // ---- the tile's points (thread t: points t, t + NB, ...), their search
   // boxes, and the tile reductions
@@ -459,13 +477,12 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   float minr = INFINITY;  // reference mode: the smallest search radius of the points
 #pragma unroll 1
   for (int pt = t; pt < NP; pt += NB) {
-    const uint32_t px = tx * T + uint32_t(pt % T), py = ty * T + uint32_t(pt / T);
+    const uint32_t px = tx * T + uint32_t(col_of(pt)), py = ty * T + uint32_t(row_of(pt));
     const uint32_t pid = py * p.lnx + px;
     const bool pv = px < p.lnx && py < p.lny && pid < p.n;
     float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
     if (pv) q = p.gen ? pixel_point(p.pg, px, py) : p.pts[pid];
-    sm.pt[pt] = make_float2(q.x, q.y);
-    if constexpr (REF) sm.box[pt] = make_uint2(0xffffu, 0xffffu);  // no such cell in a grid of < 2^32
+    uint2 box = make_uint2(0xffffu, 0xffffu);  // no such cell in a grid of < 2^32
     if (pv) {
       anyv = 1;
       bminx = fminf(bminx, q.x);
@@ -509,14 +526,27 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
           const int x0 = max(lox, 0), x1 = min(hix, 65535);
           const int y0 = max(loy, 0), y1 = min(hiy, 65535);
           if (x0 <= x1 && y0 <= y1)
-            sm.box[pt] = make_uint2(uint32_t(x0) | uint32_t(x1 - x0) << 16,
-                                    uint32_t(y0) | uint32_t(y1 - y0) << 16);
+            box = make_uint2(uint32_t(x0) | uint32_t(x1 - x0) << 16,
+                             uint32_t(y0) | uint32_t(y1 - y0) << 16);
         }
       }
     }
+    if constexpr (QUAD) {
+      my_pt = make_float2(q.x, q.y);
+      my_box = box;
+    } else {
+      sm.pt[pt] = make_float2(q.x, q.y);
+      if constexpr (REF) sm.box[pt] = box;
+    }
   }
+  // QUAD: the box of the wave's points
+  float wbx0, wby0, wbx1, wby1;
   {
     const float v0 = wave_minf(bminx), v1 = wave_minf(bminy), v2 = wave_maxf(bmaxx), v3 = wave_maxf(bmaxy);
+    wbx0 = v0;
+    wby0 = v1;
+    wbx1 = v2;
+    wby1 = v3;
     int iv[11] = {0};
     float v4 = INFINITY;
     if constexpr (REF) {
@@ -578,10 +608,18 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     return;
   }
 
-  // tile centre: the origin of the expansion form
-  const float tcx = 0.5f * (tbx0 + tbx1), tcy = 0.5f * (tby0 + tby1);
-  // a particle is "big" when h >= 2 * tile half-diagonal
-  const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
+  // the box that the wave's lists serve, the tile's or its quarter's (of no
+  // point: infinite, and nothing is kept)
+  if constexpr (!QUAD) {
+    wbx0 = tbx0;
+    wby0 = tby0;
+    wbx1 = tbx1;
+    wby1 = tby1;
+  }
+  // its centre: the origin of the expansion form
+  const float tcx = 0.5f * (wbx0 + wbx1), tcy = 0.5f * (wby0 + wby1);
+  // a particle is "big" when h >= 2 * half-diagonal
+  const float hd_x = 0.5f * (wbx1 - wbx0), hd_y = 0.5f * (wby1 - wby0);
   const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
   const float big_r2 = 4.0f * hd2 * 1.0001f + 1e-30f;
 
@@ -657,14 +695,14 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   auto eval_big = [&]() {
     if constexpr (QUARTIC) {
       const int n = uniform(nb), n4 = (n + 3) & ~3;
-      if (lane < n4 - n) L.X[kWavePool - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (lane < n4 - n) L.X[POOL - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
       if constexpr (CLIP)
-        if (lane < n4 - n) L.Xz[kWavePool - 1 - (n + lane)] = make_float2(0.f, 0.f);
+        if (lane < n4 - n) L.Xz[POOL - 1 - (n + lane)] = make_float2(0.f, 0.f);
       wave_sync();
       float lx[PPT], ly[PPT], l2[PPT];
 #pragma unroll
       for (int k = 0; k < PPT; ++k) {
-        const float2 e = sm.pt[lane + 64 * k];
+        const float2 e = QUAD ? my_pt : sm.pt[lane + 64 * k];
         lx[k] = e.x - tcx;
         ly[k] = e.y - tcy;
         l2[k] = fmaf(ly[k], ly[k], lx[k] * lx[k]);
@@ -679,8 +717,8 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
           float2 z[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            q[u] = L.X[kWavePool - 1 - (j0 + j + u)];
-            if constexpr (CLIP) z[u] = L.Xz[kWavePool - 1 - (j0 + j + u)];
+            q[u] = L.X[POOL - 1 - (j0 + j + u)];
+            if constexpr (CLIP) z[u] = L.Xz[POOL - 1 - (j0 + j + u)];
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u)
@@ -740,7 +778,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     float ex[PPT], ey[PPT];
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
-      const float2 e = sm.pt[lane + 64 * k];
+      const float2 e = QUAD ? my_pt : sm.pt[lane + 64 * k];
       ex[k] = e.x;
       ey[k] = e.y;
     }
@@ -799,7 +837,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     if constexpr (REF) {
       const int n = uniform(nm), n4 = (n + 3) & ~3;
       if (lane < n4 - n) {
-        L.S[kWavePool - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+        L.S[POOL - 1 - (n + lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
         L.M[n + lane] = 0;
       }
       wave_sync();
@@ -807,10 +845,10 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
       uint2 bx[PPT];
 #pragma unroll
       for (int k = 0; k < PPT; ++k) {
-        const float2 e = sm.pt[lane + 64 * k];
+        const float2 e = QUAD ? my_pt : sm.pt[lane + 64 * k];
         ex[k] = e.x;
         ey[k] = e.y;
-        bx[k] = sm.box[lane + 64 * k];
+        bx[k] = QUAD ? my_box : sm.box[lane + 64 * k];
       }
       for (int j0 = 0; j0 < n4; j0 += 32) {
         const int jn = min(32, n4 - j0);
@@ -822,7 +860,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
           const int cc[4] = {uniform(c4.x), uniform(c4.y), uniform(c4.z), uniform(c4.w)};
           float4 q[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) q[u] = L.S[kWavePool - 1 - (j0 + j + u)];
+          for (int u = 0; u < 4; ++u) q[u] = L.S[POOL - 1 - (j0 + j + u)];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const uint32_t cx = uint32_t(cc[u]) & 0xffffu, cy = uint32_t(cc[u]) >> 16;
@@ -844,7 +882,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
     nm = 0;
   };
 
-  stream_candidates<REF, (PPT > 1)>(
+  stream_candidates<REF, QUAD ? DEAL_ALL : (PPT > 1 ? DEAL_EVEN : DEAL_64)>(
       g, cx0, cx1, cy0, cy1, cz0, cz1, tbx0, tby0, tbx1, tby1, support,
       [&](int cx, int cy) {
         return allz_u && cy >= r_ily && cy <= r_ihy && cx >= r_ilx && cx <= r_ihx;
@@ -857,8 +895,8 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
           // (x, y, coef, 1/h^2); the quartic's z is c = coef^0.4
           const float4 q = g.part[sidx];
           if (q.z != 0.0f) {
-            const float dx = fmaxf(fmaxf(tbx0 - q.x, q.x - tbx1), 0.0f);
-            const float dy = fmaxf(fmaxf(tby0 - q.y, q.y - tby1), 0.0f);
+            const float dx = fmaxf(fmaxf(wbx0 - q.x, q.x - wbx1), 0.0f);
+            const float dy = fmaxf(fmaxf(wby0 - q.y, q.y - wby1), 0.0f);
             const float d2 = fmaf(dy, dy, dx * dx);
             keep = d2 * q.w < cull2;
           }
@@ -899,7 +937,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
           if (far) L.X[nf + int(prefix_count(bf))] = e;
         if constexpr (QUARTIC) {
           if (big && !far) {
-            const int pos = kWavePool - 1 - (nb + int(prefix_count(bb)));
+            const int pos = POOL - 1 - (nb + int(prefix_count(bb)));
             L.X[pos] = e;
             if constexpr (CLIP) L.Xz[pos] = tcl;
           }
@@ -912,7 +950,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
         if constexpr (REF) {
           if (keep && !full) {
             const int pos = nm + int(prefix_count(bm));
-            L.S[kWavePool - 1 - pos] = e;
+            L.S[POOL - 1 - pos] = e;
             L.M[pos] = cinf;
           }
         }
@@ -920,14 +958,14 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
         nb += __popcll(bb);
         ns += __popcll(bs);
         nm += __popcll(bm);
-        const int lim = done ? 1 : kWaveFlush;
+        const int lim = done ? 1 : FLUSH;
         if constexpr (FAR) {
           if (done && !far_used && nf > 0) {
             // too few far entries to pay for the tile's interpolation
             const int n = uniform(nf);
             const float4 x = lane < n ? L.X[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
             wave_sync();
-            if (lane < n) L.X[kWavePool - 1 - (nb + lane)] = x;
+            if (lane < n) L.X[POOL - 1 - (nb + lane)] = x;
             nb += n;
             nf = 0;
           }
@@ -939,6 +977,19 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
       });
   if constexpr (FAR)
     if (far_used && lane == 0) sm.far_used = 1;
+
+  if constexpr (QUAD) {
+    const uint32_t px = tx * T + uint32_t(col_of(t)), py = ty * T + uint32_t(row_of(t));
+    const uint32_t pid = py * p.lnx + px;
+    if (!(px < p.lnx && py < p.lny && pid < p.n)) return;
+    if (fused) {
+      acc_out[pid] = a64[0];
+      img_out[pid] = static_cast<float>(a64[0] * static_cast<double>(img_scale));
+    } else {
+      acc_out[pid] += a64[0];
+    }
+    return;
+  }
 
   // ---- the waves' sums, in wave order
   __syncthreads();
@@ -966,7 +1017,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   }
 #pragma unroll 1
   for (int pt = t; pt < NP; pt += NB) {
-    const uint32_t px = tx * T + uint32_t(pt % T), py = ty * T + uint32_t(pt / T);
+    const uint32_t px = tx * T + uint32_t(col_of(pt)), py = ty * T + uint32_t(row_of(pt));
     const uint32_t pid = py * p.lnx + px;
     if (!(px < p.lnx && py < p.lny && pid < p.n)) continue;
     double v = sm.sum[0][pt];
@@ -1011,7 +1062,7 @@ template <int T, int OP, int KERNEL>
 __global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSumWaves, 8))) void k_gather(
     grid_view g, point_view p, uint32_t tiles_x, uint32_t ntiles, double* __restrict__ acc_out,
     unsigned long long* __restrict__ counts, const float* __restrict__ cubic_table, float support) {
-  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT> sm;
+  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT, false> sm;
   if constexpr (KERNEL == 2) {
     for (int i = threadIdx.x; i < kCubicTable; i += 64 * kSumW) sm.tab[i] = cubic_table[i];
   }
@@ -1022,7 +1073,7 @@ __global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSum
   const uint32_t per = ntiles / 8u;
   const uint32_t tile = bid < per * 8u ? (bid % 8u) * per + bid / 8u : bid;
   const uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
-  sum_tile<T, OP, KERNEL>(g, p, tx, ty, acc_out, counts, support, sm);
+  sum_tile<T, OP, KERNEL, false>(g, p, tx, ty, acc_out, counts, support, sm);
 }
 
 // Persistent gather over (view, tile) items.  Workgroups are dealt to the 8
@@ -1031,11 +1082,11 @@ __global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSum
 // on at a time are neighbours that read the same particle spans.  A
 // workgroup drains its XCD's queue, then helps with the others; every queue
 // counter only grows, so every workgroup leaves once all queues are empty.
-template <int T, int OP, int KERNEL>
-__global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSumWaves, 8))) void k_gather_batch(
+template <int T, int OP, int KERNEL, bool QUAD>
+__global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(QUAD ? 8 : kSumWaves, 8))) void k_gather_batch(
     const view_desc* __restrict__ views, const uint2* __restrict__ items, queue_segs segs,
     uint32_t* __restrict__ counters, const float* __restrict__ cubic_table, float support) {
-  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT> sm;
+  __shared__ tile_smem<T, OP == OP_REFERENCE, KERNEL, OP == OP_CLIP, OP == OP_COUNT, QUAD> sm;
   __shared__ uint32_t next;
   if constexpr (KERNEL == 2) {
     for (int i = threadIdx.x; i < kCubicTable; i += 64 * kSumW) sm.tab[i] = cubic_table[i];
@@ -1054,7 +1105,7 @@ __global__ __launch_bounds__(64 * kSumW) __attribute__((amdgpu_waves_per_eu(kSum
       const uint32_t vi = uint32_t(uniform(int(it.x))), ti = uint32_t(uniform(int(it.y)));
       const view_desc& vd = views[vi];
       const uint32_t tiles_x = vd.tiles_x;
-      sum_tile<T, OP, KERNEL>(vd.g, vd.p, ti % tiles_x, ti / tiles_x, vd.acc, nullptr, support,
+      sum_tile<T, OP, KERNEL, QUAD>(vd.g, vd.p, ti % tiles_x, ti / tiles_x, vd.acc, nullptr, support,
                                  sm, vd.img, vd.scale, vd.fused);
     }
   }
@@ -1311,7 +1362,7 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
     }
   };
 
-  stream_candidates<false, false>(
+  stream_candidates<false, DEAL_64>(
       g, cx0, cx1, cy0, cy1, 0, g.nc[2] - 1, tbx0, tby0, tbx1, tby1, support,
       [](int, int) { return true; }, sm.cells,
       [&](bool have, uint32_t sidx, int, bool, bool done) {
@@ -1357,7 +1408,7 @@ __global__ __launch_bounds__(kBlock) void k_unpermute4(const uint32_t* __restric
   od[i] = d[s];
 }
 
-template <int T, int OP, int KERNEL>
+template <int T, int OP, int KERNEL, bool QUAD>
 struct plain_launcher {
   static int run(const grid_view& g, const point_view& p, double* acc,
                  unsigned long long* counts, const float* tab, float support, hipStream_t s) {
@@ -1365,50 +1416,61 @@ struct plain_launcher {
     const uint32_t tiles_y = (p.lny + T - 1) / T;
     const uint32_t ntiles = tiles_x * tiles_y;
     if (!ntiles) return 0;
-    hipLaunchKernelGGL((k_gather<T, OP, KERNEL>), dim3(ntiles), dim3(64 * kSumW), 0, s, g, p,
-                       tiles_x, ntiles, acc, counts, tab, support);
+    if constexpr (QUAD) {
+      fail(ILC_EINVAL, "quarter tiles are the persistent gather's");
+    } else {
+      hipLaunchKernelGGL((k_gather<T, OP, KERNEL>), dim3(ntiles), dim3(64 * kSumW), 0, s, g, p,
+                         tiles_x, ntiles, acc, counts, tab, support);
+    }
     ILC_HIP(hipGetLastError());
     return 0;
   }
 };
 
-template <int T, int OP, int KERNEL>
+template <int T, int OP, int KERNEL, bool QUAD>
 struct batch_launcher {
   static int run(const view_desc* v, const uint2* it, const queue_segs& segs, uint32_t* c,
                  const float* tab, float sup, int grid, hipStream_t s) {
-    hipLaunchKernelGGL((k_gather_batch<T, OP, KERNEL>), dim3(grid), dim3(64 * kSumW), 0, s, v,
+    hipLaunchKernelGGL((k_gather_batch<T, OP, KERNEL, QUAD>), dim3(grid), dim3(64 * kSumW), 0, s, v,
                        it, segs, c, tab, sup);
     ILC_HIP(hipGetLastError());
     return 0;
   }
 };
 
-template <int T, int OP, int KERNEL>
+template <int T, int OP, int KERNEL, bool QUAD>
 struct batch_occ {
   static int run() {
     int per_cu = 0;
     ILC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, k_gather_batch<T, OP, KERNEL>, 64 * kSumW, 0));
+        &per_cu, k_gather_batch<T, OP, KERNEL, QUAD>, 64 * kSumW, 0));
     return per_cu;
   }
 };
 
-// dispatch over (tile side, op, kernel) to F<T, OP, KERNEL>::run
-template <template <int, int, int> class F, class... A>
+// dispatch over (tile side, op, kernel, quarters) to F<T, OP, KERNEL, QUAD>::run
+template <template <int, int, int, bool> class F, class... A>
 int dispatch(const sum_shape& ts, int op, int kernel, A&&... a) {
   auto by_op = [&](auto tt) -> int {
     constexpr int T = decltype(tt)::value;
     if (op == OP_CLIP) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "the line-of-sight clip needs a quartic kernel");
-      return F<T, OP_CLIP, 0>::run(a...);
+      return F<T, OP_CLIP, 0, false>::run(a...);
     }
     if (op == OP_REFERENCE) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "reference mode uses the quartic kernel");
-      return F<T, OP_REFERENCE, 0>::run(a...);
+      return F<T, OP_REFERENCE, 0, false>::run(a...);
     }
-    if (kernel == ILC_KERNEL_CUBIC) return F<T, OP_EXACT, 2>::run(a...);
-    return F<T, OP_EXACT, 0>::run(a...);
+    if (kernel == ILC_KERNEL_CUBIC) return F<T, OP_EXACT, 2, false>::run(a...);
+    return F<T, OP_EXACT, 0, false>::run(a...);
   };
+  if (ts.quad) {
+    ILC_REQUIRE(ts.side == 16 && kernel != ILC_KERNEL_CUBIC &&
+                    (op == OP_REFERENCE || op == OP_EXACT),
+                "quarters are of 16x16 tiles of the quartic");
+    return op == OP_REFERENCE ? F<16, OP_REFERENCE, 0, true>::run(a...)
+                              : F<16, OP_EXACT, 0, true>::run(a...);
+  }
   if (ts.side == 16) return by_op(std::integral_constant<int, 16>{});
   if (ts.side == 8) return by_op(std::integral_constant<int, 8>{});
   fail(ILC_EINVAL, "gather: no tile of side %d", ts.side);
@@ -1436,6 +1498,21 @@ sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints) {
     if (ts.tw == 8 && ts.ppt == 1) return sum_shape{8};
   }
   fail(ILC_EINVAL, "gather: unsupported tile shape tw=%d ppt=%d nb=%d", ts.tw, ts.ppt, ts.nb);
+}
+
+// Slab stacks whose tiles are many and hold few rows: both forms are bound by
+// issue slots, and the quarters need 4 to 12% fewer and wait less for them.
+// Every wave of a quarter tile streams all candidates, so the tile over the
+// densest core ends four times as late; it needs enough other tiles to hide
+// behind.  The gather's time, quarters against whole tiles, over slabs of 30k to
+// 64M cells (1 to 32 halos, 4 to 32 slabs of 1024^2 to 4096^2 points), by the
+// tiles per (row in a tile) in thousands: 0.67 to 1.51 below 13, 1.20 on average;
+// 0.76 to 1.23 from 14 to 20; 0.84 on average from 25, at most 1.02 (1.06 in one
+// launch of 0.16 ms).  32 slabs of 4096^2 through 64M 28.4 -> 23.0 ms, 16 through
+// 32M 12.1 -> 9.9.  Views of any orientation close to a snapshot's centre have
+// wide supports, whose nodes they need: 1.0 to 1.9.
+bool quarter_tiles(uint64_t ntiles, uint64_t rows) {
+  return double(ntiles) * double(ntiles) >= 25000.0 * double(rows);
 }
 
 void tile_grid(const sum_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
@@ -1502,7 +1579,7 @@ void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
   const float support = kernel == ILC_KERNEL_CUBIC ? 2.0f : 1.0f;
   if (op == OP_COUNT) {
     // the count has its own tile shape: its cost is independent of the render's
-    plain_launcher<16, OP_COUNT, 0>::run(g, p, nullptr, counts, nullptr, support, s);
+    plain_launcher<16, OP_COUNT, 0, false>::run(g, p, nullptr, counts, nullptr, support, s);
     return;
   }
   if (kernel == ILC_KERNEL_CUBIC && !cubic_table)

@@ -266,11 +266,15 @@ struct tile_shape {
 
 // The tiles that a launch over npoints points works in: side x side points
 // (16 or 8), one per workgroup.  64-thread shapes ask for their own side, the
-// others leave it to the number of points.
+// others leave it to the number of points.  quad (16x16 tiles of the quartic in
+// the persistent gather): a wave for each 8x8 quarter.
 struct sum_shape {
   int side;
+  bool quad = false;
 };
 sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints);
+// whether a slab stack of that many 16x16 tiles and kept rows is summed by quarters
+bool quarter_tiles(uint64_t ntiles, uint64_t rows);
 
 void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
                    const sum_shape& ts, double* acc, unsigned long long* counts,

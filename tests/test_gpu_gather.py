@@ -316,3 +316,42 @@ def test_few_candidates_for_a_tile(B, orc, n, mode, kernel):
         assert np.max(np.abs(got - ref)) < 2e-5 * ref.max()
     else:
         assert np.all(np.abs(got - ref) <= pair_bound(pp, h, pts, kernel))
+
+
+@pytest.mark.parametrize("mode,kernel", [("reference", "quartic_ref"), ("exact", "quartic")])
+@pytest.mark.parametrize("nx,ny,n,hmax", [
+    (999, 603, 3500, 40.0),   # the last column and row of tiles with empty quarters
+    (1041, 520, 2500, 3.0),   # supports within a tile, the last row half empty
+])
+def test_slab_stack_by_quarter_tiles(B, orc, nx, ny, n, hmax, mode, kernel):
+    """Slab stacks of many tiles for their rows, summed by the quarters of
+    16x16 tiles, against the oracle on sampled points (the last tiles' among
+    them); a dense clump fills the lists many times over."""
+    rng = np.random.default_rng(nx)
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, 0], p4[:, 1] = rng.uniform(-0.55 * nx, 0.55 * nx, n), rng.uniform(-0.55 * ny, 0.55 * ny, n)
+    p4[: n // 3, :2] = rng.normal(0, 6.0, (n // 3, 2)) + (0.5 * nx - 8.0, 0.5 * ny - 9.0)
+    p4[:, 2] = rng.uniform(0, 40, n)
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    h = np.exp(rng.uniform(np.log(0.4), np.log(hmax), n)).astype(np.float32)
+    views = [dict(position=np.array([0.0, 0.0, 10.0 * k]), look_at=np.array([0.0, 0.0, 1.0]),
+                  roll=0.0, width=float(nx), nx=nx, ny=ny, depth=10.0) for k in range(4)]
+    r = B.BatchRenderer(mode=mode, kernel=kernel, tile=(16, 16, 64))
+    r.set_particles(p4[:, :3].copy(), p4[:, 3].copy(), h)
+    r.set_views(views)
+    r.render()
+    rows = sum(r.view_info(k)["num_particles"] for k in range(4))
+    tiles = 4 * -(-nx // 16) * -(-ny // 16)
+    assert tiles ** 2 >= 25000 * rows  # the rule's line
+    x, y = rng.integers(0, nx, 1500), rng.integers(0, ny, 1500)
+    x[:500], y[:500] = rng.integers(nx - 40, nx, 500), rng.integers(ny - 40, ny, 500)
+    idx = y * nx + x
+    for k, v in enumerate(views):
+        cam = orc.Camera(v["position"], v["look_at"], v["roll"], v["width"], nx, ny)
+        pp, pts = cam.project_particles(p4, v["depth"]), cam.pixel_points()[idx]
+        ref = orc.Grid(pp, h).gather_ref(pts, acc_mode=1) if mode == "reference" else \
+            orc.gather_exact(pp, h, pts, kind=1)
+        got = r.image_f64(k).cpu().numpy().reshape(-1)[idx]
+        off = np.abs(got - ref) / np.maximum(pair_bound(pp, h, pts, kernel), 1e-300)
+        print(f"quarters {nx}x{ny} {mode} slab {k}: {off.max():.2f} of the bound", flush=True)
+        assert ref.max() > 0 and off.max() <= 1.0

@@ -524,16 +524,28 @@ void plan(ilc_batch* b, hipStream_t s) {
   for (size_t v = 0; v < nv; ++v)
     npoints += uint64_t(b->views[v]->v.cam.nx) * b->views[v]->v.cam.ny;
   b->ss = sum_shape_of(b->ts, npoints);
-  for (size_t v = 0; v < nv; ++v) {
-    view_state& vs = *b->views[v];
-    tile_grid(b->ss, vs.v.cam.nx, vs.v.cam.ny, &vs.tiles_x, &vs.ntiles);
-    nitems += vs.ntiles;
-  }
-  ILC_REQUIRE(nitems < (uint64_t(1) << 32), "too many work items");
+  auto tile_views = [&] {
+    nitems = 0;
+    for (size_t v = 0; v < nv; ++v) {
+      view_state& vs = *b->views[v];
+      tile_grid(b->ss, vs.v.cam.nx, vs.v.cam.ny, &vs.tiles_x, &vs.ntiles);
+      nitems += vs.ntiles;
+    }
+  };
+  tile_views();
   bool slabs = true;
   for (auto& v : b->views) slabs = slabs && v->compact;
-  b->ss.quad = slabs && !b->clip && b->kernel != ILC_KERNEL_CUBIC && b->ss.side == 16 &&
-               quarter_tiles(nitems, ntot);
+  if (slabs && b->ss.side == 16) {
+    if (b->clip) {
+      if (b->ts.nb != 64 && small_clip_tiles(nitems, ntot)) {
+        b->ss.side = 8;
+        tile_views();
+      }
+    } else {
+      b->ss.quad = b->kernel != ILC_KERNEL_CUBIC && quarter_tiles(nitems, ntot);
+    }
+  }
+  ILC_REQUIRE(nitems < (uint64_t(1) << 32), "too many work items");
   // queue q: the q-th eighth (contiguous tiles, image order) of every view,
   // largest views first
   uint2* it = b->items_host.ensure(nitems);

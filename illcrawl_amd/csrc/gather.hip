@@ -1416,8 +1416,8 @@ struct plain_launcher {
     const uint32_t tiles_y = (p.lny + T - 1) / T;
     const uint32_t ntiles = tiles_x * tiles_y;
     if (!ntiles) return 0;
-    if constexpr (QUAD) {
-      fail(ILC_EINVAL, "quarter tiles are the persistent gather's");
+    if constexpr (QUAD || OP == OP_CLIP) {
+      fail(ILC_EINVAL, "quarter tiles and the clip are the persistent gather's");
     } else {
       hipLaunchKernelGGL((k_gather<T, OP, KERNEL>), dim3(ntiles), dim3(64 * kSumW), 0, s, g, p,
                          tiles_x, ntiles, acc, counts, tab, support);
@@ -1455,7 +1455,11 @@ int dispatch(const sum_shape& ts, int op, int kernel, A&&... a) {
     constexpr int T = decltype(tt)::value;
     if (op == OP_CLIP) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "the line-of-sight clip needs a quartic kernel");
-      return F<T, OP_CLIP, 0, false>::run(a...);
+      // 16x16 tiles by quarters: the clip has no nodes, and with four points a
+      // lane the larger pair leaves 5 waves a SIMD (four 1024^2 views of 16M
+      // particles 21.2 ms, 14.3 by quarters, 14.7 in 8x8 tiles; 2048^2 ones 70.7,
+      // 50.5, 55.4; 32 slabs of 4096^2 through 64M 98.4, 67.2, 84.1)
+      return F<T, OP_CLIP, 0, T == 16>::run(a...);
     }
     if (op == OP_REFERENCE) {
       if (kernel == ILC_KERNEL_CUBIC) fail(ILC_EINVAL, "reference mode uses the quartic kernel");
@@ -1513,6 +1517,15 @@ sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints) {
 // wide supports, whose nodes they need: 1.0 to 1.9.
 bool quarter_tiles(uint64_t ntiles, uint64_t rows) {
   return double(ntiles) * double(ntiles) >= 25000.0 * double(rows);
+}
+
+// Clipped slab stacks of few tiles for their rows, where the quarters' densest
+// tile sets the time: 8x8 tiles.  By the tiles per (row in a tile) in thousands:
+// at 0.01 (8 slabs of 512^2 through 16M particles) 9.5 ms against 32.3 by
+// quarters, at 0.06 (512^2, 1M) 1.0 against 2.0, at 0.16 (1024^2, 16M) 6.0 against
+// 24.5; at 0.44 (512^2, 100k) 0.56 against 0.38, at 0.95 (1024^2, 1M) 3.3 against 1.8.
+bool small_clip_tiles(uint64_t ntiles, uint64_t rows) {
+  return double(ntiles) * double(ntiles) < 300.0 * double(rows);
 }
 
 void tile_grid(const sum_shape& ts, uint32_t lnx, uint32_t lny, uint32_t* tiles_x,
@@ -1584,7 +1597,6 @@ void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
   }
   if (kernel == ILC_KERNEL_CUBIC && !cubic_table)
     fail(ILC_EINVAL, "cubic gather without its table");
-  if (op == OP_CLIP) ILC_REQUIRE(g.clip != nullptr, "clip gather without clip parameters");
   dispatch<plain_launcher>(ts, op, kernel, g, p, acc, counts, cubic_table, support, s);
 }
 

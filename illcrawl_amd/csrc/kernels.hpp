@@ -275,6 +275,8 @@ struct sum_shape {
 sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints);
 // whether a slab stack of that many 16x16 tiles and kept rows is summed by quarters
 bool quarter_tiles(uint64_t ntiles, uint64_t rows);
+// whether a clipped one is summed in 8x8 tiles instead
+bool small_clip_tiles(uint64_t ntiles, uint64_t rows);
 
 void launch_gather(const grid_view& g, const point_view& p, int op, int kernel,
                    const sum_shape& ts, double* acc, unsigned long long* counts,

@@ -113,6 +113,44 @@ def test_clipped_rotated_view_vs_oracle(B, orc, snap):
     assert linf < LINF_TOL and s < SUM_TOL
 
 
+@pytest.mark.parametrize("tile", [(16, 16, 64), (8, 8, 64)])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (17, 40), (50, 31)])
+def test_clip_tiles_vs_oracle(B, orc, snap, nx, ny, tile):
+    """Both tile sides, partial tiles and tiles with empty quarters."""
+    from illcrawl_amd import synth
+    v = synth.centred_view(snap.box, look_at=(0.4, -0.3, 0.85), width=1500.0, nx=nx, roll=0.7)
+    v = dict(v, ny=ny, depth=0.55 * v["depth"], quantity=0)
+    r = B.BatchRenderer(mode="exact", kernel="quartic", tile=tile)
+    r.set_particles(snap.pos, snap.mass, snap.hsml)
+    r.set_depth_clip(True)
+    r.set_views([v])
+    r.render()
+    linf, s = errors(r.image_f64(0).cpu().numpy().reshape(-1), oracle_clip(orc, snap, v, 1))
+    say(f"clip {nx}x{ny} tile {tile}: linf {linf:.2e} sum {s:.2e}")
+    assert linf < LINF_TOL and s < SUM_TOL
+
+
+def test_dense_clipped_slabs_vs_oracle(B, orc):
+    """A clipped slab stack of few tiles for its rows (8x8 tiles by the rule,
+    from enough points for 16x16 ones), on sampled points."""
+    from illcrawl_amd import synth
+    snap = synth.make_snapshot(1 << 17, 5, 10000.0, n_halos=1, rs_range=(300.0, 300.0), gas=True)
+    views = synth.slab_views(snap.box, n_slabs=4, thickness=2500.0, nx=448, quantity=0)
+    r = clip_batch(B, snap, views)
+    rows = sum(r.view_info(k)["num_particles"] for k in range(4))
+    tiles = 4 * 28 ** 2
+    assert 4 * 448 ** 2 >= 3 << 18 and tiles ** 2 < 300 * rows
+    idx = np.random.default_rng(3).choice(448 ** 2, 400, replace=False)
+    for k in (0, 2):
+        v = views[k]
+        cam = orc.Camera(v["position"], v["look_at"], v["roll"], v["width"], v["nx"], v["ny"])
+        pz = cam.project_particles_depth(snap.particles4())
+        ref = orc.gather_clip(pz, snap.hsml, cam.pixel_points()[idx], v["depth"], 0)
+        linf, s = errors(r.image_f64(k).cpu().numpy().reshape(-1)[idx], ref)
+        say(f"dense clipped slab {k}: linf {linf:.2e} sum {s:.2e}")
+        assert linf < LINF_TOL and s < SUM_TOL
+
+
 def test_clip_error_paths(B, snap):
     from illcrawl_amd import IllcrawlError, synth
     say("case: clip error paths")

@@ -197,15 +197,21 @@ __device__ inline uint32_t block_scan_excl(uint32_t v, uint32_t* total, uint32_t
   return off + incl - v;
 }
 
-// VALU-bound.  8 slices of 2048^2 through 16M particles, about 80 pairs kept and
-// 80 covered of 2000 candidates a 16 x 16 tile: 82% of the issue slots at 3.30 ms,
-// 3.54 ms (96%) with one point a lane, one list a workgroup, every row streamed
-// whole and no cover form.  A 250 x 180 slice through 60k: 50 us with 8 x 8
-// tiles, 205 us before.  A tile's fixed work is a quarter of its
-// instructions, the candidates' culling half.  5 waves a SIMD keep the registers
-// of 4 points a lane.
+// Bound by issue slots and, with 5 or 6 waves a SIMD, by waiting for them: a VALU
+// instruction issues in 81% of the busy cycles (SQ_ACTIVE_INST_VALU over
+// SQ_BUSY_CU_CYCLES).  A tile's fixed work is a quarter of its instructions, the
+// candidates' culling half (8 slices of 2048^2 through 16M particles: about 80
+// pairs kept and 80 covered of 2000 candidates a 16x16 tile).  Against one point a
+// lane at 7 waves, one list a workgroup, every row streamed whole and no cover
+// form: a 250 x 180 slice through 60k 205 -> 50 us, 4 slices of 1024^2 through 1M
+// 0.70 -> 0.55 ms, through 4M of one h 6.9 -> 4.2; 8 slices of 2048^2 through 16M 3.34
+// -> 3.40 (exact search 2.85 -> 2.79), and with the h of a neighbour search
+// 2.53 -> 3.01: as many instructions (1.46e9 against 1.50e9), issued in 81%
+// instead of 99% of the cycles.  5 waves a SIMD keep the registers of 4 points a
+// lane, 6 without search boxes (8 slices 2.98 ms at 5, 2.79 at 6, 3.13 at 7); with
+// them 6 waves spill (3.5 ms against 3.0).
 template <int T, bool REF, bool COUNT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_smooth3d(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(T == 16 && !REF ? 6 : 5, 8))) void k_smooth3d(
     grid_view g, level_view lv, point_view p, uint32_t tiles_x, double* __restrict__ acc,
     unsigned long long* __restrict__ cnt) {
   static_assert(!(REF && COUNT), "evaluations are counted with the exact search");

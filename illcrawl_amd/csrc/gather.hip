@@ -184,12 +184,16 @@ __device__ inline void node_basis(double u, double* b) {
   }
 }
 
-// A particle at r from the tile centre is far when the tile's half-diagonal a
-// is at most (0.4 + 0.22 r / h) (h - r): the interpolation then errs by at
-// most 4e-8 of the particle's value at the tile centre (the largest over all
-// directions and r / h in [0, 0.99]; s^2.5 is singular at the support's edge
-// only, h - r and h + r away), below the FP32 rounding of the direct form.
-// The adjoint's s^1.5 meets the same bound with a slope of 0.16.  Up to 0.999 h, so
+// A particle at r from the tile centre is far when a <= (0.4 + 0.22 r / h) (h - r),
+// a = sqrt(2) times the tile's larger half-side (the half-diagonal of a square
+// one): the interpolation then errs by at most 4e-8 of the particle's value at the
+// tile centre and 3.3e-7 of its value at the point itself (the largest over all
+// tile shapes, directions and r / h up to 0.999; s^2.5 is singular at the
+// support's edge only, h - r and h + r away), below the FP32 rounding of the
+// direct form.  The half-diagonal would not do in strip tiles (an image's last
+// row or column of tiles), whose nodes lie wider for it: 5.6e-7 and 6.3e-6.  The
+// adjoint's s^1.5 meets 4.1e-8 and 1.2e-7 with a slope of 0.16 (its nodes'
+// gradients are FP32: up to 2e-7 of the value at the centre more).  Up to 0.999 h, so
 // that every argument is positive by far more than its rounding (s >= 7e-4): the
 // nodes need no clamp at 0, one of the 6 issue slots of a pair (3 FMAs, clamp,
 // square, multiply-add; the square root runs beside them).  Without it, and
@@ -622,6 +626,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   const float hd_x = 0.5f * (wbx1 - wbx0), hd_y = 0.5f * (wby1 - wby0);
   const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
   const float big_r2 = 4.0f * hd2 * 1.0001f + 1e-30f;
+  const float far_a2 = 2.0f * fmaxf(hd_x * hd_x, hd_y * hd_y);  // see is_far
 
   // ---- candidate cell box
   int cx0, cx1, cy0, cy1, cz0, cz1;
@@ -922,7 +927,7 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
                 const float xr = q.x - tcx, yr = q.y - tcy;
                 const float d2r = fmaf(yr, yr, xr * xr);
                 e = make_float4(c * fmaf(-q.w, d2r, 1.0f), 2.0f * ci2 * xr, 2.0f * ci2 * yr, -ci2);
-                if constexpr (FAR) far = is_far(d2r, q.w, hd2);
+                if constexpr (FAR) far = is_far(d2r, q.w, far_a2);
               } else {
                 e = make_float4(q.x, q.y, ci2, c);
               }
@@ -1221,11 +1226,11 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
   if (!(tbx0 <= tbx1)) return;  // no gradient in the tile
   const float tcx = 0.5f * (tbx0 + tbx1), tcy = 0.5f * (tby0 + tby1);
   const float hd_x = 0.5f * (tbx1 - tbx0), hd_y = 0.5f * (tby1 - tby0);
-  const float hd2 = fmaf(hd_y, hd_y, hd_x * hd_x);
+  const float far_a2 = 2.0f * fmaxf(hd_x * hd_x, hd_y * hd_y);  // see is_far
 
   // ---- the gradients at the nodes (when any particle is wide enough; an
   // infinite one would meet weights of either sign there)
-  const bool nodes = FAR && !uniform(wild) && g.max_h * g.max_h * 0.16f >= hd2;
+  const bool nodes = FAR && !uniform(wild) && g.max_h * g.max_h * 0.16f >= far_a2;
   if constexpr (FAR) {
     if (nodes) {
       double b[kNodes];
@@ -1374,7 +1379,7 @@ __global__ __launch_bounds__(64 * kSumW) void k_adjoint(grid_view g, point_view 
           keep = fmaf(dy, dy, dx * dx) * q.w < cull2;
           if constexpr (FAR) {
             const float xr = q.x - tcx, yr = q.y - tcy;
-            far = keep && nodes && is_far(fmaf(yr, yr, xr * xr), q.w, hd2, 0.16f);
+            far = keep && nodes && is_far(fmaf(yr, yr, xr * xr), q.w, far_a2, 0.16f);
           }
         }
         const uint64_t bf = FAR ? __ballot(far) : 0ull;

@@ -355,3 +355,37 @@ def test_slab_stack_by_quarter_tiles(B, orc, nx, ny, n, hmax, mode, kernel):
         off = np.abs(got - ref) / np.maximum(pair_bound(pp, h, pts, kernel), 1e-300)
         print(f"quarters {nx}x{ny} {mode} slab {k}: {off.max():.2f} of the bound", flush=True)
         assert ref.max() > 0 and off.max() <= 1.0
+
+
+# The nodes' interpolation errs by at most 3.3e-7 of a far particle's own value
+# at a point of the tile, whatever the tile's shape (in FP64, over all directions
+# and distances that the rule takes).  A sum over many particles averages their
+# FP32 rounding (6e-8 left: three deviations of 5e-6 over 65536), but not the kernel
+# constant's (2^-24 twice).
+@pytest.mark.parametrize("nx,ny", [(16, 1), (1, 16), (16, 4), (3, 16), (16, 16)])
+@pytest.mark.parametrize("of", ["diagonal", "side"])
+def test_far_particles_of_strip_tiles(B, orc, nx, ny, of):
+    """Particles 0.9 h from the tile's centre, along its longer side, whose
+    supports are just wide enough by its half-diagonal, or by sqrt 2 times its
+    larger half-side."""
+    rng = np.random.default_rng(nx * 20 + ny)
+    n, hx, hy = 65536, 0.5 * (nx - 1), 0.5 * (ny - 1)
+    a = np.hypot(hx, hy) if of == "diagonal" else np.sqrt(2.0) * max(hx, hy)
+    p4 = np.zeros((n, 4), np.float32)
+    h = (a / (0.975 * (0.4 + 0.9 * 0.22) * 0.1) * (1.0 + 0.004 * rng.random(n))).astype(np.float32)
+    p4[:, :2] = rng.uniform(-5e-4, 5e-4, (n, 2)) * h[:, None]
+    p4[:, 0 if nx >= ny else 1] += 0.9 * h
+    p4[:, 3] = rng.uniform(0.5, 1.5, n)
+    view = dict(position=np.array([0.0, 0.0, -20.0]), look_at=np.array([0.0, 0.0, 1.0]),
+                roll=0.0, width=float(nx), nx=nx, ny=ny, depth=40.0)
+    cam = orc.Camera(view["position"], view["look_at"], view["roll"], view["width"], nx, ny)
+    pts = cam.pixel_points()
+    p4[:, :2] += 0.5 * (pts[:, :2].min(0) + pts[:, :2].max(0))  # the points are the pixels' corners
+    r = B.BatchRenderer(mode="exact", kernel="quartic", tile=(16, 16, 64))
+    r.set_particles(p4[:, :3].copy(), p4[:, 3].copy(), h)
+    r.set_views([view])
+    r.render()
+    ref = orc.gather_exact(cam.project_particles(p4, view["depth"]), h, pts, kind=1)
+    off = np.max(np.abs(r.image_f64(0).cpu().numpy().reshape(-1) / ref - 1.0))
+    print(f"far strip {nx}x{ny} by the {of}: {off:.2e}", flush=True)
+    assert off < 3.3e-7 + 2 * 2.0 ** -24 + 6e-8

@@ -20,6 +20,9 @@ LIB = os.path.join(LIBDIR, "libilcpsg.so")
 # C++ program driving the library through include/illcrawl_backend.hpp (GPU tests run it)
 DEMO_SRC = os.path.join(ROOT, "tests", "cpp", "backend_demo.cpp")
 DEMO = os.path.join(LIBDIR, "backend_demo")
+# the sorted order of the grids (GPU tests run it)
+SORT_SRC = os.path.join(ROOT, "tests", "cpp", "sort_order.cpp")
+SORT = os.path.join(LIBDIR, "sort_order")
 # C++ data crawler over an HDF5 snapshot (include/illcrawl_crawler.hpp)
 CRAWL_SRC = os.path.join(ROOT, "tests", "cpp", "crawl_demo.cpp")
 CRAWL = os.path.join(LIBDIR, "crawl_demo")
@@ -99,11 +102,13 @@ def build(verbose=False, jobs=None):
         cmd = [cc, "-shared", f"--offload-arch={ARCH}", "-o", tmp_lib] + objs
         subprocess.run(cmd, check=True)
         os.replace(tmp_lib, LIB)
-        if os.path.exists(DEMO_SRC):
-            cmd = [cc, "-O2", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "include"),
-                   DEMO_SRC, "-L", LIBDIR, "-lilcpsg", "-Wl,-rpath,$ORIGIN", "-o", DEMO + ".tmp"]
-            subprocess.run(cmd, check=True)
-            os.replace(DEMO + ".tmp", DEMO)
+        for src, out in ((DEMO_SRC, DEMO), (SORT_SRC, SORT)):
+            if os.path.exists(src):
+                cmd = [cc, "-O2", "-std=c++17", "-Wall", f"--offload-arch={ARCH}",
+                       "-I", os.path.join(ROOT, "include"), "-I", CSRC, src, "-L", LIBDIR,
+                       "-lilcpsg", "-Wl,-rpath,$ORIGIN", "-o", out + ".tmp"]
+                subprocess.run(cmd, check=True)
+                os.replace(out + ".tmp", out)
         # the data crawler and the render tool (HDF5 in, FITS out) need
         # HDF5's C++ API and cfitsio
         if os.path.exists(os.path.join(IO_PREFIX, "include", "H5Cpp.h")):

@@ -168,18 +168,53 @@ def test_adjoint_tiles(B, orc, nx, ny):
         assert e < 1e-4
 
 
-@pytest.mark.parametrize("n", [1, 2, 1024, 1025, 131072, 131073, 1 << 20, (1 << 20) + 1])
-def test_grid_sort_at_the_tile_and_path_limits(B, orc, n):
-    """The sort's tiles of 1024 and 4096 rows and its three paths (digit counts
-    by the passes, by a count launch, scanned): cells, ranges, max h and order
-    equal the oracle's bit for bit, and every cell holds its particles by
-    descending h (top 16 bits), ties in input order."""
+SORT_SIZES = [1, 2, 1024, 1025, 131072, 131073, 1 << 20, (1 << 20) + 1]
+
+
+def sort_input(n):
     rng = np.random.default_rng(n)
     p4 = np.zeros((n, 4), np.float32)
     p4[:, :2] = rng.normal(0, 30.0, (n, 2))
     p4[:, 3] = 1.0
     h = np.exp(rng.uniform(-8, 8, n)).astype(np.float32)
     h[rng.random(n) < 0.5] = 1.5
+    return p4, h
+
+
+@pytest.mark.parametrize("target", [40, 3])
+def test_cells_hold_their_particles_by_descending_h(orc, tmp_path, target):
+    """The order that the gather searches: by cell, in a cell by descending h (the
+    top 16 bits of its pattern), ties in input order, at the sort's limits."""
+    import os
+    import subprocess
+    from illcrawl_amd import build
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    if not os.path.exists(build.SORT):
+        pytest.fail("sort_order is not built (run __graft_entry__.build())")
+    for n in SORT_SIZES:
+        p4, h = sort_input(n)
+        p4.tofile(tmp_path / f"p4_{n}.f32")
+        h.tofile(tmp_path / f"h_{n}.f32")
+    r = subprocess.run([build.SORT, str(tmp_path), str(target)] + [str(n) for n in SORT_SIZES],
+                       capture_output=True, text=True, timeout=100)
+    print(r.stdout + r.stderr, flush=True)
+    assert r.returncode == 0
+    for n in SORT_SIZES:
+        p4, h = sort_input(n)
+        cell = orc.Grid(p4, h, target=target).keys(p4)
+        order = np.lexsort((np.arange(n), -(h.view(np.uint32) >> 16).astype(np.int64), cell))
+        assert np.array_equal(np.fromfile(tmp_path / f"perm_{n}.u32", np.uint32), order)
+        assert np.array_equal(np.fromfile(tmp_path / f"key_{n}.u32", np.uint32), cell[order])
+
+
+@pytest.mark.parametrize("n", SORT_SIZES)
+def test_grid_sort_at_the_tile_and_path_limits(B, orc, n):
+    """The sort's tiles of 1024 and 4096 rows and its three paths (digit counts
+    by the passes, by a count launch, scanned): cells, ranges, max h and the
+    reference's order (sorted again from the input's) equal the oracle's bit for
+    bit."""
+    p4, h = sort_input(n)
     b = B.ProjectiveSmoothingGrid(target_particles_per_cell=40)
     b.init_backend(n)
     b.setup_projected_particles(p4, h)

@@ -1491,10 +1491,15 @@ int dispatch(const sum_shape& ts, int op, int kernel, A&&... a) {
 // at 64 nodes; 8x8 tiles give four times the workgroups and waste fewer pairs
 // at the supports' edges.  Below kPointsFor16 points the launch cannot fill
 // the GPU with 16x16 tiles and the heaviest one sets its time.  One view of
-// 1M / 16M / 100k particles, 8x8 against 16x16 tiles: 300^2 points 0.64, 3.1,
-// 0.33 against 1.30, 4.8, 0.48 ms; 700^2 1.03, 3.9, 0.51 against 1.26, 4.3,
-// 0.52; 1024^2 1.59, 5.0, 0.75 against 1.51, 4.7, 0.62; 2048^2 4.8, 11.1, 2.2
-// against 3.0, 7.4, 1.2.
+// 1M / 16M / 100k particles, 8x8 against 16x16 tiles: 300^2 points 0.30, 1.0,
+// 0.11 against 0.99, 3.8, 0.21 ms; 700^2 0.61, 1.10, 0.31 against 0.75, 1.71,
+// 0.24; 1024^2 1.12, 2.0, 0.57 against 0.93, 1.38, 0.31; 2048^2 3.9, 6.7, 2.0
+// against 2.1, 2.9, 0.82.  The cubic, which has no nodes: 300^2 1.2, 2.3, 0.51
+// against 3.9, 11.4, 1.1; 1024^2 6.6, 9.6, 3.0 against 6.8, 9.4, 2.7; 2048^2 22.6,
+// 34.6, 9.8 against 18.8, 27.4, 8.1.  The number of points is the whole launch's:
+// many small views of one batch would be faster in 8x8 tiles past the line, too
+// (64 of 128^2 through 1M 2.7 against 6.6 ms), which the caller can ask for or
+// have timed (ilc_batch_autotune).
 constexpr uint64_t kPointsFor16 = 3u << 18;
 
 sum_shape sum_shape_of(const tile_shape& ts, uint64_t npoints) {

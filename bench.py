@@ -58,8 +58,9 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-# the gather's two tiles, as exact requests (w, h, threads per workgroup)
-PLAIN_TILES = [(16, 16, 64), (8, 8, 64)]
+# the gather's two tiles, as exact requests (w, h, threads per workgroup), and
+# the side that each view's number of points picks
+PLAIN_TILES = [(16, 16, 64), (8, 8, 64), (16, 16, 256)]
 
 
 def parse_tile(text):

@@ -69,7 +69,9 @@ typedef struct {
                                         (dm_reconstruction_backend_grid.hpp:39) */
   int mode;                          /* ilc_mode */
   int kernel;                        /* ilc_kernel */
-  int tile_w, tile_h;                /* gather tile in points; 0 -> default */
+  int tile_w, tile_h;                /* gather tile in points, 0 -> default: every shape leaves
+                                        the side of the tiles to the number of points (see
+                                        ilc_batch_set_tile_wg for the batch's exact requests) */
 } ilc_psg_config;
 
 typedef struct {

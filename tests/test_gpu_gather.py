@@ -390,6 +390,10 @@ def test_slab_stack_by_quarter_tiles(B, orc, nx, ny, n, hmax, mode, kernel):
         off = np.abs(got - ref) / np.maximum(pair_bound(pp, h, pts, kernel), 1e-300)
         print(f"quarters {nx}x{ny} {mode} slab {k}: {off.max():.2f} of the bound", flush=True)
         assert ref.max() > 0 and off.max() <= 1.0
+    eager = [r.image_f64(k) for k in range(4)]
+    for _ in range(3):  # the graph's replays, with eager work between them
+        r.render(graph=True)
+        assert all(torch.equal(r.image_f64(k), eager[k]) for k in range(4))
 
 
 # The nodes' interpolation errs by at most 3.3e-7 of a far particle's own value

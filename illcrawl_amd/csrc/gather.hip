@@ -1058,9 +1058,10 @@ __device__ __attribute__((always_inline)) inline void sum_tile(
   }
 }
 
-// Waves per SIMD asked of the compiler: at 5 (96 VGPRs, 12 spilled in the
-// reference-mode batch) 32 views of a 16M snapshot take 50.0 ms, at 4 (no
-// spills) 53.5, at 3 60.2.  The LDS allows 5 workgroups per CU.
+// Waves per SIMD asked of the compiler for whole tiles: at 5 (96 VGPRs; 12 spilled
+// in the reference-mode batch when this was measured, 3 now) 32 views of a 16M
+// snapshot take 50.0 ms, at 4 (no spills) 53.5, at 3 60.2.  The LDS allows 5
+// workgroups per CU.  Quarters take 8 (64 VGPRs, 3 spilled).
 constexpr int kSumWaves = 5;
 
 template <int T, int OP, int KERNEL>
